@@ -366,6 +366,7 @@ __global__ __launch_bounds__(kBlock, MOM ? 8 : 1) void k_euler(const EulerArgs a
   constexpr bool kHeston = MODEL == SDEGPU_MODEL_HESTON;
   constexpr int N = kHeston ? M / 2 : M;
 
+  gauss_init<T>();
   // With fused row moments every thread of the block takes part in the LDS
   // reductions, so the lanes beyond the last path step a copy of the last
   // path and store nothing; otherwise they leave at once.

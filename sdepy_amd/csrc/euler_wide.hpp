@@ -37,6 +37,7 @@ __global__ __launch_bounds__(kBlock) void k_euler_wide(const EulerArgs a,
   constexpr bool kOU = MODEL == SDEGPU_MODEL_OU;
   constexpr int H = W / 2;
   constexpr int NS = kHeston ? H : W;  // state arrays, and counters of the info
+  gauss_init<T>();
   const int64_t gid = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (gid >= a.paths) return;
   const int64_t P = a.paths;
@@ -326,6 +327,7 @@ __global__ __launch_bounds__(kBlock) void k_wiener_fill_wide(
     uint32_t k0, uint32_t k1, uint32_t epoch, uint32_t c2, int64_t paths, int64_t nslots,
     const T* __restrict__ coef, int ncoef, int has_corr, int m, int comp0, int m_total,
     T* __restrict__ out) {
+  gauss_init<T>();
   const int64_t gid = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (gid >= paths) return;
   const uint32_t path = (uint32_t)gid;

@@ -247,6 +247,7 @@ __global__ __launch_bounds__(kBlock, (heston_waves<T, TV>())) void k_heston_adjo
     const HestonArgs a, const T* __restrict__ tb, const TV* __restrict__ tv,
     TV* __restrict__ ck, const double* __restrict__ sum_ds) {
   static_assert(C % 2 == 0, "one Philox block feeds two steps");
+  gauss_init<T>();
   const int64_t gid = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   const bool live = gid < a.paths;
   const uint32_t path = (uint32_t)gid;
@@ -345,6 +346,7 @@ template <typename T, typename TV>
 __global__ __launch_bounds__(kBlock, (heston_waves<T, TV>())) void k_heston_tangent(
     const HestonArgs a, const T* __restrict__ tb, const TV* __restrict__ tv,
     const double* __restrict__ sum_ds) {
+  gauss_init<T>();
   const int64_t gid = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   const bool live = gid < a.paths;
   const uint32_t path = (uint32_t)gid;
@@ -447,6 +449,7 @@ template <typename T>
 __global__ __launch_bounds__(kBlock) void k_loglin_greeks(const LogArgs a,
                                                           const T* __restrict__ st,
                                                           const double* __restrict__ pois) {
+  gauss_init<T>();
   const int64_t gid = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   const bool live = gid < a.paths;
   const uint32_t path = (uint32_t)gid;

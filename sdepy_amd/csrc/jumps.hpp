@@ -46,7 +46,7 @@ __device__ __forceinline__ float unit_exponential<float>(uint32_t x) {
 }
 template <>
 __device__ __forceinline__ double unit_exponential<double>(uint32_t x) {
-  return -log(u01_f64(x));
+  return 0.5 * neg2_log(x);
 }
 
 template <typename T>

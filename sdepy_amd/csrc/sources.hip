@@ -39,6 +39,7 @@ __global__ __launch_bounds__(kBlock) void k_wiener_fill(uint32_t k0, uint32_t k1
                                                         const T* __restrict__ coef, int ncoef,
                                                         int has_corr, int comp0, int m_total,
                                                         T* __restrict__ out) {
+  gauss_init<T>();
   const int64_t gid = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (gid >= paths) return;
   const uint32_t path = (uint32_t)gid;
@@ -94,6 +95,7 @@ __global__ __launch_bounds__(kBlock) void k_poisson_fill(uint32_t k0, uint32_t k
                                                          long long* __restrict__ dn_out,
                                                          const double* __restrict__ lamp,
                                                          int64_t lamp_step) {
+  gauss_init<T>();
   const int64_t gid = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (gid >= paths) return;
   const uint32_t path = (uint32_t)gid;
