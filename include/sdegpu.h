@@ -429,9 +429,8 @@ int sdegpu_cpoisson_fill_paths(int32_t dtype, const uint32_t key[2], uint32_t ep
  * of their squares (the host divides by paths and forms standard errors).
  *
  * Heston (NG = 7): d/d(x0, r, k, theta, xi, rho, y0); r is both the drift mu
- * of log x and the discount rate.  Reverse sweep over checkpoint segments of
- * 16 steps recomputed from the Philox counters; the workspace holds
- * ceil(nsteps/16) variance checkpoints per path plus block partials.
+ * of log x and the discount rate.  The workspace holds the expanded step
+ * table and block partials.
  * steps: device [nsteps][2] = (ds, sqrt(ds)) in dtype.  Scalar rho builds
  * corr = [[1, rho], [rho, 1]] as sdepy does (infrastructure.py:128-150).
  */
@@ -445,13 +444,12 @@ typedef struct sdegpu_heston_greeks {
   double strike, maturity;
   uint32_t key[2]; /* Philox key of the dw source */
   uint32_t epoch;
-  int32_t method;  /* 0: reverse-mode adjoint (variance checkpoints every 8 steps,
-                      recomputed segment by segment); 1: forward mode, the
-                      derivatives carried along the one forward pass (no
-                      checkpoints); the same estimator either way */
-  int32_t variance_f64; /* SDEGPU_F32 only, 1: the variance, its checkpoints and its
-                           adjoint (forward mode: every derivative) in FP64, the log
-                           price, the Philox normals and Box-Muller in FP32; where the
+  int32_t method;  /* 0: reverse-mode adjoint (swept over segments of the path, each
+                      while its partial derivatives are in registers); 1: forward
+                      mode, the derivatives carried along step by step; the same
+                      estimator either way */
+  int32_t variance_f64; /* SDEGPU_F32 only, 1: the variance and every derivative in
+                           FP64, the log price, the Philox normals and Box-Muller in FP32; where the
                            Feller condition fails the pathwise variance Greeks go
                            through 1/sqrt(v) near v = 0, and FP32 rounding of v moves
                            single paths' values by more than their standard error */

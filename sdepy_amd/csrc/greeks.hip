@@ -8,21 +8,31 @@
 // return is the forward kernel's price and the gradients are those of that
 // estimator (checked against common-random-number finite differences).
 //
-// Heston: the variance recursion is not invertible (max(y, 0)), so the
-// reverse sweep needs the forward states.  They are not stored: pass 1 runs
-// forward and keeps the variance every C steps (checkpoints, C = 8); the
-// reverse sweep then walks the segments backwards, recomputing each segment's
-// variances and normals from its checkpoint and the Philox counters into
-// registers, and sweeping them in reverse.  Memory: ceil(n/C) values per path.
+// Heston: the variance recursion is not invertible (max(y, 0)), so a reverse
+// sweep over the whole path needs its states again.  With an FP64 variance
+// the adjoint sweeps segments of a few steps instead, each right after its
+// forward steps while their partial derivatives are still in registers, for
+// the two adjoint seeds a segment can receive (its final variance and the log
+// price), and chains the segments' results forward; nothing is stored or drawn
+// twice.  FP32 runs sweep the whole path: pass 1 keeps the variance every C
+// steps (checkpoints, C = 8), and the sweep walks the segments backwards,
+// recomputing each segment's variances and normals into registers.  There
+// the order of the FP32 operations shows: where the variance reaches 0, single
+// paths dominate the sums of 1 / sqrt(v), and the segment form moves the
+// variance's Greeks of 4M paths by 6e-7.
 #include "common.hpp"
 #include "philox.hpp"
 
 namespace sdegpu {
 
-// Steps per checkpoint segment (even: one Philox block feeds 2 steps).  8
-// keeps the segment's registers (3 values per step) small enough for 8 waves
-// per SIMD; the checkpoints then cost ~0.7 GB of traffic at 4M x 365.
+// Steps per checkpoint segment of the FP32 adjoint (even: one Philox block
+// feeds 2 steps).  8 keeps the segment's registers (3 values per step) small
+// enough for 8 waves per SIMD; the checkpoints then cost ~0.7 GB of traffic
+// at 4M x 365.
 constexpr int kHestonSeg = 8;
+// Steps per segment of the FP64 adjoint.  1M x 365: 1.48 ms with 2, 1.47 with
+// 4, 1.64 with 8.
+constexpr int kHestonSeg64 = 4;
 constexpr int kHestonNG = 7;    // x0, r, k, theta, xi, rho, y0
 constexpr int kHestonNS = 2 + 2 * kHestonNG;
 constexpr int kLogNG = 5;       // x0, mu, sigma, a, b
@@ -30,7 +40,7 @@ constexpr int kLogNS = 2 + 2 * kLogNG;
 
 struct HestonArgs {
   const void* steps;  // [n][2] (ds, sqrt ds)
-  void* ckpt;         // [nseg][paths]
+  void* ckpt;         // [nseg][paths] (FP32 adjoint)
   double* part;       // [nblocks][kHestonNS]
   int64_t paths;
   int32_t nsteps, payoff;
@@ -132,20 +142,21 @@ __global__ __launch_bounds__(kBlock) void k_heston_table(const T* __restrict__ s
   if (threadIdx.x == 0) *sum_ds = sh[0];
 }
 
-// Reverse-mode adjoint of the full-truncation Heston Euler scheme.
+// Derivatives of the full-truncation Heston Euler scheme.
 //
 // The log-price recursion has unit Jacobian in X, so its adjoint Xbar is the
-// payoff's dP/dX_T at every step and every X-dependent parameter adjoint is a
-// forward sum (d/dr of the drift = Xbar sum ds).  What remains reverse is the
-// variance adjoint: with Vbar the adjoint of V_{n+1}, step n contributes
-//   k:      Vbar (theta - y+) ds          theta: Vbar k ds
-//   xi:     Vbar sv sq w                  rho:   Vbar xi sv sq (z0 - rho/rhoc z1)
-//                                                = xi/rhoc^2 Vbar sv sq (z0 - rho w)
-// and, where V_n > 0 (d y+/dV = 1; 0 otherwise),
-//   Vbar += Vbar (xi sq w / (2 sv) - k ds) + Xbar (sigma sq z0 / (2 sv) - sigma^2/2 ds).
-// k and theta only need S1 = sum Vbar ds and S2 = sum Vbar y+ ds, xi and rho
-// the sums of Vbar sv sq w and Vbar sv sq (z0 - rho w); the constant factors
-// are applied once per path at the end.
+// payoff's dP/dX_T at every step and every Greek is Xbar times the
+// derivative of X_T along a direction.  With
+//   a = 1 - k ds + xi sq w / (2 sv),  b = -sigma^2/2 ds + sigma sq z0 / (2 sv)
+// where V_n > 0 (d y+/dV = 1), a = 1 and b = 0 elsewhere, a step's partial
+// derivatives are dV' = a dV + c, dX' = dX + b dV, with the explicit partials c of
+// the directions
+//   1: ds               k: theta * 1 - 2,  theta: k * 1
+//   2: y+ ds
+//   x: sv sq w          xi
+//   r: sv sq (z0 - rho w)   rho: times xi / rhoc^2
+//   v: none, dV_0 = 1   v0
+// (d/d rho of w = rho z0 + rhoc z1 is z0 - rho/rhoc z1 = (z0 - rho w) / rhoc^2).
 template <typename T>
 __device__ __forceinline__ T pos_part(T v) {
   return v > (T)0 ? v : (T)0;
@@ -159,15 +170,6 @@ __device__ __forceinline__ float pos_part<float>(float v) {
   return __builtin_bit_cast(float, b > 0 ? b : 0);
 }
 
-// Running reverse-sweep state of one path: the variance adjoint and the four
-// parameter sums, all per unit of the constant log-price adjoint Xbar (every
-// term of the variance adjoint is Xbar times a path quantity, so the sweep
-// carries U = Vbar / Xbar and the sums are scaled by Xbar once at the end).
-template <typename T>
-struct HestonRev {
-  T vbar, s1, s2, sx, sr;
-};
-
 // Waves per SIMD the Heston kernels are built for: FP32 8, FP32 with an FP64
 // variance state 4 (its variance registers take twice the room), FP64 1.
 template <typename T, typename TV>
@@ -175,40 +177,153 @@ constexpr int heston_waves() {
   return sizeof(TV) == 8 ? (sizeof(T) == 4 ? 4 : 1) : 8;
 }
 
+// One path's state and the derivatives of (X, V) along the five directions.
+// The log price is held in T, the variance and every derivative in TV (T, or
+// FP64 with FP32 normals).  The normals are those of normals4_folded
+// (divided by kGaussFold<T>): rho and rhoc come multiplied by it, table
+// columns 6 and 9 too, and the rho direction is taken per unit of it
+// (rho_r = rho / kGaussFold<T>).
+template <typename T, typename TV>
+struct HestonPath {
+  T X;
+  TV V;
+  TV x1, v1, x2, v2, xx, vx, xr, vr, xv, vv;
+};
+
+// The partial derivatives of one step (the direction-1 partial is the
+// table's ds).
+template <typename TV>
+struct HestonPartials {
+  TV a, b, c2, cx, cr;
+};
+
+// Steps (X, V) by the table row at rx, r with the normals z0, z1; the partials
+// there.  FLAT forms both selected partials on every lane; otherwise the
+// compiler puts each behind a branch with its own scalar loads and a wait for
+// them.  1M x 365 FP64: adjoint 1.48 ms flat, 1.52 with the branches; tangent
+// 1.53 flat, 1.50 with the branches (FP32, 4M x 365: 2.04 and 1.92).
+template <bool FLAT, typename T, typename TV>
+__device__ __forceinline__ HestonPartials<TV> heston_step(HestonPath<T, TV>& p,
+                                                          const T* __restrict__ rx,
+                                                          const TV* __restrict__ r, T z0t, T z1t,
+                                                          TV rho, TV rhoc, TV rho_r) {
+  HestonPartials<TV> d;
+  const TV z0 = (TV)z0t;
+  const TV w = rho * z0 + rhoc * (TV)z1t;
+  const TV vp = pos_part(p.V);
+  const TV sv = tsqrt<TV>(vp);
+  const TV h = trcp<TV>(sv);
+  const bool pos = sv > (TV)0;
+  if constexpr (FLAT) {
+    TV da = fma(w * r[8], h, r[10]), db = fma(z0 * r[9], h, -r[3]);
+    asm("" : "+v"(da), "+v"(db));
+    d.a = pos ? da : (TV)1;
+    d.b = pos ? db : (TV)0;
+  } else {
+    d.a = pos ? fma(w * r[8], h, r[10]) : (TV)1;
+    d.b = pos ? fma(z0 * r[9], h, -r[3]) : (TV)0;
+  }
+  const TV ssq = sv * r[1];
+  d.c2 = vp * r[0];
+  d.cx = ssq * w;
+  d.cr = ssq * fma(-rho_r, w, z0);
+  // the deterministic r ds terms are added once, after the loop
+  p.X = fma(-rx[3], (T)vp, fma((T)sv * rx[6], z0t, p.X));
+  p.V = p.V + fma(-r[4], vp, fma(sv * r[7], w, r[5]));
+  return d;
+}
+
+// Carries the derivatives over one step (forward mode).
+template <typename T, typename TV>
+__device__ __forceinline__ void heston_tangent_step(HestonPath<T, TV>& p,
+                                                    const HestonPartials<TV>& d, TV ds) {
+  p.x1 = fma(p.v1, d.b, p.x1);
+  p.v1 = fma(p.v1, d.a, ds);
+  p.x2 = fma(p.v2, d.b, p.x2);
+  p.v2 = fma(p.v2, d.a, d.c2);
+  p.xx = fma(p.vx, d.b, p.xx);
+  p.vx = fma(p.vx, d.a, d.cx);
+  p.xr = fma(p.vr, d.b, p.xr);
+  p.vr = fma(p.vr, d.a, d.cr);
+  p.xv = fma(p.vv, d.b, p.xv);
+  p.vv = p.vv * d.a;
+}
+
+template <typename T, typename TV>
+__device__ __forceinline__ HestonPath<T, TV> heston_start(const HestonArgs& a) {
+  HestonPath<T, TV> p = {};
+  p.X = (T)a.lx0;
+  p.V = (TV)a.y0;
+  p.vv = (TV)1;
+  return p;
+}
+
+// Payoff, Greeks and their squares of one path.
+template <typename T, typename TV>
+__device__ __forceinline__ void heston_greeks_of(const HestonArgs& a, const HestonPath<T, TV>& p,
+                                                 double sum_ds, double (&acc)[kHestonNS]) {
+  const double S = exp((double)p.X + a.r * sum_ds);
+  const bool call = a.payoff == 0;
+  const double intr = call ? S - a.strike : a.strike - S;
+  const bool itm = intr > 0.0;
+  const double pay = itm ? a.disc * intr : 0.0;
+  // dP/dX_T = disc * (+-S) on the money
+  const double xbar = itm ? (call ? a.disc * S : -a.disc * S) : 0.0;
+  const double d1 = (double)p.x1;
+  // out of the money every Greek is 0, whatever the derivatives hold
+  const double g[kHestonNG] = {
+      xbar / a.x0,
+      xbar * sum_ds - a.maturity * pay,
+      itm ? xbar * (a.th * d1 - (double)p.x2) : 0.0,
+      itm ? xbar * a.k * d1 : 0.0,
+      itm ? xbar * (double)p.xx : 0.0,
+      itm ? xbar * a.xi / (a.rhoc * a.rhoc) * kGaussFold<T> * (double)p.xr : 0.0,
+      itm ? xbar * (double)p.xv : 0.0};
+  acc[0] = pay;
+  acc[1] = pay * pay;
+#pragma unroll
+  for (int i = 0; i < kHestonNG; ++i) {
+    acc[2 + 2 * i] = g[i];
+    acc[3 + 2 * i] = g[i] * g[i];
+  }
+}
+
+// Running reverse-sweep state of one path: the variance adjoint and the four
+// parameter sums, all per unit of the constant log-price adjoint Xbar (every
+// term of the variance adjoint is Xbar times a path quantity, so the sweep
+// carries U = Vbar / Xbar and the sums are scaled by Xbar once at the end).
+struct HestonRev {
+  float vbar, s1, s2, sx, sr;
+};
+
 // One checkpoint segment of the reverse sweep: recompute the segment's
 // variances and normals from its checkpoint and the Philox counters into
 // registers, then walk its steps backwards.  FULL segments hold C steps.
-// The normals are those of normals4_folded (divided by kGaussFold<T>): rho
-// and rhoc come multiplied by it, table columns 6 and 9 too, and the rho
-// sum is taken per unit of it (rho_sr = rho / kGaussFold<T>).
-// The normals are drawn in T; the variance, its adjoint and the parameter
-// sums are carried in TV (T, or FP64 with FP32 normals), with the step
-// constants of the table tv of that type.
-template <typename T, typename TV, int C, bool FULL>
-__device__ __forceinline__ void heston_segment(const HestonArgs& a, const TV* __restrict__ tv,
-                                               const TV* __restrict__ ck, int64_t gid,
-                                               uint32_t path, int c, int n, TV rho, TV rhoc,
-                                               TV rho_sr, HestonRev<TV>& rv) {
+// rho, rhoc and rho_r as in heston_step.
+template <int C, bool FULL>
+__device__ __forceinline__ void heston_segment(const HestonArgs& a, const float* __restrict__ tb,
+                                               const float* __restrict__ ck, int64_t gid,
+                                               uint32_t path, int c, int n, float rho, float rhoc,
+                                               float rho_r, HestonRev& rv) {
   const int s0 = c * C;
-  TV svs[C], ws[C];
-  T z0s[C];
-  TV v = ck[(int64_t)c * a.paths + gid];
+  float svs[C], ws[C], z0s[C];
+  float v = ck[(int64_t)c * a.paths + gid];
 #pragma unroll
   for (int j = 0; j < C; j += 2) {
     if (FULL || s0 + j < n) {
       __asm__ volatile("" ::: "memory");
-      T z[4];
-      normals4_folded<T>((uint32_t)((s0 + j) >> 1), path, kStreamNormal, a.epoch, a.k0, a.k1,
-                         z);
+      float z[4];
+      normals4_folded<float>((uint32_t)((s0 + j) >> 1), path, kStreamNormal, a.epoch, a.k0, a.k1,
+                             z);
 #pragma unroll
       for (int q = 0; q < 2; ++q) {
         const int s = s0 + j + q;
         z0s[j + q] = z[2 * q];
-        ws[j + q] = rho * (TV)z[2 * q] + rhoc * (TV)z[2 * q + 1];
+        ws[j + q] = rho * z[2 * q] + rhoc * z[2 * q + 1];
         if (FULL || s < n) {
-          const TV* r = tv + (int64_t)s * kHestonTab;
-          const TV vp = pos_part(v);
-          const TV sv = tsqrt<TV>(vp);
+          const float* r = tb + (int64_t)s * kHestonTab;
+          const float vp = pos_part(v);
+          const float sv = tsqrt<float>(vp);
           svs[j + q] = sv;
           v = v + fma(-r[4], vp, fma(sv * r[7], ws[j + q], r[5]));
         }
@@ -222,126 +337,184 @@ __device__ __forceinline__ void heston_segment(const HestonArgs& a, const TV* __
       // keep the scalar table loads next to their step: hoisting all of a
       // segment's rows at once overflows the SGPR file into VGPR lanes
       __asm__ volatile("" ::: "memory");
-      const TV* r = tv + (int64_t)s * kHestonTab;
-      const TV sv = svs[j], z0 = (TV)z0s[j], w = ws[j];
-      const TV vb = rv.vbar;
-      const TV u = vb * r[0];
+      const float* r = tb + (int64_t)s * kHestonTab;
+      const float sv = svs[j], z0 = z0s[j], w = ws[j];
+      const float vb = rv.vbar;
+      const float u = vb * r[0];
       rv.s1 = rv.s1 + u;
       rv.s2 = fma(u, sv * sv, rv.s2);
-      const TV b = vb * (sv * r[1]);
+      const float b = vb * (sv * r[1]);
       rv.sx = fma(b, w, rv.sx);
-      rv.sr = fma(b, fma(-rho_sr, w, z0), rv.sr);
-      const TV h = trcp<TV>(sv);
-      const TV c1 = fma(w, h * r[8], -r[4]);
-      const TV c2 = fma(z0, h * r[9], -r[3]);
-      const TV d = fma(vb, c1, c2);
-      rv.vbar = sv > (TV)0 ? vb + d : vb;
+      rv.sr = fma(b, fma(-rho_r, w, z0), rv.sr);
+      const float h = trcp<float>(sv);
+      const float c1 = fma(w, h * r[8], -r[4]);
+      const float c2 = fma(z0, h * r[9], -r[3]);
+      const float d = fma(vb, c1, c2);
+      rv.vbar = sv > 0.f ? vb + d : vb;
     }
   }
 }
 
-// tb: the step constants in T (the log-price update); tv: the same in TV
-// (the variance, its adjoint and the parameter sums; tv == tb when TV == T).
-template <typename T, typename TV, int C>
-__global__ __launch_bounds__(kBlock, (heston_waves<T, TV>())) void k_heston_adjoint(
-    const HestonArgs a, const T* __restrict__ tb, const TV* __restrict__ tv,
-    TV* __restrict__ ck, const double* __restrict__ sum_ds) {
+// Reverse mode over the whole path in FP32, from variance checkpoints.  The
+// adjoint of V carries U = Vbar / Xbar; k and theta need the sums of U ds and
+// U y+ ds, xi and rho those of U sv sq w and U sv sq (z0 - rho w): the
+// derivatives of X_T along the same directions.
+template <int C>
+__global__ __launch_bounds__(kBlock, (heston_waves<float, float>())) void k_heston_adjoint(
+    const HestonArgs a, const float* __restrict__ tb, float* __restrict__ ck,
+    const double* __restrict__ sum_ds) {
   static_assert(C % 2 == 0, "one Philox block feeds two steps");
-  gauss_init<T>();
   const int64_t gid = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   const bool live = gid < a.paths;
   const uint32_t path = (uint32_t)gid;
   const int64_t P = a.paths;
   const int n = a.nsteps;
-  // the normals come divided by zf (normals4_folded): their coefficients
-  // carry it (table columns 6 and 9 too), the rho sum is per unit of it
-  constexpr double zf = kGaussFold<T>;
-  const TV rho_v = (TV)(a.rho * zf), rhoc_v = (TV)(a.rhoc * zf), rho_sr = (TV)(a.rho / zf);
+  constexpr double zf = kGaussFold<float>;
+  const float rho = (float)(a.rho * zf), rhoc = (float)(a.rhoc * zf), rho_r = (float)(a.rho / zf);
 
   double acc[kHestonNS];
 #pragma unroll
   for (int i = 0; i < kHestonNS; ++i) acc[i] = 0.0;
 
   if (live) {
+    HestonPath<float, float> p = heston_start<float, float>(a);
     // ---- pass 1: forward, variance checkpoints every C steps ----
-    T X = (T)a.lx0;
-    TV V = (TV)a.y0;
     for (int s0 = 0; s0 < n; s0 += 2) {
-      T z[4];
-      normals4_folded<T>((uint32_t)(s0 >> 1), path, kStreamNormal, a.epoch, a.k0, a.k1, z);
+      float z[4];
+      normals4_folded<float>((uint32_t)(s0 >> 1), path, kStreamNormal, a.epoch, a.k0, a.k1, z);
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
         const int s = s0 + j;
         if (s < n) {
-          if (s % C == 0) ck[(int64_t)(s / C) * P + gid] = V;
-          const T* r = tb + (int64_t)s * kHestonTab;
-          const TV* rv = tv + (int64_t)s * kHestonTab;
-          const T z0 = z[2 * j];
-          const TV w = rho_v * (TV)z0 + rhoc_v * (TV)z[2 * j + 1];
-          const TV vp = pos_part(V);
-          const TV sv = tsqrt<TV>(vp);
+          if (s % C == 0) ck[(int64_t)(s / C) * P + gid] = p.V;
+          const float* r = tb + (int64_t)s * kHestonTab;
+          const float z0 = z[2 * j];
+          const float w = rho * z0 + rhoc * z[2 * j + 1];
+          const float vp = pos_part(p.V);
+          const float sv = tsqrt<float>(vp);
           // the deterministic r ds terms are added once, after the loop
-          X = fma(-r[3], (T)vp, fma((T)sv * r[6], z0, X));
-          V = V + fma(-rv[4], vp, fma(sv * rv[7], w, rv[5]));
+          p.X = fma(-r[3], vp, fma(sv * r[6], z0, p.X));
+          p.V = p.V + fma(-r[4], vp, fma(sv * r[7], w, r[5]));
         }
       }
     }
-
-    // ---- payoff and terminal adjoints ----
-    const double S = exp((double)X + a.r * *sum_ds);
-    const bool call = a.payoff == 0;
-    const double intr = call ? S - a.strike : a.strike - S;
-    const bool itm = intr > 0.0;
-    const double pay = itm ? a.disc * intr : 0.0;
-    // dP/dX_T = disc * (+-S) on the money
-    const double xbar = itm ? (call ? a.disc * S : -a.disc * S) : 0.0;
-
     // ---- reverse sweep over the checkpoint segments, per unit of Xbar ----
     // Full segments run without step guards; only the last one can be short.
-    HestonRev<TV> rv{(TV)0, (TV)0, (TV)0, (TV)0, (TV)0};
+    HestonRev rv{0.f, 0.f, 0.f, 0.f, 0.f};
     const int nfull = n / C;
     if (nfull * C < n)
-      heston_segment<T, TV, C, false>(a, tv, ck, gid, path, nfull, n, rho_v, rhoc_v, rho_sr,
-                                      rv);
+      heston_segment<C, false>(a, tb, ck, gid, path, nfull, n, rho, rhoc, rho_r, rv);
     for (int c = nfull - 1; c >= 0; --c)
-      heston_segment<T, TV, C, true>(a, tv, ck, gid, path, c, n, rho_v, rhoc_v, rho_sr, rv);
-    const TV Vbar = rv.vbar, S1 = rv.s1, S2 = rv.s2, Sx = rv.sx, Sr = rv.sr;
-
-    // out of the money every Greek is 0, whatever the per-unit sums hold
-    const double s1 = (double)S1;
-    const double g[kHestonNG] = {xbar / a.x0,
-                                 xbar * *sum_ds - a.maturity * pay,
-                                 itm ? xbar * (a.th * s1 - (double)S2) : 0.0,
-                                 itm ? xbar * a.k * s1 : 0.0,
-                                 itm ? xbar * (double)Sx : 0.0,
-                                 itm ? xbar * a.xi / (a.rhoc * a.rhoc) * zf * (double)Sr : 0.0,
-                                 itm ? xbar * (double)Vbar : 0.0};
-    acc[0] = pay;
-    acc[1] = pay * pay;
-#pragma unroll
-    for (int i = 0; i < kHestonNG; ++i) {
-      acc[2 + 2 * i] = g[i];
-      acc[3 + 2 * i] = g[i] * g[i];
-    }
+      heston_segment<C, true>(a, tb, ck, gid, path, c, n, rho, rhoc, rho_r, rv);
+    p.x1 = rv.s1;
+    p.x2 = rv.s2;
+    p.xx = rv.sx;
+    p.xr = rv.sr;
+    p.xv = rv.vbar;
+    heston_greeks_of(a, p, *sum_ds, acc);
   }
   block_reduce_store<kHestonNS>(acc, a.part);
 }
 
-// Forward-mode (tangent) differentiation of the same scheme.  One forward
-// pass carries, beside (X, V), the derivatives of (X, V) along five
-// directions, so it needs no checkpoints and no recomputation; with this few
-// parameters it issues fewer instructions than the reverse sweep.  Where
-// V_n > 0 (d y+/dV = 1; else a = 1, b = 0):
-//   dV' = a dV + c,  dX' = dX + b dV,
-//   a = 1 - k ds + xi sq w / (2 sv),  b = -sigma^2/2 ds + sigma sq z0 / (2 sv),
-// with the explicit partials c of the directions
-//   1: ds               k: theta * 1 - 2,  theta: k * 1
-//   2: y+ ds
-//   x: sv sq w          xi
-//   r: sv sq (z0 - rho w)   rho: times xi / rhoc^2
-//   v: none, dV_0 = 1   v0
-// and each Greek xbar dX_T along its direction: the same numbers as the
-// adjoint's sums (S1 = dX_1, S2 = dX_2, ...), in another order of operations.
+// Reverse mode segment by segment (FP64 variance).  After the C forward steps of a segment
+// its partials are in registers, and two adjoints are swept back over them
+// together: lam, of the segment's final variance (seed 1), and mu, of the
+// log price (seed 1; its own recursion is the identity).  Per step, with the
+// partials c of each direction,
+//   dX += mu c,  G += lam c,  mu <- a mu + b,  lam <- a lam,
+// so that at the segment's start d X_end/d V_start = mu, d V_end/d V_start =
+// lam and G holds d V_end along the directions; the segments are then chained
+// by dX += mu dV, dV <- lam dV + G.  The last step's sweep is free (lam = 1,
+// mu = 0), which pays for the chaining: 10 FMAs per step.
+//
+// VALU-bound (the Philox draws and Box-Muller are half of the
+// instructions).  The reverse sweep over the whole path drew every normal
+// twice and moved the variance checkpoints: 1M x 365 FP64 2.50 ms with it,
+// 1.47 ms now; FP32 with an FP64 variance 1.67 and 1.07 ms.
+// tb: the step constants in T (the log-price update); tv: the same in TV
+// (tv == tb when TV == T).
+template <typename T, typename TV, int C>
+__global__ __launch_bounds__(kBlock, (heston_waves<T, TV>())) void k_heston_adjoint_seg(
+    const HestonArgs a, const T* __restrict__ tb, const TV* __restrict__ tv,
+    const double* __restrict__ sum_ds) {
+  static_assert(C % 2 == 0, "one Philox block feeds two steps");
+  gauss_init<T>();
+  const int64_t gid = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  const bool live = gid < a.paths;
+  const uint32_t path = (uint32_t)gid;
+  const int n = a.nsteps;
+  constexpr double zf = kGaussFold<T>;
+  const TV rho = (TV)(a.rho * zf), rhoc = (TV)(a.rhoc * zf), rho_r = (TV)(a.rho / zf);
+
+  double acc[kHestonNS];
+#pragma unroll
+  for (int i = 0; i < kHestonNS; ++i) acc[i] = 0.0;
+
+  if (live) {
+    HestonPath<T, TV> p = heston_start<T, TV>(a);
+    int s0 = 0;
+    for (; s0 + C <= n; s0 += C) {
+      HestonPartials<TV> d[C];
+#pragma unroll
+      for (int j = 0; j < C; j += 2) {
+        T z[4];
+        normals4_folded<T>((uint32_t)((s0 + j) >> 1), path, kStreamNormal, a.epoch, a.k0, a.k1,
+                           z);
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          const int64_t row = (int64_t)(s0 + j + q) * kHestonTab;
+          d[j + q] = heston_step<true, T, TV>(p, tb + row, tv + row, z[2 * q], z[2 * q + 1], rho, rhoc,
+                                        rho_r);
+        }
+      }
+      const TV* r = tv + (int64_t)(s0 + C - 1) * kHestonTab;
+      TV g1 = r[0], g2 = d[C - 1].c2, gx = d[C - 1].cx, gr = d[C - 1].cr;
+      TV lam = d[C - 1].a, mu = d[C - 1].b;
+#pragma unroll
+      for (int j = C - 2; j >= 0; --j) {
+        r -= kHestonTab;
+        p.x1 = fma(mu, r[0], p.x1);
+        g1 = fma(lam, r[0], g1);
+        p.x2 = fma(mu, d[j].c2, p.x2);
+        g2 = fma(lam, d[j].c2, g2);
+        p.xx = fma(mu, d[j].cx, p.xx);
+        gx = fma(lam, d[j].cx, gx);
+        p.xr = fma(mu, d[j].cr, p.xr);
+        gr = fma(lam, d[j].cr, gr);
+        mu = fma(mu, d[j].a, d[j].b);
+        lam = lam * d[j].a;
+      }
+      p.x1 = fma(mu, p.v1, p.x1);
+      p.v1 = fma(lam, p.v1, g1);
+      p.x2 = fma(mu, p.v2, p.x2);
+      p.v2 = fma(lam, p.v2, g2);
+      p.xx = fma(mu, p.vx, p.xx);
+      p.vx = fma(lam, p.vx, gx);
+      p.xr = fma(mu, p.vr, p.xr);
+      p.vr = fma(lam, p.vr, gr);
+      p.xv = fma(mu, p.vv, p.xv);
+      p.vv = lam * p.vv;
+    }
+    // the steps past the last whole segment, one at a time
+    for (; s0 < n; s0 += 2) {
+      T z[4];
+      normals4_folded<T>((uint32_t)(s0 >> 1), path, kStreamNormal, a.epoch, a.k0, a.k1, z);
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        if (s0 + q < n) {
+          const int64_t row = (int64_t)(s0 + q) * kHestonTab;
+          const HestonPartials<TV> d = heston_step<true, T, TV>(p, tb + row, tv + row, z[2 * q],
+                                                          z[2 * q + 1], rho, rhoc, rho_r);
+          heston_tangent_step(p, d, tv[row]);
+        }
+      }
+    }
+    heston_greeks_of(a, p, *sum_ds, acc);
+  }
+  block_reduce_store<kHestonNS>(acc, a.part);
+}
+
+// Forward mode (tangent): the derivatives are carried along step by step.
 template <typename T, typename TV>
 __global__ __launch_bounds__(kBlock, (heston_waves<T, TV>())) void k_heston_tangent(
     const HestonArgs a, const T* __restrict__ tb, const TV* __restrict__ tv,
@@ -351,7 +524,6 @@ __global__ __launch_bounds__(kBlock, (heston_waves<T, TV>())) void k_heston_tang
   const bool live = gid < a.paths;
   const uint32_t path = (uint32_t)gid;
   const int n = a.nsteps;
-  // normals divided by zf, as in k_heston_adjoint
   constexpr double zf = kGaussFold<T>;
   const TV rho = (TV)(a.rho * zf), rhoc = (TV)(a.rhoc * zf), rho_r = (TV)(a.rho / zf);
 
@@ -360,68 +532,21 @@ __global__ __launch_bounds__(kBlock, (heston_waves<T, TV>())) void k_heston_tang
   for (int i = 0; i < kHestonNS; ++i) acc[i] = 0.0;
 
   if (live) {
-    // the log price in T, the variance and every derivative in TV
-    T X = (T)a.lx0;
-    TV V = (TV)a.y0;
-    TV x1 = (TV)0, v1 = (TV)0, x2 = (TV)0, v2 = (TV)0, xx = (TV)0, vx = (TV)0;
-    TV xr = (TV)0, vr = (TV)0, xv = (TV)0, vv = (TV)1;
+    HestonPath<T, TV> p = heston_start<T, TV>(a);
     for (int s0 = 0; s0 < n; s0 += 2) {
       T z[4];
       normals4_folded<T>((uint32_t)(s0 >> 1), path, kStreamNormal, a.epoch, a.k0, a.k1, z);
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
-        const int s = s0 + j;
-        if (s < n) {
-          const T* rx = tb + (int64_t)s * kHestonTab;
-          const TV* r = tv + (int64_t)s * kHestonTab;
-          const TV z0 = (TV)z[2 * j];
-          const TV w = rho * z0 + rhoc * (TV)z[2 * j + 1];
-          const TV vp = pos_part(V);
-          const TV sv = tsqrt<TV>(vp);
-          const TV h = trcp<TV>(sv);
-          const bool pos = sv > (TV)0;
-          const TV av = pos ? fma(w * r[8], h, r[10]) : (TV)1;
-          const TV bx = pos ? fma(z0 * r[9], h, -r[3]) : (TV)0;
-          const TV ssq = sv * r[1];
-          const TV c2 = vp * r[0];
-          const TV cx = ssq * w;
-          const TV cr = ssq * fma(-rho_r, w, z0);
-          x1 = fma(v1, bx, x1);
-          v1 = fma(v1, av, r[0]);
-          x2 = fma(v2, bx, x2);
-          v2 = fma(v2, av, c2);
-          xx = fma(vx, bx, xx);
-          vx = fma(vx, av, cx);
-          xr = fma(vr, bx, xr);
-          vr = fma(vr, av, cr);
-          xv = fma(vv, bx, xv);
-          vv = vv * av;
-          X = fma(-rx[3], (T)vp, fma((T)sv * rx[6], z[2 * j], X));
-          V = V + fma(-r[4], vp, fma(sv * r[7], w, r[5]));
+        if (s0 + j < n) {
+          const int64_t row = (int64_t)(s0 + j) * kHestonTab;
+          const HestonPartials<TV> d = heston_step<false, T, TV>(p, tb + row, tv + row, z[2 * j],
+                                                          z[2 * j + 1], rho, rhoc, rho_r);
+          heston_tangent_step(p, d, tv[row]);
         }
       }
     }
-    const double S = exp((double)X + a.r * *sum_ds);
-    const bool call = a.payoff == 0;
-    const double intr = call ? S - a.strike : a.strike - S;
-    const bool itm = intr > 0.0;
-    const double pay = itm ? a.disc * intr : 0.0;
-    const double xbar = itm ? (call ? a.disc * S : -a.disc * S) : 0.0;
-    const double d1 = (double)x1;
-    const double g[kHestonNG] = {xbar / a.x0,
-                                 xbar * *sum_ds - a.maturity * pay,
-                                 xbar * (a.th * d1 - (double)x2),
-                                 xbar * a.k * d1,
-                                 xbar * (double)xx,
-                                 xbar * a.xi / (a.rhoc * a.rhoc) * zf * (double)xr,
-                                 xbar * (double)xv};
-    acc[0] = pay;
-    acc[1] = pay * pay;
-#pragma unroll
-    for (int i = 0; i < kHestonNG; ++i) {
-      acc[2 + 2 * i] = g[i];
-      acc[3 + 2 * i] = g[i] * g[i];
-    }
+    heston_greeks_of(a, p, *sum_ds, acc);
   }
   block_reduce_store<kHestonNS>(acc, a.part);
 }
@@ -580,28 +705,28 @@ __global__ __launch_bounds__(kBlock) void k_sum_columns(const double* __restrict
   if (threadIdx.x == 0) out[c] = sh[0];
 }
 
-// Workspace of one Heston adjoint launch, in this order (each part 256-byte
+// Workspace of one Heston Greeks launch, in this order (each part 256-byte
 // aligned): the per-step table [n][kHestonTab] of the dtype, with an FP64
-// variance state the same table in FP64, the FP64 sum of ds, the variance
-// checkpoints [nseg][paths] (of the variance's type) and the per-block
-// partial sums.
+// variance state the same table in FP64, the FP64 sum of ds, for an FP32
+// adjoint the variance checkpoints [nseg][paths], and the per-block partial
+// sums.
 struct HestonWs {
   size_t tab, tabv, sum, ckpt, part, total;
 };
 
 static size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
-static HestonWs heston_ws(int dtype, bool v64, int64_t paths, int nsteps) {
+static HestonWs heston_ws(int dtype, bool v64, int method, int64_t paths, int nsteps) {
   const size_t es = dtype == SDEGPU_F32 ? 4 : 8;
   const size_t ev = v64 ? 8 : es;
-  const int64_t nseg = (nsteps + kHestonSeg - 1) / kHestonSeg;
   const size_t rows = (size_t)(nsteps > 0 ? nsteps : 1) * kHestonTab;
   HestonWs w;
   w.tab = 0;
   w.tabv = align256(rows * es);
   w.sum = w.tabv + (ev != es ? align256(rows * ev) : 0);
+  const int64_t nseg = ev == 4 && method == 0 ? (nsteps + kHestonSeg - 1) / kHestonSeg : 0;
   w.ckpt = w.sum + 256;
-  w.part = w.ckpt + align256((size_t)(nseg > 0 ? nseg : 1) * (size_t)paths * ev);
+  w.part = w.ckpt + align256((size_t)nseg * (size_t)paths * ev);
   w.total = w.part + (size_t)blocks_for(paths) * kHestonNS * sizeof(double);
   return w;
 }
@@ -612,7 +737,7 @@ using namespace sdegpu;
 
 extern "C" size_t sdegpu_heston_greeks_workspace(const sdegpu_heston_greeks* g) {
   if (!g || g->paths < 1) return 0;
-  return heston_ws(g->dtype, g->variance_f64 != 0, g->paths, g->nsteps).total;
+  return heston_ws(g->dtype, g->variance_f64 != 0, g->method, g->paths, g->nsteps).total;
 }
 
 extern "C" int sdegpu_heston_greeks_run(const sdegpu_heston_greeks* g, double* out, void* ws,
@@ -639,7 +764,7 @@ extern "C" int sdegpu_heston_greeks_run(const sdegpu_heston_greeks* g, double* o
     return fail(SDEGPU_ENOMEM, "heston_greeks: workspace of %zu bytes, %zu needed", ws_bytes, need);
   HestonArgs a = {};
   a.steps = g->steps;
-  const HestonWs lay = heston_ws(g->dtype, v64, g->paths, g->nsteps);
+  const HestonWs lay = heston_ws(g->dtype, v64, g->method, g->paths, g->nsteps);
   char* base = (char*)ws;
   a.ckpt = base + lay.ckpt;
   a.part = (double*)(base + lay.part);
@@ -682,16 +807,15 @@ extern "C" int sdegpu_heston_greeks_run(const sdegpu_heston_greeks* g, double* o
         hipLaunchKernelGGL((k_heston_tangent<float, double>), dim3(nb), dim3(kBlock), 0, st, a,
                            (const float*)tab, (const double*)tabv, (const double*)sum_ds);
       else
-        hipLaunchKernelGGL((k_heston_adjoint<float, double, kHestonSeg>), dim3(nb), dim3(kBlock),
-                           0, st, a, (const float*)tab, (const double*)tabv, (double*)a.ckpt,
+        hipLaunchKernelGGL((k_heston_adjoint_seg<float, double, kHestonSeg64>), dim3(nb), dim3(kBlock),
+                           0, st, a, (const float*)tab, (const double*)tabv,
                            (const double*)sum_ds);
     } else if (g->method == 1) {
       hipLaunchKernelGGL((k_heston_tangent<float, float>), dim3(nb), dim3(kBlock), 0, st, a,
                          (const float*)tab, (const float*)tab, (const double*)sum_ds);
     } else {
-      hipLaunchKernelGGL((k_heston_adjoint<float, float, kHestonSeg>), dim3(nb), dim3(kBlock), 0,
-                         st, a, (const float*)tab, (const float*)tab, (float*)a.ckpt,
-                         (const double*)sum_ds);
+      hipLaunchKernelGGL(k_heston_adjoint<kHestonSeg>, dim3(nb), dim3(kBlock), 0, st, a,
+                         (const float*)tab, (float*)a.ckpt, (const double*)sum_ds);
     }
   } else {
     double* tab = (double*)(base + lay.tab);
@@ -703,8 +827,8 @@ extern "C" int sdegpu_heston_greeks_run(const sdegpu_heston_greeks* g, double* o
       hipLaunchKernelGGL((k_heston_tangent<double, double>), dim3(nb), dim3(kBlock), 0, st, a,
                          (const double*)tab, (const double*)tab, (const double*)sum_ds);
     else
-      hipLaunchKernelGGL((k_heston_adjoint<double, double, kHestonSeg>), dim3(nb), dim3(kBlock),
-                         0, st, a, (const double*)tab, (const double*)tab, (double*)a.ckpt,
+      hipLaunchKernelGGL((k_heston_adjoint_seg<double, double, kHestonSeg64>), dim3(nb), dim3(kBlock),
+                         0, st, a, (const double*)tab, (const double*)tab,
                          (const double*)sum_ds);
   }
   if (int e = launch_status(g->method == 1 ? "k_heston_tangent" : "k_heston_adjoint")) return e;

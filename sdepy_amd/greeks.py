@@ -13,9 +13,9 @@ its preset processes define:
 
 The kernels run the forward Euler pass on the same Philox draws as the
 process classes (a process built with the same ``rng`` seed gives the same
-paths) and sweep the adjoint backwards; for Heston the variance path is
-recomputed segment by segment from checkpoints and the Philox counters, so no
-path history is stored.  ``heston_price_fd`` is the FP64 forward plus central
+paths) and sweep the adjoint backwards; for Heston over segments of the path,
+each while its partial derivatives are in registers, so no path history is
+stored or recomputed.  ``heston_price_fd`` is the FP64 forward plus central
 finite-difference baseline on common random numbers.
 
 ``HestonPrice.apply(params, config)`` exposes the price to torch autograd:
@@ -119,13 +119,12 @@ class GreeksResult:
 class HestonGreeks:
     """A prepared Heston Greeks run (step table, workspace and output on the
     device); ``launch()`` issues the kernels, ``result()`` reads the sums.
-    ``method='adjoint'`` sweeps the reverse-mode adjoint over recomputed
-    checkpoint segments; ``method='tangent'`` carries the five derivative
-    directions along the forward pass instead (fewer instructions for this
-    few parameters); both give the same pathwise estimator.
-    ``variance_dtype=np.float64`` with an FP32 run carries the variance, its
-    checkpoints and its adjoint (every derivative, in forward mode) in FP64,
-    with the log price and the normals in FP32."""
+    ``method='adjoint'`` sweeps the reverse-mode adjoint over segments of the
+    path and chains them; ``method='tangent'`` carries the five derivative
+    directions along the forward pass step by step; both give the same
+    pathwise estimator.
+    ``variance_dtype=np.float64`` with an FP32 run carries the variance and
+    every derivative in FP64, with the log price and the normals in FP32."""
 
     def __init__(self, *, x0=100., r=0.02, sigma=1., k=2., theta=.04, xi=.5,
                  rho=-.7, y0=.04, strike=100., maturity=1., steps=365,
