@@ -137,6 +137,57 @@ __device__ __forceinline__ double fast_sqrt<double>(double v) {
   return sqrt(v);
 }
 
+// One step of cox_ingersoll_ross_SDE (integration.py:2360-2365):
+// x+ = max(x, 0); {'dt': k*(theta - x+), 'dw': xi*sqrt(x+)}.
+template <typename T>
+__device__ __forceinline__ T cir_next(T x, T theta, T k, T xi, T ds, T dw) {
+  const T xp = x > (T)0 ? x : (T)0;
+  const T adt = k * (theta - xp);
+  const T adw = xi * fast_sqrt<T>(xp);
+  return x + (adt * ds + adw * dw);
+}
+
+// One step of one pair of full_heston_SDE (full truncation): y+ = max(y, 0);
+//   log x: {'dt': mu - sigma*sigma*y+/2, 'dw': sigma*sqrt(y+)}
+//   y:     {'dt': k*(theta - y+),        'dw': xi*sqrt(y+)}
+// cnt counts the steps that start at y < 0.
+template <typename T>
+__device__ __forceinline__ void heston_next(T& x, T& y, int& cnt, T mu, T sig, T th, T kk, T xi,
+                                            T ds, T dwx, T dwy) {
+  cnt += (y < (T)0) ? 1 : 0;
+  const T yp = y > (T)0 ? y : (T)0;
+  const T sy = fast_sqrt<T>(yp);
+  const T axt = mu - sig * sig * yp * (T)0.5;
+  const T axw = sig * sy;
+  const T ayt = kk * (th - yp);
+  const T ayw = xi * sy;
+  x = x + (axt * ds + axw * dwx);
+  y = y + (ayt * ds + ayw * dwy);
+}
+
+// The word below which every Poisson word of a pass is a count of 0: a word w
+// draws 0 when (w + 0.5) 2^-32 <= exp(-lam |ds|), so every w below the smallest
+// exp(-lam |ds|) 2^32 of the n table rows does, whatever its step; words
+// at or above it take the inversion, which re-checks.  Costs a step one
+// integer comparison with a scalar where forming and comparing the FP64
+// uniform, selecting the sum and counting took a dozen instructions: Merton
+// 2M x 252 FP32, 2 rows 691 -> 562 us, 253 rows 1087 -> 964 us (a bound per
+// step, from the table or beside it, cost more than it saved).  Every thread
+// of the block must call it.
+__device__ __forceinline__ uint32_t zero_count_bound(const double* __restrict__ pois, int64_t n) {
+  __shared__ double sh[16];
+  double p = 1.0;
+  for (int64_t i = threadIdx.x; i < n; i += blockDim.x) p = fmin(p, pois[2 * i + 1]);
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) p = fmin(p, __shfl_xor(p, off, 64));
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = p;
+  __syncthreads();
+  for (unsigned w = 0; w < blockDim.x >> 6; ++w) p = fmin(p, sh[w]);
+  const double b = p * 0x1p32;
+  const uint32_t bound = b < 0x1p32 ? (uint32_t)b : 0xFFFFFFFFu;
+  return __builtin_amdgcn_readfirstlane(bound);
+}
+
 // Heston working state (SDEs.pack, integration.py:1759-1783, with the two
 // equations stacked on the last vshape axis of length D): groups of 2D
 // components, D log x followed by the D y of the same leading index.  The
@@ -367,6 +418,10 @@ __global__ __launch_bounds__(kBlock, MOM ? 8 : 1) void k_euler(const EulerArgs a
   constexpr int N = kHeston ? M / 2 : M;
 
   gauss_init<T>();
+  // words below it are counts of 0 (per-path intensities: none are known to be)
+  const uint32_t zero_below = kJump && !(GEN && (a.replay_dj || a.lamp))
+                                  ? zero_count_bound(pois, (int64_t)a.nsteps * M)
+                                  : 0u;
   // With fused row moments every thread of the block takes part in the LDS
   // reductions, so the lanes beyond the last path step a copy of the last
   // path and store nothing; otherwise they leave at once.
@@ -458,9 +513,9 @@ __global__ __launch_bounds__(kBlock, MOM ? 8 : 1) void k_euler(const EulerArgs a
   // stored steps are sparse; with a store at most steps the bookkeeping
   // costs more than it saves.
   constexpr int kJumpEvents = 4;
-  uint32_t jev[kDefer ? kJumpEvents : 1];
-#pragma unroll
-  for (int k = 0; k < (kDefer ? kJumpEvents : 1); ++k) jev[k] = 0u;
+  // one LDS column per lane: recording an event is a store at a lane-computed
+  // address, not a select into each of 4 registers
+  __shared__ uint32_t jev[kDefer ? kJumpEvents : 1][kDefer ? kBlock : 1];
   int njev = 0;
   // sum of the n jump sizes of component v at step s, of the law whose
   // parameters are the step row's blocks 2, 3 (and 4 but for the normal law)
@@ -471,18 +526,16 @@ __global__ __launch_bounds__(kBlock, MOM ? 8 : 1) void k_euler(const EulerArgs a
                          pr[3 * M + v], p2);
   };
   auto flush_jumps = [&]() {
-    while (njev > 0) {
-      const uint32_t e = jev[0];
+    for (int q = 0; q < njev; ++q) {
+      const uint32_t e = jev[q][threadIdx.x];
       const int s = (int)(e >> 12), v = (int)((e >> 8) & 7u), n = (int)(e & 255u);
       const T* pr = coef + (int64_t)s * a.ncoef + a.poff;
       T acc = jump_sum(s, v, n, pr);
       acc = (e >> 11) & 1u ? -acc : acc;
 #pragma unroll
       for (int w = 0; w < M; ++w) x[w] = x[w] + (w == v ? acc : (T)0);
-#pragma unroll
-      for (int q = 0; q + 1 < kJumpEvents; ++q) jev[q] = jev[q + 1];
-      --njev;
     }
+    njev = 0;
   };
 
   const bool replay = GEN && a.replay_dw != nullptr;
@@ -606,44 +659,28 @@ __global__ __launch_bounds__(kBlock, MOM ? 8 : 1) void k_euler(const EulerArgs a
           for (int v = 0; v < M; ++v) x[v] = p[v] * x[v] + (p[M + v] + p[2 * M + v] * dw[v]);
         }
       } else if constexpr (MODEL == SDEGPU_MODEL_CIR) {
-        // cox_ingersoll_ross_SDE: x+ = max(x, 0); {'dt': k*(theta - x+), 'dw': xi*sqrt(x+)}
 #pragma unroll
-        for (int v = 0; v < M; ++v) {
-          const T xp = x[v] > (T)0 ? x[v] : (T)0;
-          const T adt = p[M + v] * (p[v] - xp);
-          const T adw = p[2 * M + v] * fast_sqrt<T>(xp);
-          x[v] = x[v] + (adt * ds + adw * dw[v]);
-        }
+        for (int v = 0; v < M; ++v)
+          x[v] = cir_next<T>(x[v], p[v], p[M + v], p[2 * M + v], ds, dw[v]);
       } else if constexpr (kHeston) {
-        // full_heston_SDE (full truncation): y+ = max(y, 0);
-        //   log x: {'dt': mu - sigma*sigma*y+/2, 'dw': sigma*sqrt(y+)}
-        //   y:     {'dt': k*(theta - y+),        'dw': xi*sqrt(y+)}
         using L = HestonLayout<D>;
 #pragma unroll
         for (int i = 0; i < N; ++i) {
           const int ix = L::xi(i), iy = L::yi(i);
-          const T y = x[iy];
-          cnt[i] += (y < (T)0) ? 1 : 0;
-          const T yp = y > (T)0 ? y : (T)0;
-          const T sy = fast_sqrt<T>(yp);
-          const T mu = p[i], sig = p[N + i], th = p[2 * N + i], kk = p[3 * N + i],
-                  xi = p[4 * N + i];
-          const T axt = mu - sig * sig * yp * (T)0.5;
-          const T axw = sig * sy;
-          const T ayt = kk * (th - yp);
-          const T ayw = xi * sy;
-          x[ix] = x[ix] + (axt * ds + axw * dw[ix]);
-          x[iy] = y + (ayt * ds + ayw * dw[iy]);
+          heston_next<T>(x[ix], x[iy], cnt[i], p[i], p[N + i], p[2 * N + i], p[3 * N + i],
+                         p[4 * N + i], ds, dw[ix], dw[iy]);
         }
       } else if constexpr (kJump) {
         // jumpdiff_SDE: {'dt': mu - sigma^2/2, 'dw': sigma, 'dj': 1}, no martingale correction;
         // dj = sign(ds) * sum of n ~ Poisson(lam*|ds|) jump sizes of the law
         // jump_law (cpoisson_source.__call__; norm_rv(a, b) for Merton).
-        T dj[M];
+        T inc[M];
+#pragma unroll
+        for (int v = 0; v < M; ++v) inc[v] = p[v] * ds + p[M + v] * dw[v];
         if (replay_j) {
           const T* rp = (const T*)a.replay_dj + ((int64_t)s * mt + c0) * P + gid;
 #pragma unroll
-          for (int v = 0; v < M; ++v) dj[v] = rp[v * P];
+          for (int v = 0; v < M; ++v) inc[v] = inc[v] + rp[v * P];
         } else {
           const double* pq = pois + (int64_t)s * M * 2;
           const bool neg = ds < (T)0;
@@ -652,6 +689,7 @@ __global__ __launch_bounds__(kBlock, MOM ? 8 : 1) void k_euler(const EulerArgs a
           const bool stored = store_row[s] >= 0;
 #pragma unroll
           for (int v = 0; v < M; ++v) {
+            if (upois[k * M + v] < zero_below) continue;
             double lamds = pq[2 * v], p0 = pq[2 * v + 1];
             if (GEN && a.lamp) {
               // per-path intensity: pois holds |ds|
@@ -659,26 +697,22 @@ __global__ __launch_bounds__(kBlock, MOM ? 8 : 1) void k_euler(const EulerArgs a
               p0 = exp(-lamds);
             }
             const int n = poisson_inv(u01_f64(upois[k * M + v]), lamds, p0, kPoissonCap);
-            T acc = (T)0;
             if (n > 0) {
               if (kDefer && !stored && njev < kJumpEvents && n < 256 && s < (1 << 20)) {
-                const uint32_t e = ((uint32_t)s << 12) | ((neg ? 1u : 0u) << 11) |
-                                   ((uint32_t)v << 8) | (uint32_t)n;
-#pragma unroll
-                for (int q = 0; q < kJumpEvents; ++q) jev[q] = njev == q ? e : jev[q];
+                jev[njev][threadIdx.x] = ((uint32_t)s << 12) | ((neg ? 1u : 0u) << 11) |
+                                         ((uint32_t)v << 8) | (uint32_t)n;
                 ++njev;
               } else {
-                acc = jump_sum(s, v, n, c + a.poff);
+                const T acc = jump_sum(s, v, n, c + a.poff);
+                inc[v] = inc[v] + (neg ? -acc : acc);
               }
+              cnt[v] += neg ? -n : n;
+              interval_jumps += neg ? -n : n;
             }
-            dj[v] = neg ? -acc : acc;
-            cnt[v] += neg ? -n : n;
-            interval_jumps += neg ? -n : n;
           }
         }
 #pragma unroll
-        for (int v = 0; v < M; ++v)
-          x[v] = x[v] + ((p[v] * ds + p[M + v] * dw[v]) + dj[v]);
+        for (int v = 0; v < M; ++v) x[v] = x[v] + inc[v];
       }
 
       const int row = store_row[s];

@@ -175,18 +175,8 @@ __global__ __launch_bounds__(kBlock) void k_euler_wide(const EulerArgs a,
 #pragma unroll
       for (int i = 0; i < H; ++i) {
         if (i < n) {
-          const T y = vy[i];
-          cnt[i] += (y < (T)0) ? 1 : 0;
-          const T yp = y > (T)0 ? y : (T)0;
-          const T sy = fast_sqrt<T>(yp);
-          const T mu = par(p, 0, i), sig = par(p, 1, i), th = par(p, 2, i), kk = par(p, 3, i),
-                  xi = par(p, 4, i);
-          const T axt = mu - sig * sig * yp * (T)0.5;
-          const T axw = sig * sy;
-          const T ayt = kk * (th - yp);
-          const T ayw = xi * sy;
-          x[i] = x[i] + (axt * ds + axw * zx[i]);
-          vy[i] = y + (ayt * ds + ayw * zy[i]);
+          heston_next<T>(x[i], vy[i], cnt[i], par(p, 0, i), par(p, 1, i), par(p, 2, i),
+                         par(p, 3, i), par(p, 4, i), ds, zx[i], zy[i]);
         }
       }
     } else {
@@ -257,12 +247,8 @@ __global__ __launch_bounds__(kBlock) void k_euler_wide(const EulerArgs a,
       } else if constexpr (MODEL == SDEGPU_MODEL_CIR) {
 #pragma unroll
         for (int v = 0; v < W; ++v) {
-          if (v < m) {
-            const T xp = x[v] > (T)0 ? x[v] : (T)0;
-            const T adt = par(p, 1, v) * (par(p, 0, v) - xp);
-            const T adw = par(p, 2, v) * fast_sqrt<T>(xp);
-            x[v] = x[v] + (adt * ds + adw * z[v]);
-          }
+          if (v < m)
+            x[v] = cir_next<T>(x[v], par(p, 0, v), par(p, 1, v), par(p, 2, v), ds, z[v]);
         }
       } else if constexpr (kJump) {
         // each component's jump total is added as it is drawn (no dj array:
