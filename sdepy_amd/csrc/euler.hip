@@ -1,6 +1,7 @@
 // Entry point of the Euler path kernels (the kernels are in euler_kernel.hpp):
 // validation of the problem, the kernel choice and the launch.
 #include "euler_kernel.hpp"
+#include "euler_split.hpp"
 #include "euler_wide.hpp"
 
 namespace sdegpu {
@@ -40,6 +41,31 @@ static uint32_t expected_exp_mask(int model, int m, int nout, int d) {
   for (int o = 0; o < m && o < 32; ++o)
     if (o % (2 * d) < d) mask |= 1u << o;
   return mask;
+}
+
+// Waves that share 64 paths (k_euler_split); 1: one wave each (k_euler).
+//
+// One wave per 64 paths leaves SIMDs idle below 1024 of them (256 CUs of 4); up to there
+// sharing wins, above it the repeated recursion costs more than the idle slots
+// give (100,000 paths, lognormal FP64 full path: 91 us alone, 94 with 8).
+// Twice the share for the models whose recursion is a sum or an FMA: 4096
+// waves for them, 2048 for Heston and CIR, whose every wave repeats a square
+// root per step.  Microseconds for 252 steps alone / with 2, 4, 8 waves:
+//   lognormal FP64, 253 rows   10,000 paths  79 / 53, 32, 25
+//                              32,768        79 / 67, 40, 36
+//                              65,536        78 / 66, 60, 63
+//   Heston FP64, 253 rows      10,000       160 / 115, 79, 77
+//                              32,768       159 / 141, 99, 119
+//                              65,536       160 / 142, 159, 223
+//   Kou FP32, 2 rows           10,000        62 / 52, 35, 28
+//                              65,536        63 / 59, 50, 56
+static int split_waves(int64_t paths, int model) {
+  constexpr int64_t kSimds = 1024;
+  const int64_t waves = (paths + 63) / 64;
+  if (waves > kSimds) return 1;
+  const bool root = model == SDEGPU_MODEL_HESTON || model == SDEGPU_MODEL_CIR;
+  const int64_t room = (root ? 2 : 4) * kSimds / waves;
+  return room >= 8 ? 8 : room >= 4 ? 4 : 2;
 }
 
 static int param_blocks(int model, int m) {
@@ -210,6 +236,24 @@ extern "C" int sdegpu_euler(const sdegpu_euler_problem* pr, void* stream) {
                 "fused row moments with per-path parameters: reduce the output separately");
   const dim3 grid(blocks_for(pr->paths)), block(kBlock);
   hipStream_t st = (hipStream_t)stream;
+  // runs of few paths: several waves share 64 paths
+  const bool can_split = !wide && !mom && !pp && !grouped && !pr->replay_dw && !pr->replay_dj &&
+                         !(jump && pr->lam_paths);
+  const int share = can_split ? split_waves(pr->paths, pr->model) : 1;
+  if (share > 1) {
+    const dim3 sgrid(blocks_for(pr->paths, 64)), sblock(64 * share);
+    if (pr->dtype == SDEGPU_F32) {
+      if (EulerKernel<float> k = euler_split_kernel<float>(pr->model, m, hd)) {
+        hipLaunchKernelGGL(k, sgrid, sblock, 0, st, a, (const float*)pr->coef, pr->store_row,
+                           pr->pois, (float*)pr->out);
+        return launch_status("k_euler_split");
+      }
+    } else if (EulerKernel<double> k = euler_split_kernel<double>(pr->model, m, hd)) {
+      hipLaunchKernelGGL(k, sgrid, sblock, 0, st, a, (const double*)pr->coef, pr->store_row,
+                         pr->pois, (double*)pr->out);
+      return launch_status("k_euler_split");
+    }
+  }
   if (pr->dtype == SDEGPU_F32) {
     EulerKernel<float> k = wide ? euler_wide_kernel<float>(pr->model, m)
                                 : choose<float>(plain, mom, pp, pr->model, m, hd, defer);

@@ -134,7 +134,7 @@ __device__ __forceinline__ float fast_sqrt<float>(float v) {
 }
 template <>
 __device__ __forceinline__ double fast_sqrt<double>(double v) {
-  return sqrt(v);
+  return sqrt_nonneg(v);
 }
 
 // One step of cox_ingersoll_ross_SDE (integration.py:2360-2365):
@@ -174,15 +174,16 @@ __device__ __forceinline__ void heston_next(T& x, T& y, int& cnt, T mu, T sig, T
 // 2M x 252 FP32, 2 rows 691 -> 562 us, 253 rows 1087 -> 964 us (a bound per
 // step, from the table or beside it, cost more than it saved).  Every thread
 // of the block must call it.
-__device__ __forceinline__ uint32_t zero_count_bound(const double* __restrict__ pois, int64_t n) {
+__device__ __forceinline__ uint32_t zero_count_bound(const double* __restrict__ pois, int64_t n,
+                                                     unsigned threads = kBlock) {
   __shared__ double sh[16];
   double p = 1.0;
-  for (int64_t i = threadIdx.x; i < n; i += blockDim.x) p = fmin(p, pois[2 * i + 1]);
+  for (int64_t i = threadIdx.x; i < n; i += threads) p = fmin(p, pois[2 * i + 1]);
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) p = fmin(p, __shfl_xor(p, off, 64));
   if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = p;
   __syncthreads();
-  for (unsigned w = 0; w < blockDim.x >> 6; ++w) p = fmin(p, sh[w]);
+  for (unsigned w = 0; w < threads >> 6; ++w) p = fmin(p, sh[w]);
   const double b = p * 0x1p32;
   const uint32_t bound = b < 0x1p32 ? (uint32_t)b : 0xFFFFFFFFu;
   return __builtin_amdgcn_readfirstlane(bound);

@@ -142,13 +142,14 @@ __device__ __forceinline__ GaussTab& gauss_tab() {
 }
 
 // Every kernel that draws normals (or exponentials) in T calls this first,
-// with all threads of the block: FP64 needs its tables in LDS, FP32 nothing.
+// with all threads of the block (256 unless given): FP64 needs its tables in
+// LDS, FP32 nothing.
 template <typename T>
-__device__ __forceinline__ void gauss_init() {
+__device__ __forceinline__ void gauss_init(unsigned threads = 256) {
   if constexpr (sizeof(T) == 8) {
     const uint4* src = reinterpret_cast<const uint4*>(&kGaussTab);
     uint4* dst = reinterpret_cast<uint4*>(&gauss_tab());
-    for (unsigned i = threadIdx.x; i < sizeof(GaussTab) / sizeof(uint4); i += blockDim.x)
+    for (unsigned i = threadIdx.x; i < sizeof(GaussTab) / sizeof(uint4); i += threads)
       dst[i] = src[i];
     __syncthreads();
   }
@@ -187,6 +188,19 @@ __device__ __forceinline__ double sqrt_mid(double v) {
   g = fma(g, e, g);
   h = fma(h, e, h);
   return fma(fma(-g, g, v), h, g);
+}
+
+// sqrt(v) for v >= 0 (0, infinity and NaN as sqrt gives them; below 1e-300 only
+// the order of magnitude): sqrt_mid's steps without the scaling of tiny
+// arguments that a full-range sqrt takes.
+__device__ __forceinline__ double sqrt_nonneg(double v) {
+  const double y = __builtin_amdgcn_rsq(fmax(v, 1e-300));
+  double g = v * y, h = 0.5 * y;
+  const double e = fma(-h, g, 0.5);
+  g = fma(g, e, g);
+  h = fma(h, e, h);
+  g = fma(fma(-g, g, v), h, g);
+  return v == __builtin_inf() ? v : g;
 }
 
 template <>

@@ -698,6 +698,14 @@ class _Pass:
             _lib.check(_lib.lib().sdegpu_euler(p, st))
 
 
+# Paths up to which prepare(moments=True) reduces the rows by a pass after the
+# kernels: there several waves share 64 paths (k_euler_split, up to 1024 waves
+# of paths), which the kernels with the moments fused in do not, and the rows
+# are still in the caches.  10,000 x 252 lognormal FP64, launch and both moments
+# read back: 110 us, 172 us with the moments fused in.
+_SEPARATE_PATHS = 65536
+
+
 class PreparedRun:
     """A simulation with its tables uploaded and its output allocated on the
     device (``xx_dev``, shaped (N_t, nout, paths)).  ``launch()`` may be
@@ -707,12 +715,13 @@ class PreparedRun:
     def __init__(self, sde, passes, xx_dev, tt, tt_asis, odt):
         self.sde, self.passes, self.xx_dev = sde, passes, xx_dev
         self.tt, self.tt_asis, self.odt = tt, tt_asis, odt
-        self._row_mom = None
+        self._row_mom = self._mom_mean = self._mom_ws = None
 
     def _fuse_moments(self):
         """Have every pass reduce its stored rows as it stores them: block
         partials [ceil(paths/256)][rows][2], merged after each launch into
-        the FP64 (mean, m2) of every row."""
+        the FP64 (mean, m2) of every row.  Runs of few paths are reduced by
+        a pass of its own within the launch (_SEPARATE_PATHS)."""
         if any(prob.param_paths or prob.nvars > _lib.MAX_VARS
                for p in self.passes for prob in p.probs):
             # per-path parameters or a wide coupled block: the separate
@@ -720,10 +729,14 @@ class PreparedRun:
             return
         n_t, nout, P = self.xx_dev.shape
         rows = n_t * nout
-        nblocks = (P + 255) // 256
-        self._row_mom = _lib.empty((nblocks, rows, 2), np.float64)
         self._mom_mean = _lib.empty((rows,), np.float64)
         self._mom_m2 = _lib.empty((rows,), np.float64)
+        if P <= _SEPARATE_PATHS:
+            self._mom_nbytes = _lib.lib().sdegpu_moments_workspace(rows, P)
+            self._mom_ws = _lib.workspace(self._mom_nbytes)
+            return
+        nblocks = (P + 255) // 256
+        self._row_mom = _lib.empty((nblocks, rows, 2), np.float64)
         for p in self.passes:
             for prob in p.probs:
                 prob.row_moments = self._row_mom.data_ptr()
@@ -739,6 +752,13 @@ class PreparedRun:
             _lib.check(_lib.lib().sdegpu_row_moments_merge(
                 _lib.ptr(self._row_mom), n_t * nout, P, _lib.ptr(self._mom_mean),
                 _lib.ptr(self._mom_m2), _lib.stream()))
+        elif self._mom_ws is not None:
+            n_t, nout, P = self.xx_dev.shape
+            _lib.check(_lib.lib().sdegpu_path_moments(
+                _lib.ptr(self.xx_dev),
+                _lib.F32 if self.xx_dev.dtype == _lib.torch_mod().float32 else _lib.F64,
+                n_t * nout, P, _lib.ptr(self._mom_mean), _lib.ptr(self._mom_m2),
+                _lib.ptr(self._mom_ws), self._mom_nbytes, _lib.stream()))
 
     def result(self):
         for p in self.passes:
@@ -774,8 +794,8 @@ class PreparedRun:
         return sde._result(self.tt_asis, xx)
 
     def _moments(self):
-        if self._row_mom is not None:
-            # reduced by the kernels as they stored the rows
+        if self._mom_mean is not None:
+            # reduced within the launch
             shape = self.xx_dev.shape[:2]
             return (float(self.xx_dev.shape[2]),
                     _lib.to_host(self._mom_mean).reshape(shape),
