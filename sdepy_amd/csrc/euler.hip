@@ -234,7 +234,10 @@ extern "C" int sdegpu_euler(const sdegpu_euler_problem* pr, void* stream) {
   if (pp && mom)
     return fail(SDEGPU_EUNSUPPORTED,
                 "fused row moments with per-path parameters: reduce the output separately");
-  const dim3 grid(blocks_for(pr->paths)), block(kBlock);
+  const int block_paths = wide ? 64 : kBlock;
+  const dim3 grid(blocks_for(pr->paths, block_paths));
+  const dim3 block(wide ? 64 * wide_shape(pr->model, m).waves : kBlock);
+  const bool wide_gen = pr->replay_dw || pr->replay_dj || pp || (jump && pr->lam_paths);
   hipStream_t st = (hipStream_t)stream;
   // runs of few paths: several waves share 64 paths
   const bool can_split = !wide && !mom && !pp && !grouped && !pr->replay_dw && !pr->replay_dj &&
@@ -255,13 +258,13 @@ extern "C" int sdegpu_euler(const sdegpu_euler_problem* pr, void* stream) {
     }
   }
   if (pr->dtype == SDEGPU_F32) {
-    EulerKernel<float> k = wide ? euler_wide_kernel<float>(pr->model, m)
+    EulerKernel<float> k = wide ? euler_wide_kernel<float>(pr->model, m, wide_gen)
                                 : choose<float>(plain, mom, pp, pr->model, m, hd, defer);
     if (!k) return fail(SDEGPU_EUNSUPPORTED, "no kernel for model %d with %d components", pr->model, m);
     hipLaunchKernelGGL(k, grid, block, 0, st, a, (const float*)pr->coef, pr->store_row,
                        pr->pois, (float*)pr->out);
   } else {
-    EulerKernel<double> k = wide ? euler_wide_kernel<double>(pr->model, m)
+    EulerKernel<double> k = wide ? euler_wide_kernel<double>(pr->model, m, wide_gen)
                                  : choose<double>(plain, mom, pp, pr->model, m, hd, defer);
     if (!k) return fail(SDEGPU_EUNSUPPORTED, "no kernel for model %d with %d components", pr->model, m);
     hipLaunchKernelGGL(k, grid, block, 0, st, a, (const double*)pr->coef, pr->store_row,

@@ -5,29 +5,53 @@
 // (wiener_source.__call__, infrastructure.py:1524-1553) and steps it with the
 // same euler_next update as any other state (integration.py:707-723).
 //
-// The block's width m is a run-time value (EulerArgs::nvars); the kernel is
-// compiled for a capacity W of 16, 32 or 64 components, holds the state in W
-// registers and guards every component loop by v < m (uniform over the
-// wave).  It does everything the general k_euler instance does (component
-// groups, recorded increments, antithetic halves, per-path parameters,
-// correlation tables that change in time, the jump laws and the jump
-// information, the backward pass) except the fused row moments and the
-// deferred jump form: the jumps are summed in place, in sdepy's order.
+// W waves share 64 paths and split the components: wave w holds components
+// (Heston: pairs) w, w + W, w + 2 W, ..., at most R of them.  Per step the
+// waves draw the block's normals together, one Philox block of 4 after the
+// other, into LDS, and after a barrier each applies its rows of the
+// correlation and steps its components; the cyclic rows give every wave about
+// the same share of the triangle.  The step's table row is fetched a step ahead and
+// spread out in LDS as a square with zeros above the diagonal, so that a wave
+// reads its coefficients as 16-byte broadcasts at fixed offsets (with scalar
+// loads and a wait per piece of a row the kernel took twice as long).  Bound
+// by LDS reads and VALU about equally.  One lane per path with the whole
+// state, which this replaces, took up to 256 registers, one or two waves
+// per SIMD, and its FP64 jump instances spilled: 100,000 paths x 252 steps of
+// 20 correlated lognormals FP64 2.54 ms, 1.64 ms now; 64 of them, 20,000 x
+// 100, 4.88 and 1.12 ms; FP32 12 of them, 200,000 x 100, 0.68 and 0.28 ms.
+//
+// The block's width m is a run-time value.  The kernel does everything the
+// general k_euler instance does (component groups, recorded increments,
+// antithetic halves, per-path parameters, correlation tables that change in
+// time, the jump laws and the jump information, the backward pass) except the
+// fused row moments and the deferred jump form: the jumps are summed in place,
+// in sdepy's order.
 //
 // Correlation: dw = L z sqrt|ds| with the packed Cholesky rows of the step,
-// row i summed over j = 0..i in order, as in k_euler.  It is computed in
-// place from the last row to the first (row i reads z_0..z_i, which the rows
-// below it have not overwritten), so z and dw share registers.  The Heston
-// state [log x_0..x_{n-1}, y_0..y_{n-1}] is held as two arrays of W/2, so
-// that pair i reads its variance at a compile-time index; its correlation
-// rows are split the same way (the y rows first: they read every x normal).
+// row i summed over j = 0..i in order, as in k_euler; the sum runs on over the zeros
+// of the square (of the coefficients and of the normals past the width).
 #pragma once
 #include "euler_kernel.hpp"
 
 namespace sdegpu {
 
-template <int MODEL, typename T, int W>
-__global__ __launch_bounds__(kBlock) void k_euler_wide(const EulerArgs a,
+template <bool B>
+struct Flag {
+  static constexpr bool value = B;
+};
+
+// The square of one row's coefficients: N rows and columns, the columns
+// padded to whole 16-byte reads.
+template <typename T, int N>
+struct WideSquare {
+  static constexpr int CK = 16 / sizeof(T);  // coefficients per LDS read
+  static constexpr int COLS = (N + CK - 1) / CK * CK;
+  static constexpr int SIZE = N * COLS;
+};
+
+// GEN: recorded increments, per-path parameters and per-path intensities.
+template <int MODEL, typename T, int W, int R, bool GEN>
+__global__ __launch_bounds__(64 * W) void k_euler_wide(const EulerArgs a,
                                                        const T* __restrict__ coef,
                                                        const int32_t* __restrict__ store_row,
                                                        const double* __restrict__ pois,
@@ -35,274 +59,342 @@ __global__ __launch_bounds__(kBlock) void k_euler_wide(const EulerArgs a,
   constexpr bool kJump = MODEL == SDEGPU_MODEL_JUMPDIFF;
   constexpr bool kHeston = MODEL == SDEGPU_MODEL_HESTON;
   constexpr bool kOU = MODEL == SDEGPU_MODEL_OU;
-  constexpr int H = W / 2;
-  constexpr int NS = kHeston ? H : W;  // state arrays, and counters of the info
-  gauss_init<T>();
-  const int64_t gid = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (gid >= a.paths) return;
+  constexpr int N = R * W;
+  using Sq = WideSquare<T, N>;
+  constexpr int CK = Sq::CK, COLS = Sq::COLS;
+  constexpr int NS = kHeston ? 3 : 1;  // squares: of log x (or all); y by x, y by y
+  constexpr int NB = kHeston ? 2 : 1;  // normals' buffers: of log x (or all), of y
+  constexpr int NPAR = 5 * N;
+  __shared__ __align__(16) T chol[NS * Sq::SIZE];
+  __shared__ __align__(16) T par_lds[2 + NPAR];  // ds, sqrt|ds|, the parameter blocks
+  __shared__ T z[NB][COLS][64];
+  __shared__ uint32_t words[kJump ? N : 1][kJump ? 64 : 1];
+
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int m = a.nvars;
+  const int n = kHeston ? m / 2 : m;  // width of a parameter block
+  gauss_init<T>(64 * W);
+  const bool replay = GEN && a.replay_dw != nullptr;
+  const bool replay_j = GEN && a.replay_dj != nullptr;
+  const bool pp = GEN && a.ppar != nullptr;
+  const uint32_t zero_below = kJump && !(GEN && (a.replay_dj || a.lamp))
+                                  ? zero_count_bound(pois, (int64_t)a.nsteps * m, 64 * W)
+                                  : 0u;
+  for (int i = threadIdx.x; i < NS * Sq::SIZE; i += 64 * W) chol[i] = (T)0;
+  for (int i = threadIdx.x; i < NB * COLS * 64; i += 64 * W) (&z[0][0][0])[i] = (T)0;
+
+  // Table element e of a step: the header and the parameters go to par_lds, the
+  // triangle's (i, j) to its square.  Thread t moves elements t, t + 64 W, ...
+  constexpr int MAXC = 2 + (kHeston ? 2 * N * (2 * N + 1) / 2 : N * (N + 1) / 2) + NPAR;
+  constexpr int NE = (MAXC + 64 * W - 1) / (64 * W);
+  const int ncoef = a.ncoef < 2 + NPAR + (a.poff - 2) ? a.ncoef : 2 + NPAR + (a.poff - 2);
+  T* dst[NE];
+#pragma unroll
+  for (int k = 0; k < NE; ++k) {
+    const int e = k * 64 * W + (int)threadIdx.x;
+    dst[k] = nullptr;
+    if (e >= ncoef) continue;
+    if (e < 2 || e >= a.poff) {
+      dst[k] = par_lds + (e < 2 ? e : e - (a.poff - 2));
+    } else {
+      // row i holds elements i (i + 1) / 2 .. of the packed triangle
+      const int q = e - 2;
+      int i = (int)((sqrtf(8.f * (float)q + 1.f) - 1.f) * .5f);
+      while ((i + 1) * (i + 2) / 2 <= q) ++i;
+      while (i * (i + 1) / 2 > q) --i;
+      const int j = q - i * (i + 1) / 2;
+      if (!kHeston || i < n)
+        dst[k] = chol + i * COLS + j;
+      else if (j < n)
+        dst[k] = chol + Sq::SIZE + (i - n) * COLS + j;
+      else
+        dst[k] = chol + 2 * Sq::SIZE + (i - n) * COLS + (j - n);
+    }
+  }
+  T ahead[NE];
+  auto fetch = [&](int s) {
+#pragma unroll
+    for (int k = 0; k < NE; ++k)
+      if (dst[k]) ahead[k] = coef[(int64_t)s * a.ncoef + k * 64 * W + (int)threadIdx.x];
+  };
+
   const int64_t P = a.paths;
+  const int64_t tid = (int64_t)blockIdx.x * 64 + lane;
+  // lanes beyond the last path step a copy of it and store nothing
+  const bool live = tid < P;
+  const int64_t gid = live ? tid : P - 1;
   const uint32_t path = (uint32_t)gid;
   const bool flip_w = a.anti_w > 0 && gid >= a.anti_w;
   const uint32_t path_w = flip_w ? (uint32_t)(gid - a.anti_w) : path;
   const uint32_t path_j = (a.anti_j > 0 && gid >= a.anti_j) ? (uint32_t)(gid - a.anti_j) : path;
-  const int m = a.nvars;
-  const int n = kHeston ? m / 2 : m;  // width of a parameter block
   const int64_t mt = a.m_total, c0 = a.comp0;
-  const bool replay = a.replay_dw != nullptr;
-  const bool replay_j = a.replay_dj != nullptr;
-  const bool pp = a.ppar != nullptr;
   const int64_t mtb = kHeston ? mt / 2 : mt, c0b = kHeston ? c0 / 2 : c0;
   const T* __restrict__ ppar = (const T*)a.ppar;
   const T* __restrict__ x0p = (const T*)a.x0_paths;
   auto x0_of = [&](int v) -> T {
     return x0p ? x0p[(c0 + v) * P + gid] : (T)a.x0[v];
   };
-  // parameter b of component (Heston: pair) v at a step whose block starts at
-  // p (per path: at the step's offset pbase into ppar)
+  // the wave's r-th component, and whether it has one (uniform over the wave);
+  // rows without one step zeros
+  auto comp = [&](int r) { return r * W + w; };
+  auto has = [&](int r) { return r * W + w < n; };
+  // parameter block b of component (Heston: pair) v at a step (per path: at the
+  // step's offset pbase into ppar)
   int64_t pbase = 0;
-  auto par = [&](const T* p, int b, int v) -> T {
-    return pp ? ppar[pbase + ((int64_t)b * mtb + c0b + v) * P + gid] : p[b * n + v];
+  auto par = [&](int b, int v) -> T {
+    if (pp) return v < n ? ppar[pbase + ((int64_t)b * mtb + c0b + v) * P + gid] : (T)0;
+    return par_lds[2 + (v < n ? b * n + v : 0)];
   };
 
-  T x[NS];   // log x for Heston
-  T vy[kHeston ? H : 1];
+  T x[R];  // log x for Heston
+  T vy[kHeston ? R : 1];
 #pragma unroll
-  for (int v = 0; v < NS; ++v) x[v] = v < n ? x0_of(v) : (T)0;
-  if constexpr (kHeston) {
-#pragma unroll
-    for (int i = 0; i < H; ++i) vy[i] = i < n ? x0_of(n + i) : (T)0;
+  for (int r = 0; r < R; ++r) {
+    x[r] = has(r) ? x0_of(comp(r)) : (T)0;
+    if constexpr (kHeston) vy[r] = has(r) ? x0_of(n + comp(r)) : (T)0;
   }
+  int cnt[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) cnt[r] = 0;
+  int interval_jumps = 0;
 
+  // Every thread of the block must call it.
   auto store = [&](int row) {
     T* o_row = out + ((int64_t)row * a.out_stride + a.out0) * P + gid;
-    if constexpr (kHeston) {
-      const bool whole = a.nout == m;
+    if (kOU && a.out_group != 1) {
+      // hull_white_SDE.let: the sum over the block's factors (out_group = m),
+      // in order, from the waves' values in the normals' buffer
+      __syncthreads();
 #pragma unroll
-      for (int i = 0; i < H; ++i) {
-        if (i < n) {
-          __builtin_nontemporal_store((T)exp(x[i]), o_row + i * P);
-          if (whole) __builtin_nontemporal_store(vy[i], o_row + (n + i) * P);
-        }
+      for (int r = 0; r < R; ++r)
+        if (has(r)) z[0][comp(r)][lane] = x[r];
+      __syncthreads();
+      if (w == 0 && live) {
+        T val = (T)0;
+        for (int v = 0; v < m; ++v) val = val + z[0][v][lane];
+        __builtin_nontemporal_store(val, o_row);
       }
-    } else if (kOU && a.out_group != 1) {
-      // hull_white_SDE.let: the sum over the block's factors (out_group = m)
-      T val = (T)0;
+      return;
+    }
+    if (!live) return;
 #pragma unroll
-      for (int v = 0; v < W; ++v)
-        if (v < m) val = val + x[v];
-      __builtin_nontemporal_store(val, o_row);
-    } else {
-#pragma unroll
-      for (int o = 0; o < W; ++o) {
-        if (o < a.nout) {
-          T val = x[o];
-          if constexpr (OutRule<MODEL>::exp_all) val = exp(val);
-          __builtin_nontemporal_store(val, o_row + o * P);
-        }
+    for (int r = 0; r < R; ++r) {
+      if (!has(r)) break;
+      const int v = comp(r);
+      if constexpr (kHeston) {
+        __builtin_nontemporal_store((T)exp(x[r]), o_row + v * P);
+        if (a.nout == m) __builtin_nontemporal_store(vy[r], o_row + (n + v) * P);
+      } else if (v < a.nout) {
+        T val = x[r];
+        if constexpr (OutRule<MODEL>::exp_all) val = exp(val);
+        __builtin_nontemporal_store(val, o_row + v * P);
       }
     }
   };
-  if (a.row0 >= 0) store(a.row0);
 
-  int cnt[NS];
+  // The flat indices g .. g+m-1 of a stream lie in Philox blocks g/4 ...; f
+  // gets a block and the component of its first value, wave w every W-th one.
+  auto each_block = [&](uint64_t g, auto f) {
+    const uint32_t b0 = (uint32_t)(g >> 2);
+    const int off = (int)(g & 3u);
+    const int nb = (off + m + 3) >> 2;
+    for (int i = 0; i * W < nb; ++i) {
+      const int q = i * W + w;
+      if (q >= nb) break;
+      f(b0 + q, 4 * q - off);
+    }
+  };
+
+  // acc[r] += sum over columns of square[row of r][column] zz[column]; of a
+  // triangle only the columns up to the rows r of any wave.
+  auto apply = [&](T(&acc)[R], const T* square, const T(*zz)[64], auto triangle) {
+    const T* mine = square + w * COLS;
 #pragma unroll
-  for (int v = 0; v < NS; ++v) cnt[v] = 0;
-  int interval_jumps = 0;
+    for (int q = 0; q < COLS / CK; ++q) {
+      T zc[CK];
+#pragma unroll
+      for (int l = 0; l < CK; ++l) zc[l] = zz[q * CK + l][lane];
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        if (decltype(triangle)::value && (r + 1) * W <= q * CK) continue;
+        T cf[CK];
+        __builtin_memcpy(cf, __builtin_assume_aligned(mine + r * W * COLS + q * CK, 16), 16);
+#pragma unroll
+        for (int l = 0; l < CK; ++l) acc[r] = acc[r] + cf[l] * zc[l];
+      }
+    }
+  };
+
+  if (a.nsteps > 0) fetch(0);
+  __syncthreads();
+  if (a.row0 >= 0) store(a.row0);
+  __syncthreads();
 
   for (int s = 0; s < a.nsteps; ++s) {
-    const T* c = coef + (int64_t)s * a.ncoef;
-    const T ds = c[0];
-    const T sq = c[1];
-    const T* L = c + 2;
-    const T* p = c + a.poff;
     const uint64_t g = (uint64_t)s * mt + c0;  // flat index of the block's first normal
     pbase = (int64_t)s * a.ppar_step;
     const T* rp = replay ? (const T*)a.replay_dw + (int64_t)g * P + gid : nullptr;
 
+    // the step's table row, normals and Poisson words into LDS
+#pragma unroll
+    for (int k = 0; k < NE; ++k)
+      if (dst[k]) *dst[k] = ahead[k];
+    if (!replay) {
+      each_block(g, [&](uint32_t blk, int v0) {
+        T zz[4];
+        normals4<T>(blk, path_w, a.c2w, a.ew, a.kw0, a.kw1, zz);
+#pragma unroll
+        for (int l = 0; l < 4; ++l) {
+          const int v = v0 + l;
+          const T val = flip_w ? -zz[l] : zz[l];
+          if (v >= 0 && v < m) {
+            if (!kHeston || v < n)
+              z[0][v][lane] = val;
+            else
+              z[NB - 1][v - n][lane] = val;
+          }
+        }
+      });
+    }
+    if constexpr (kJump) {
+      if (!replay_j) {
+        each_block(g, [&](uint32_t blk, int v0) {
+          const ctr4 u = philox4x32_10(ctr4{blk, path_j, a.c2p, a.ej}, a.kj0, a.kj1);
+          const uint32_t uu[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+          for (int l = 0; l < 4; ++l)
+            if (v0 + l >= 0 && v0 + l < m) words[v0 + l][lane] = uu[l];
+        });
+      }
+    }
+    __syncthreads();
+    if (s + 1 < a.nsteps) fetch(s + 1);
+    const int row = store_row[s];
+    const T ds = par_lds[0], sq = par_lds[1];
+
     if constexpr (kHeston) {
       // dw of the log-x values (zx) and of the variances (zy)
-      T zx[H], zy[H];
+      T zx[R], zy[R];
+#pragma unroll
+      for (int r = 0; r < R; ++r) zx[r] = zy[r] = (T)0;
       if (replay) {
 #pragma unroll
-        for (int i = 0; i < H; ++i) {
-          zx[i] = i < n ? rp[(int64_t)i * P] : (T)0;
-          zy[i] = i < n ? rp[(int64_t)(n + i) * P] : (T)0;
+        for (int r = 0; r < R; ++r) {
+          if (has(r)) {
+            zx[r] = rp[(int64_t)comp(r) * P];
+            zy[r] = rp[(int64_t)(n + comp(r)) * P];
+          }
         }
       } else {
-        normals_span<T, H>(g, n, path_w, a.c2w, a.ew, a.kw0, a.kw1, zx);
-        normals_span<T, H>(g + n, n, path_w, a.c2w, a.ew, a.kw0, a.kw1, zy);
-        if (flip_w) {
-#pragma unroll
-          for (int i = 0; i < H; ++i) {
-            zx[i] = -zx[i];
-            zy[i] = -zy[i];
-          }
-        }
         if (a.has_corr) {
-#pragma unroll
-          for (int i = H - 1; i >= 0; --i) {
-            if (i < n) {
-              const int r = n + i;
-              const T* Lr = L + r * (r + 1) / 2;
-              T acc = (T)0;
-#pragma unroll
-              for (int j = 0; j < H; ++j)
-                if (j < n) acc = acc + Lr[j] * zx[j];
-#pragma unroll
-              for (int j = 0; j <= i; ++j) acc = acc + Lr[n + j] * zy[j];
-              zy[i] = acc * sq;
-            }
-          }
-#pragma unroll
-          for (int i = H - 1; i >= 0; --i) {
-            if (i < n) {
-              const T* Lr = L + i * (i + 1) / 2;
-              T acc = (T)0;
-#pragma unroll
-              for (int j = 0; j <= i; ++j) acc = acc + Lr[j] * zx[j];
-              zx[i] = acc * sq;
-            }
-          }
+          // the y rows: every column of log x, then the triangle of y
+          apply(zx, chol, z[0], Flag<true>{});
+          apply(zy, chol + Sq::SIZE, z[0], Flag<false>{});
+          apply(zy, chol + 2 * Sq::SIZE, z[NB - 1], Flag<true>{});
         } else {
 #pragma unroll
-          for (int i = 0; i < H; ++i) {
-            zx[i] = zx[i] * sq;
-            zy[i] = zy[i] * sq;
+          for (int r = 0; r < R; ++r) {
+            zx[r] = z[0][comp(r)][lane];
+            zy[r] = z[NB - 1][comp(r)][lane];
           }
         }
-      }
-      // full_heston_SDE (full truncation), as in k_euler
 #pragma unroll
-      for (int i = 0; i < H; ++i) {
-        if (i < n) {
-          heston_next<T>(x[i], vy[i], cnt[i], par(p, 0, i), par(p, 1, i), par(p, 2, i),
-                         par(p, 3, i), par(p, 4, i), ds, zx[i], zy[i]);
+        for (int r = 0; r < R; ++r) {
+          zx[r] = zx[r] * sq;
+          zy[r] = zy[r] * sq;
         }
+      }
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const int v = comp(r);
+        heston_next<T>(x[r], vy[r], cnt[r], par(0, v), par(1, v), par(2, v), par(3, v),
+                       par(4, v), ds, zx[r], zy[r]);
       }
     } else {
-      T z[W];
-      if (replay) {
-#pragma unroll
-        for (int v = 0; v < W; ++v) z[v] = v < m ? rp[(int64_t)v * P] : (T)0;
-      } else {
-        normals_span<T, W>(g, m, path_w, a.c2w, a.ew, a.kw0, a.kw1, z);
-        if (flip_w) {
-#pragma unroll
-          for (int v = 0; v < W; ++v) z[v] = -z[v];
-        }
-      }
       // OU with correlations and table parameters: sigma_i sqrt|ds| is folded
       // into the Cholesky rows by the host, as for k_euler
       const bool ou_folded = kOU && a.has_corr && !replay && !pp;
-      if (!replay && !ou_folded) {
-        if (a.has_corr) {
+      T dw[R];
 #pragma unroll
-          for (int i = W - 1; i >= 0; --i) {
-            if (i < m) {
-              const T* Li = L + i * (i + 1) / 2;
-              T acc = (T)0;
+      for (int r = 0; r < R; ++r)
+        dw[r] = ou_folded ? fma(par(0, comp(r)), x[r], par(1, comp(r))) : (T)0;
+      if (replay) {
 #pragma unroll
-              for (int j = 0; j <= i; ++j) acc = acc + Li[j] * z[j];
-              z[i] = acc * sq;
-            }
-          }
-        } else {
+        for (int r = 0; r < R; ++r)
+          if (has(r)) dw[r] = rp[(int64_t)comp(r) * P];
+      } else if (a.has_corr) {
+        apply(dw, chol, z[0], Flag<true>{});
+        if (!ou_folded) {
 #pragma unroll
-          for (int v = 0; v < W; ++v) z[v] = z[v] * sq;
+          for (int r = 0; r < R; ++r) dw[r] = dw[r] * sq;
         }
+      } else {
+#pragma unroll
+        for (int r = 0; r < R; ++r) dw[r] = z[0][comp(r)][lane] * sq;
       }
-
-      if constexpr (MODEL == SDEGPU_MODEL_WIENER || MODEL == SDEGPU_MODEL_LOGNORM) {
 #pragma unroll
-        for (int v = 0; v < W; ++v)
-          if (v < m) x[v] = x[v] + (par(p, 0, v) * ds + par(p, 1, v) * z[v]);
-      } else if constexpr (kOU) {
-        if (ou_folded) {
-#pragma unroll
-          for (int i = 0; i < W; ++i) {
-            if (i < m) {
-              const T* Li = L + i * (i + 1) / 2;
-              T acc = fma(p[i], x[i], p[m + i]);
-#pragma unroll
-              for (int j = 0; j <= i; ++j) acc = fma(Li[j], z[j], acc);
-              x[i] = acc;
-            }
+      for (int r = 0; r < R; ++r) {
+        const int v = comp(r);
+        if constexpr (MODEL == SDEGPU_MODEL_WIENER || MODEL == SDEGPU_MODEL_LOGNORM) {
+          x[r] = x[r] + (par(0, v) * ds + par(1, v) * dw[r]);
+        } else if constexpr (kOU) {
+          if (ou_folded) {
+            x[r] = dw[r];
+          } else {
+            const T av = pp ? fma(-par(0, v), ds, (T)1) : par(0, v);
+            const T bv = pp ? par(1, v) * ds : par(1, v);
+            x[r] = av * x[r] + (bv + par(2, v) * dw[r]);
           }
-        } else {
-#pragma unroll
-          for (int v = 0; v < W; ++v) {
-            if (v < m) {
-              T av, bv;
-              if (pp) {
-                av = fma(-par(p, 0, v), ds, (T)1);
-                bv = par(p, 1, v) * ds;
-              } else {
-                av = p[v];
-                bv = p[m + v];
-              }
-              x[v] = av * x[v] + (bv + par(p, 2, v) * z[v]);
-            }
-          }
-        }
-      } else if constexpr (MODEL == SDEGPU_MODEL_CIR) {
-#pragma unroll
-        for (int v = 0; v < W; ++v) {
-          if (v < m)
-            x[v] = cir_next<T>(x[v], par(p, 0, v), par(p, 1, v), par(p, 2, v), ds, z[v]);
-        }
-      } else if constexpr (kJump) {
-        // each component's jump total is added as it is drawn (no dj array:
-        // the FP64 W = 32 instance would not fit its registers otherwise)
-        if (replay_j) {
-          const T* rj = (const T*)a.replay_dj + (int64_t)g * P + gid;
-#pragma unroll
-          for (int v = 0; v < W; ++v)
-            if (v < m)
-              x[v] = x[v] + ((par(p, 0, v) * ds + par(p, 1, v) * z[v]) + rj[(int64_t)v * P]);
-        } else {
-          uint32_t u[W];
-          words_span<W>(g, m, path_j, a.c2p, a.ej, a.kj0, a.kj1, u);
-          const double* pq = pois + (int64_t)s * m * 2;
-          const bool neg = ds < (T)0;
-#pragma unroll
-          for (int v = 0; v < W; ++v) {
-            if (v < m) {
-              double lamds = pq[2 * v], p0 = pq[2 * v + 1];
-              if (a.lamp) {
+        } else if constexpr (MODEL == SDEGPU_MODEL_CIR) {
+          x[r] = cir_next<T>(x[r], par(0, v), par(1, v), par(2, v), ds, dw[r]);
+        } else if constexpr (kJump) {
+          T inc = par(0, v) * ds + par(1, v) * dw[r];
+          if (replay_j) {
+            if (has(r)) inc = inc + ((const T*)a.replay_dj)[((int64_t)g + v) * P + gid];
+          } else if (has(r)) {
+            const uint32_t word = words[v][lane];
+            if (word >= zero_below) {
+              const double* pq = pois + ((int64_t)s * m + v) * 2;
+              double lamds = pq[0], p0 = pq[1];
+              if (GEN && a.lamp) {
                 // per-path intensity: pois holds |ds|
                 lamds = a.lamp[(int64_t)s * a.lamp_step + (c0 + v) * P + gid] * lamds;
                 p0 = exp(-lamds);
               }
-              const int nj = poisson_inv(u01_f64(u[v]), lamds, p0, kPoissonCap);
-              T acc = (T)0;
+              const int nj = poisson_inv(u01_f64(word), lamds, p0, kPoissonCap);
               if (nj > 0) {
-                const T p2 = a.jump_law == SDEGPU_JUMP_NORMAL ? (T)0 : p[4 * m + v];
-                acc = jump_total<T>(a.jump_law, nj, (uint32_t)(g + v), path_j, a.c2j, a.ej,
-                                    a.kj0, a.kj1, p[2 * m + v], p[3 * m + v], p2);
+                const bool neg = ds < (T)0;
+                const T* pj = par_lds + 2;
+                const T p2 = a.jump_law == SDEGPU_JUMP_NORMAL ? (T)0 : pj[4 * m + v];
+                const T acc = jump_total<T>(a.jump_law, nj, (uint32_t)(g + v), path_j, a.c2j,
+                                            a.ej, a.kj0, a.kj1, pj[2 * m + v], pj[3 * m + v],
+                                            p2);
+                inc = inc + (neg ? -acc : acc);
+                cnt[r] += neg ? -nj : nj;
+                interval_jumps += neg ? -nj : nj;
               }
-              cnt[v] += neg ? -nj : nj;
-              interval_jumps += neg ? -nj : nj;
-              x[v] = x[v] + ((par(p, 0, v) * ds + par(p, 1, v) * z[v]) + (neg ? -acc : acc));
             }
           }
+          x[r] = x[r] + inc;
         }
       }
     }
 
-    const int row = store_row[s];
     if (row >= 0) {
       store(row);
       if constexpr (kJump) {
-        if (a.info_rows) add_interval_jumps(a, row, true, interval_jumps);
+        if (a.info_rows) add_interval_jumps(a, row, live, interval_jumps);
         interval_jumps = 0;
       }
     }
+    __syncthreads();
   }
 
-  if (a.info_paths && (kHeston || kJump)) {
+  if (a.info_paths && (kHeston || kJump) && live) {
 #pragma unroll
-    for (int v = 0; v < NS; ++v)
-      if (v < n) a.info_paths[(c0b + v) * P + gid] = cnt[v];
+    for (int r = 0; r < R; ++r)
+      if (has(r)) a.info_paths[(c0b + comp(r)) * P + gid] = cnt[r];
   }
 }
 
@@ -343,10 +435,27 @@ __global__ __launch_bounds__(kBlock) void k_wiener_fill_wide(
   }
 }
 
+// Waves that share 64 paths and components (Heston: pairs) per wave for a width:
+// the smallest of the instantiated shapes that holds it.
+struct WideShape {
+  int waves, rows;
+};
+inline WideShape wide_shape(int model, int m) {
+  const bool h = model == SDEGPU_MODEL_HESTON;
+  const int n = h ? m / 2 : m;
+  const WideShape all[2][7] = {{{2, 6}, {2, 8}, {3, 7}, {3, 8}, {4, 8}, {6, 8}, {8, 8}},
+                               {{2, 3}, {2, 4}, {3, 4}, {4, 4}, {6, 4}, {8, 4}, {8, 4}}};
+  for (const WideShape& s : all[h ? 1 : 0])
+    if (s.waves * s.rows >= n) return s;
+  return WideShape{0, 0};
+}
+
 // k_euler_wide and k_wiener_fill_wide instances (euler_wide_f32.hip,
-// euler_wide_f64.hip): the kernel for a model and a width of 9..32, or null.
+// euler_wide_f64.hip): the kernel for a model and a width of 9..64, or null.
+// Blocks of 64 * wide_shape(model, m).waves threads, one per 64 paths; gen: recorded
+// increments, per-path parameters or intensities.
 template <typename T>
-EulerKernel<T> euler_wide_kernel(int model, int m);
+EulerKernel<T> euler_wide_kernel(int model, int m, bool gen);
 
 template <typename T>
 using WienerFillWide = void (*)(uint32_t, uint32_t, uint32_t, uint32_t, int64_t, int64_t,
@@ -354,37 +463,65 @@ using WienerFillWide = void (*)(uint32_t, uint32_t, uint32_t, uint32_t, int64_t,
 template <typename T>
 WienerFillWide<T> wiener_fill_wide_kernel(int m);
 template <>
-EulerKernel<float> euler_wide_kernel<float>(int model, int m);
+EulerKernel<float> euler_wide_kernel<float>(int model, int m, bool gen);
 template <>
-EulerKernel<double> euler_wide_kernel<double>(int model, int m);
+EulerKernel<double> euler_wide_kernel<double>(int model, int m, bool gen);
 template <>
 WienerFillWide<float> wiener_fill_wide_kernel<float>(int m);
 template <>
 WienerFillWide<double> wiener_fill_wide_kernel<double>(int m);
 
-#define SDEGPU_WIDE_PICK(MODEL, T)                                                        \
-  (m <= 16 ? k_euler_wide<MODEL, T, 16>                                                   \
-           : m <= 32 ? k_euler_wide<MODEL, T, 32> : k_euler_wide<MODEL, T, 64>)
+template <int MODEL, typename T, bool GEN>
+EulerKernel<T> pick_wide(int m) {
+  const WideShape s = wide_shape(MODEL, m);
+  if constexpr (MODEL == SDEGPU_MODEL_HESTON) {
+    switch (s.waves * 16 + s.rows) {
+      case 2 * 16 + 3: return k_euler_wide<MODEL, T, 2, 3, GEN>;
+      case 2 * 16 + 4: return k_euler_wide<MODEL, T, 2, 4, GEN>;
+      case 3 * 16 + 4: return k_euler_wide<MODEL, T, 3, 4, GEN>;
+      case 4 * 16 + 4: return k_euler_wide<MODEL, T, 4, 4, GEN>;
+      case 6 * 16 + 4: return k_euler_wide<MODEL, T, 6, 4, GEN>;
+      case 8 * 16 + 4: return k_euler_wide<MODEL, T, 8, 4, GEN>;
+      default: return nullptr;
+    }
+  } else {
+    switch (s.waves * 16 + s.rows) {
+      case 2 * 16 + 6: return k_euler_wide<MODEL, T, 2, 6, GEN>;
+      case 2 * 16 + 8: return k_euler_wide<MODEL, T, 2, 8, GEN>;
+      case 3 * 16 + 7: return k_euler_wide<MODEL, T, 3, 7, GEN>;
+      case 3 * 16 + 8: return k_euler_wide<MODEL, T, 3, 8, GEN>;
+      case 4 * 16 + 8: return k_euler_wide<MODEL, T, 4, 8, GEN>;
+      case 6 * 16 + 8: return k_euler_wide<MODEL, T, 6, 8, GEN>;
+      case 8 * 16 + 8: return k_euler_wide<MODEL, T, 8, 8, GEN>;
+      default: return nullptr;
+    }
+  }
+}
 
-#define SDEGPU_EULER_WIDE_SET(T)                                                          \
-  template <>                                                                             \
-  EulerKernel<T> euler_wide_kernel<T>(int model, int m) {                                 \
-    if (m <= SDEGPU_MAX_VARS || m > SDEGPU_MAX_COUPLED) return nullptr;                    \
-    switch (model) {                                                                      \
-      case SDEGPU_MODEL_WIENER: return SDEGPU_WIDE_PICK(SDEGPU_MODEL_WIENER, T);           \
-      case SDEGPU_MODEL_LOGNORM: return SDEGPU_WIDE_PICK(SDEGPU_MODEL_LOGNORM, T);         \
-      case SDEGPU_MODEL_OU: return SDEGPU_WIDE_PICK(SDEGPU_MODEL_OU, T);                   \
-      case SDEGPU_MODEL_CIR: return SDEGPU_WIDE_PICK(SDEGPU_MODEL_CIR, T);                 \
-      case SDEGPU_MODEL_HESTON: return SDEGPU_WIDE_PICK(SDEGPU_MODEL_HESTON, T);           \
-      case SDEGPU_MODEL_JUMPDIFF: return SDEGPU_WIDE_PICK(SDEGPU_MODEL_JUMPDIFF, T);       \
-      default: return nullptr;                                                            \
-    }                                                                                     \
-  }                                                                                       \
-  template <>                                                                             \
-  WienerFillWide<T> wiener_fill_wide_kernel<T>(int m) {                                   \
-    if (m <= SDEGPU_MAX_VARS || m > SDEGPU_MAX_COUPLED) return nullptr;                    \
-    return m <= 16 ? k_wiener_fill_wide<T, 16>                                            \
-                   : m <= 32 ? k_wiener_fill_wide<T, 32> : k_wiener_fill_wide<T, 64>;     \
+template <int MODEL, typename T>
+EulerKernel<T> pick_wide(int m, bool gen) {
+  return gen ? pick_wide<MODEL, T, true>(m) : pick_wide<MODEL, T, false>(m);
+}
+
+#define SDEGPU_EULER_WIDE_SET(T)                                                         \
+  template <>                                                                            \
+  EulerKernel<T> euler_wide_kernel<T>(int model, int m, bool gen) {                      \
+    if (m <= SDEGPU_MAX_VARS || m > SDEGPU_MAX_COUPLED) return nullptr;                  \
+    switch (model) {                                                                     \
+      case SDEGPU_MODEL_WIENER: return pick_wide<SDEGPU_MODEL_WIENER, T>(m, gen);        \
+      case SDEGPU_MODEL_LOGNORM: return pick_wide<SDEGPU_MODEL_LOGNORM, T>(m, gen);      \
+      case SDEGPU_MODEL_OU: return pick_wide<SDEGPU_MODEL_OU, T>(m, gen);                \
+      case SDEGPU_MODEL_CIR: return pick_wide<SDEGPU_MODEL_CIR, T>(m, gen);              \
+      case SDEGPU_MODEL_HESTON: return pick_wide<SDEGPU_MODEL_HESTON, T>(m, gen);        \
+      case SDEGPU_MODEL_JUMPDIFF: return pick_wide<SDEGPU_MODEL_JUMPDIFF, T>(m, gen);    \
+      default: return nullptr;                                                           \
+    }                                                                                    \
+  }                                                                                      \
+  template <>                                                                            \
+  WienerFillWide<T> wiener_fill_wide_kernel<T>(int m) {                                  \
+    if (m <= SDEGPU_MAX_VARS || m > SDEGPU_MAX_COUPLED) return nullptr;                  \
+    return m <= 16 ? k_wiener_fill_wide<T, 16>                                           \
+                   : m <= 32 ? k_wiener_fill_wide<T, 32> : k_wiener_fill_wide<T, 64>;    \
   }
 
 }  // namespace sdegpu
