@@ -1399,6 +1399,20 @@ def piecewise(t=0., *, x=None, v=None, dtype=None, mode='mid'):
     return out
 
 
+def device_moments(dx):
+    """FP64 device tensors (mean, m2) of the rows of a device tensor
+    [rows][paths] (``sdegpu_path_moments``)."""
+    rows, paths = int(dx.shape[0]), int(dx.shape[1])
+    code = _lib.F32 if dx.dtype == _lib.torch_mod().float32 else _lib.F64
+    mean, m2 = _lib.empty((2, rows), np.float64)
+    nbytes = _lib.lib().sdegpu_moments_workspace(rows, paths)
+    ws = _lib.workspace(nbytes)
+    _lib.check(_lib.lib().sdegpu_path_moments(
+        _lib.ptr(dx), code, rows, paths, _lib.ptr(mean), _lib.ptr(m2),
+        _lib.ptr(ws), nbytes, _lib.stream()))
+    return mean, m2
+
+
 def path_moments(x, device_tensor=None, paths=None):
     """FP64 (n, mean, m2) over the last axis of ``x``, reduced on the GPU
     (``sdegpu_path_moments``).  ``device_tensor``, when given, is a device
@@ -1411,16 +1425,10 @@ def path_moments(x, device_tensor=None, paths=None):
             .format(x.dtype))
     paths = x.shape[-1] if paths is None else int(paths)
     rows = int(np.prod(x.shape[:-1], dtype=int))
-    code, cdt, _ = _gpu_dtype(x.dtype)
+    cdt = _gpu_dtype(x.dtype)[1]
     _lib.require_gpu()
     dx = device_tensor if device_tensor is not None else \
         _lib.to_device(x.astype(cdt, copy=False).reshape(rows, paths))
-    mean = _lib.empty((rows,), np.float64)
-    m2 = _lib.empty((rows,), np.float64)
-    nbytes = _lib.lib().sdegpu_moments_workspace(rows, paths)
-    ws = _lib.workspace(nbytes)
-    _lib.check(_lib.lib().sdegpu_path_moments(
-        _lib.ptr(dx), code, rows, paths, _lib.ptr(mean), _lib.ptr(m2),
-        _lib.ptr(ws), nbytes, _lib.stream()))
+    mean, m2 = device_moments(dx)
     return (float(paths), _lib.to_host(mean).reshape(x.shape[:-1]),
             _lib.to_host(m2).reshape(x.shape[:-1]))

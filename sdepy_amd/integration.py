@@ -26,6 +26,7 @@ the recorded increments in the kernel.
 """
 import ctypes
 import inspect
+import math
 
 import numpy as np
 
@@ -68,7 +69,9 @@ def consolidate_timeline(timeline, steps, i0):
         raise ValueError(
             'the integration timeline should be a one-dimensional array, '
             'not an array of shape {}'.format(tt.shape))
-    if not np.array_equal(tt, np.unique(tt)):
+    # (the comparison settles the common case; np.unique sorts)
+    if not ((tt.size > 1 and tt.dtype.kind in 'iuf' and (tt[1:] > tt[:-1]).all())
+            or np.array_equal(tt, np.unique(tt))):
         raise ValueError(
             'the integration timeline sholud be an array of strictly '
             'increasing numbers, but {} was given'.format(tt))
@@ -216,7 +219,7 @@ class _gpu_sde:
         return self._rng
 
     def _nvars(self):
-        return int(np.prod(self.wshape, dtype=int))
+        return math.prod(self.wshape)
 
     def _init_state(self, P, cdt):
         """Working state after SDE.init (and the log of SDE.begin for log
@@ -296,6 +299,9 @@ class _gpu_sde:
         callable, [nsteps][NB][M][paths] (each step's values at its start,
         t0s) when one is.  A callable counts as per-path when its value at
         the first step varies across paths."""
+        if all(not callable(self._args[name]) and np.ndim(self._args[name]) == 0
+               for name in self.sde_defaults):
+            return None
         shape, P = self._param_shape(), self.paths
 
         def to_paths(name, z):
@@ -346,7 +352,9 @@ class _gpu_sde:
     def _eval(self, name, t0s, shape):
         """Values of parameter `name` at each step start: (nsteps, prod(shape))."""
         z = self._args[name]
-        n = int(np.prod(shape, dtype=int))
+        n = math.prod(shape)
+        if not callable(z) and np.ndim(z) == 0:
+            return np.full((len(t0s), n), float(z))
         if callable(z):
             return np.stack([per_component(z(t), shape, name) for t in t0s]) \
                 if len(t0s) else np.zeros((0, n))
@@ -356,7 +364,8 @@ class _gpu_sde:
     # integration ----------------------------------------------------------
 
     def __call__(self, timeline):
-        return self.prepare(timeline).run()
+        # (launched right away on the current stream, behind the uploads)
+        return self._prepare(timeline, wait=False).run()
 
     def prepare(self, timeline, moments=False):
         """Validate the timeline, build the step tables, upload them and
@@ -367,6 +376,14 @@ class _gpu_sde:
         its FP64 moments as they store it, so that the run's ``pmean``,
         ``pvar``, ``psum`` and ``pstd`` need no further pass over the
         output."""
+        run = self._prepare(timeline)
+        if moments:
+            run._fuse_moments()
+        return run
+
+    def _prepare(self, timeline, wait=True):
+        """prepare() without moments; the tables' uploads are waited for, or
+        only ordered on the current stream."""
         tt, tt_asis, steps_tt = consolidate_timeline(timeline, self.steps,
                                                      self.i0)
         i0 = self.i0
@@ -388,15 +405,12 @@ class _gpu_sde:
         x0 = self._x0_state(cdt)
         prepared = [self._prepare_pass(sp, tp, row_of, reverse, k == 0, x0,
                                        code, cdt, xx_dev,
-                                       (nout, out_mode, out_group, exp_mask))
+                                       (nout, out_mode, out_group, exp_mask), wait)
                     for k, (sp, tp, row_of, reverse) in enumerate(passes)]
-        run = PreparedRun(self, prepared, xx_dev, tt, tt_asis, odt)
-        if moments:
-            run._fuse_moments()
-        return run
+        return PreparedRun(self, prepared, xx_dev, tt, tt_asis, odt)
 
     def _prepare_pass(self, steps_pass, tt_pass, row_of, reverse, first, x0,
-                      code, cdt, xx_dev, outmap):
+                      code, cdt, xx_dev, outmap, wait):
         nout, out_mode, out_group, exp_mask = outmap
         M = self._nvars()
         P = self.paths
@@ -415,6 +429,7 @@ class _gpu_sde:
         prob.row0 = int(row_of(0)) if first else -1
         prob.stream_tag = _lib.STREAM_BACKWARD if reverse else 0
         keep = []   # device buffers alive until the call is done
+        tables = []     # (array, setter of its device address), uploaded together
 
         # Wiener source: in-kernel Philox draws, or recorded increments
         dw = self.sources['dw']
@@ -509,10 +524,6 @@ class _gpu_sde:
                 host_sources['dj'] = dj
         self._host_dj = 'dj' in host_sources
         prob.has_corr = int(has_corr)
-        if nsteps:
-            d_rows = _lib.to_device(rows)
-            keep.append(d_rows)
-            prob.store_row = d_rows.data_ptr()
         if self.model == _lib.MODEL_JUMPDIFF:
             # jump sizes drawn at the next stored step: pays when at most one
             # step in 8 stores a row
@@ -521,7 +532,7 @@ class _gpu_sde:
         # host sources, drawn in sorted id order per step (SDE.dZ)
         recorded = {k: [] for k in host_sources}
         dn_host = [] if dn_big is None else list(dn_big)
-        for s, d in zip(t0s, ds):
+        for s, d in zip(t0s, ds) if host_sources else ():
             for sid in sorted(host_sources):
                 z = np.asarray(host_sources[sid](s, d), dtype=float)
                 recorded[sid].append(np.broadcast_to(
@@ -547,7 +558,9 @@ class _gpu_sde:
         info_paths = info_rows = None
         if self.getinfo and (self.model == _lib.MODEL_HESTON or (
                 self.model == _lib.MODEL_JUMPDIFF and not self._anti_dj)):
-            info_paths = _lib.zeros((M, P), np.int32)
+            # (every launch writes all of its paths' counts)
+            info_paths = _lib.empty(
+                (M // 2 if self.model == _lib.MODEL_HESTON else M, P), np.int32)
             prob.info_paths = info_paths.data_ptr()
             if self.model == _lib.MODEL_JUMPDIFF:
                 # jump totals per output row, spread over INFO_SLOTS counters
@@ -584,14 +597,9 @@ class _gpu_sde:
                 tab = np.concatenate((tab, extra), axis=1)
             gp.ncoef = tab.shape[1]
             if nsteps:
-                d_tab = _lib.to_device(tab.astype(cdt))
-                keep.append(d_tab)
-                gp.coef = d_tab.data_ptr()
+                tables.append((tab.astype(cdt), (gp, 'coef')))
                 if pois is not None:
-                    d_pois = _lib.to_device(
-                        np.ascontiguousarray(pois[:, g0:g0 + mg, :]))
-                    keep.append(d_pois)
-                    gp.pois = d_pois.data_ptr()
+                    tables.append((pois[:, g0:g0 + mg, :], (gp, 'pois')))
             if x0.shape == (M,):
                 for v in range(mg):
                     gp.x0[v] = float(x0[g0 + v])
@@ -601,6 +609,13 @@ class _gpu_sde:
                     g0, mg, nout, out_mode, out_group)
                 gp.out_stride = nout
             probs.append(gp)
+        if nsteps:
+            bufs, addr = _lib.upload([rows] + [t for t, _ in tables], wait)
+            keep += bufs
+            for gp in probs:
+                gp.store_row = addr[0]
+            for (_, (gp, field)), at in zip(tables, addr[1:]):
+                setattr(gp, field, at)
 
         def post():
             if self.getinfo:
@@ -729,8 +744,7 @@ class PreparedRun:
             return
         n_t, nout, P = self.xx_dev.shape
         rows = n_t * nout
-        self._mom_mean = _lib.empty((rows,), np.float64)
-        self._mom_m2 = _lib.empty((rows,), np.float64)
+        self._mom_mean, self._mom_m2 = _lib.empty((2, rows), np.float64)
         if P <= _SEPARATE_PATHS:
             self._mom_nbytes = _lib.lib().sdegpu_moments_workspace(rows, P)
             self._mom_ws = _lib.workspace(self._mom_nbytes)
@@ -793,19 +807,17 @@ class PreparedRun:
             self.tt.shape + sde.xshape + (1,))
         return sde._result(self.tt_asis, xx)
 
-    def _moments(self):
+    def _moments(self, which):
+        """(paths, FP64 moment of every row): the mean (0) or the sum of
+        squared deviations (1)."""
+        n_t, nout, P = self.xx_dev.shape
         if self._mom_mean is not None:
             # reduced within the launch
-            shape = self.xx_dev.shape[:2]
-            return (float(self.xx_dev.shape[2]),
-                    _lib.to_host(self._mom_mean).reshape(shape),
-                    _lib.to_host(self._mom_m2).reshape(shape))
-        from .infrastructure import path_moments
-        rows = self._rows()
-        f32 = rows.dtype == _lib.torch_mod().float32
-        return path_moments(np.empty((rows.shape[0], 0),
-                                     dtype=np.float32 if f32 else np.float64),
-                            device_tensor=rows, paths=rows.shape[1])
+            mom = self._mom_m2 if which else self._mom_mean
+        else:
+            from .infrastructure import device_moments
+            mom = device_moments(self._rows())[which]
+        return float(P), _lib.to_host(mom).reshape(n_t, nout)
 
     def _minmax(self):
         rows = self._rows()
@@ -834,22 +846,21 @@ class PreparedRun:
 
     def psum(self, dtype=None):
         """Sum across paths (FP64 accumulation on the device)."""
-        n, mean, _ = self._moments()
+        n, mean = self._moments(0)
         return self._summary(mean * n, dtype)
 
     def pmean(self, dtype=None):
         """Mean across paths (FP64 accumulation on the device)."""
-        _, mean, _ = self._moments()
-        return self._summary(mean, dtype)
+        return self._summary(self._moments(0)[1], dtype)
 
     def pvar(self, dtype=None, ddof=0):
         """Variance across paths (FP64 accumulation on the device)."""
-        n, _, m2 = self._moments()
+        n, m2 = self._moments(1)
         return self._summary(m2 / (n - ddof), dtype)
 
     def pstd(self, dtype=None, ddof=0):
         """Standard deviation across paths (FP64 on the device)."""
-        n, _, m2 = self._moments()
+        n, m2 = self._moments(1)
         return self._summary(np.sqrt(m2 / (n - ddof)), dtype)
 
     # process.tmin/tmax/tsum/tmean/tvar/tstd (infrastructure.py:963-1027)
@@ -1182,7 +1193,7 @@ class full_heston_process(_gpu_sde):
         if info_paths is None:
             return
         N = self._nvars() // 2
-        cnt = _lib.to_host(info_paths)[:N].astype(int)
+        cnt = _lib.to_host(info_paths).astype(int)
         self.info['negative_y_count'] = cnt.reshape(self.vshape + (self.paths,))
 
 
