@@ -91,6 +91,16 @@ __device__ __forceinline__ A sqrt_round(A a) {
   return (A)sqrt((double)a);
 }
 
+// f on the entries k .. k + N - 1, all loaded before the first is used
+template <typename T, int V, int N, typename At, typename F>
+__device__ __forceinline__ void axis_group(At& at, int64_t k, F& f) {
+  T v[N][V];
+#pragma unroll
+  for (int i = 0; i < N; ++i) VecLoad<T, V>::load(at(k + i), v[i]);
+#pragma unroll
+  for (int i = 0; i < N; ++i) f(v[i]);
+}
+
 template <typename T, typename A, int OP, int V>
 __global__ __launch_bounds__(kBlock) void k_axis_reduce(const T* __restrict__ x, const AxisArgs a,
                                                         void* __restrict__ out) {
@@ -103,11 +113,21 @@ __global__ __launch_bounds__(kBlock) void k_axis_reduce(const T* __restrict__ x,
   const T* __restrict__ base = x + o * a.so + c;
   const int64_t n = a.n;
   auto at = [&](int64_t k) -> const T* { return base + (a.nmap ? a.off[k] : k * a.sk); };
+  // f on the entries first, first + 1, ... n - 1, in order.  Below one block
+  // per CU the loads in flight bound the pass, and 8 of them per thread are
+  // better than 4 (500 rows of 100,000 FP32 values: maximum 71 -> 53 us,
+  // variance 122 -> 85); above, 4 read as fast (500,000 columns: 79 and 81).
+  const bool deep = gridDim.x < 256;
+  auto walk = [&](int64_t first, auto& f) {
+    int64_t k = first;
+    for (; deep && k + 7 < n; k += 8) axis_group<T, V, 8>(at, k, f);
+    for (; k + 3 < n; k += 4) axis_group<T, V, 4>(at, k, f);
+    for (; k < n; ++k) axis_group<T, V, 1>(at, k, f);
+  };
 
   if constexpr (OP == SDEGPU_REDUCE_MIN || OP == SDEGPU_REDUCE_MAX) {
     T m[V];
     VecLoad<T, V>::load(at(0), m);
-    int64_t k = 1;
     auto step = [&](const T (&v)[V]) {
 #pragma unroll
       for (int l = 0; l < V; ++l) {
@@ -116,22 +136,7 @@ __global__ __launch_bounds__(kBlock) void k_axis_reduce(const T* __restrict__ x,
         m[l] = keep ? m[l] : v[l];
       }
     };
-    for (; k + 3 < n; k += 4) {
-      T v0[V], v1[V], v2[V], v3[V];
-      VecLoad<T, V>::load(at(k), v0);
-      VecLoad<T, V>::load(at(k + 1), v1);
-      VecLoad<T, V>::load(at(k + 2), v2);
-      VecLoad<T, V>::load(at(k + 3), v3);
-      step(v0);
-      step(v1);
-      step(v2);
-      step(v3);
-    }
-    for (; k < n; ++k) {
-      T v[V];
-      VecLoad<T, V>::load(at(k), v);
-      step(v);
-    }
+    walk(1, step);
     VecLoad<T, V>::store((T*)out + o * a.inner + c, m);
   } else {
     // pass 1: sum in A, in index order from 0
@@ -142,23 +147,7 @@ __global__ __launch_bounds__(kBlock) void k_axis_reduce(const T* __restrict__ x,
 #pragma unroll
       for (int l = 0; l < V; ++l) s[l] = s[l] + (A)v[l];
     };
-    int64_t k = 0;
-    for (; k + 3 < n; k += 4) {
-      T v0[V], v1[V], v2[V], v3[V];
-      VecLoad<T, V>::load(at(k), v0);
-      VecLoad<T, V>::load(at(k + 1), v1);
-      VecLoad<T, V>::load(at(k + 2), v2);
-      VecLoad<T, V>::load(at(k + 3), v3);
-      add(v0);
-      add(v1);
-      add(v2);
-      add(v3);
-    }
-    for (; k < n; ++k) {
-      T v[V];
-      VecLoad<T, V>::load(at(k), v);
-      add(v);
-    }
+    walk(0, add);
     if constexpr (OP == SDEGPU_REDUCE_MEAN || OP == SDEGPU_REDUCE_VAR ||
                   OP == SDEGPU_REDUCE_STD) {
 #pragma unroll
@@ -177,23 +166,7 @@ __global__ __launch_bounds__(kBlock) void k_axis_reduce(const T* __restrict__ x,
           q[l] = q[l] + d2;
         }
       };
-      k = 0;
-      for (; k + 3 < n; k += 4) {
-        T v0[V], v1[V], v2[V], v3[V];
-        VecLoad<T, V>::load(at(k), v0);
-        VecLoad<T, V>::load(at(k + 1), v1);
-        VecLoad<T, V>::load(at(k + 2), v2);
-        VecLoad<T, V>::load(at(k + 3), v3);
-        dev(v0);
-        dev(v1);
-        dev(v2);
-        dev(v3);
-      }
-      for (; k < n; ++k) {
-        T v[V];
-        VecLoad<T, V>::load(at(k), v);
-        dev(v);
-      }
+      walk(0, dev);
       const int64_t dof = n - a.ddof > 0 ? n - a.ddof : 0;
 #pragma unroll
       for (int l = 0; l < V; ++l) {

@@ -26,9 +26,7 @@
 namespace sdegpu {
 
 constexpr int64_t kMcChunk = 16384;  // as kChunk of the path moments
-// values per histogram block: its counts flush to global memory once per
-// block, so it keeps larger chunks (16384 measured 5% slower)
-constexpr int64_t kMcHistChunk = 65536;
+constexpr int64_t kMcHistMin = 4096, kMcHistMax = 65536;  // values per histogram block
 constexpr int kMcMoments = 5;      // sum d, d^2, d^3, d^4, sum v
 constexpr int kMcLdsBins = 4096;   // histograms up to this size count in LDS
 constexpr int kMcLdsCounterWords = 8192;  // LDS words for the counter copies
@@ -117,17 +115,25 @@ __global__ __launch_bounds__(kBlock) void k_mc_minmax(const T* __restrict__ x, i
   }
 }
 
-__global__ void k_mc_minmax_final(int64_t rows, int64_t nchunks, const double* __restrict__ part,
-                                  double* __restrict__ out) {
-  const int64_t row = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+// One wave per row: lane l takes the chunks l, l + 64, ..., then a butterfly
+// merges the lanes.  A thread per row waited for its chunks one after the
+// other: 253 rows of 31 chunks take 3 us so, and took 11.
+__global__ __launch_bounds__(kBlock) void k_mc_minmax_final(int64_t rows, int64_t nchunks,
+                                                            const double* __restrict__ part,
+                                                            double* __restrict__ out) {
+  const int64_t row = (int64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
   if (row >= rows) return;
   double mn = __builtin_inf(), mx = -__builtin_inf(), nan = 0.0;
-  for (int64_t c = 0; c < nchunks; ++c) {
+  for (int64_t c = threadIdx.x & 63; c < nchunks; c += 64) {
     const double* p = part + (row * nchunks + c) * 3;
     mn = fmin(mn, p[0]);
     mx = fmax(mx, p[1]);
     nan += p[2];
   }
+  mn = mc_wave_min(mn);
+  mx = mc_wave_max(mx);
+  nan = mc_wave_sum(nan);
+  if (threadIdx.x & 63) return;
   out[3 * row] = mn;
   out[3 * row + 1] = mx;
   out[3 * row + 2] = nan;
@@ -172,15 +178,20 @@ __global__ __launch_bounds__(kBlock) void k_mc_moments(const T* __restrict__ x, 
   }
 }
 
-__global__ void k_mc_moments_final(int64_t rows, int64_t nchunks, const double* __restrict__ part,
-                                   double* __restrict__ out) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+// One wave per sum: lane l adds the chunks l, l + 64, ... in order, then a
+// butterfly adds the lanes.
+__global__ __launch_bounds__(kBlock) void k_mc_moments_final(int64_t rows, int64_t nchunks,
+                                                             const double* __restrict__ part,
+                                                             double* __restrict__ out) {
+  const int64_t t = (int64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
   if (t >= rows * kMcMoments) return;
   const int64_t row = t / kMcMoments;
   const int k = (int)(t % kMcMoments);
   double a = 0.0;
-  for (int64_t c = 0; c < nchunks; ++c) a += part[(row * nchunks + c) * kMcMoments + k];
-  out[t] = a;
+  for (int64_t c = threadIdx.x & 63; c < nchunks; c += 64)
+    a += part[(row * nchunks + c) * kMcMoments + k];
+  a = mc_wave_sum(a);
+  if ((threadIdx.x & 63) == 0) out[t] = a;
 }
 
 __global__ void k_zero_u64(unsigned long long* __restrict__ p, int64_t n) {
@@ -229,7 +240,7 @@ __device__ __forceinline__ int mc_bin(const double* e, int nb, double v) {
 // memory.  Without LDS (more bins than fit), global 64-bit atomics.
 template <typename T, bool LDS>
 __global__ __launch_bounds__(kBlock) void k_mc_histogram(const T* __restrict__ x, int64_t paths,
-                                                         int64_t n, int use,
+                                                         int64_t n, int64_t span, int use,
                                                          const double* __restrict__ edges,
                                                          int nb, int uniform, int copies,
                                                          unsigned long long* __restrict__ counts) {
@@ -253,8 +264,8 @@ __global__ __launch_bounds__(kBlock) void k_mc_histogram(const T* __restrict__ x
   }
   const double lo_edge = e[0], hi_edge = e[nb];
   const double scale = hi_edge > lo_edge ? (double)nb / (hi_edge - lo_edge) : 0.0;
-  const int64_t lo = chunk * kMcHistChunk;
-  const int64_t hi = lo + kMcHistChunk < n ? lo + kMcHistChunk : n;
+  const int64_t lo = chunk * span;
+  const int64_t hi = lo + span < n ? lo + span : n;
   auto visit = [&](T t) {
     const double v = (double)t;
     const int b = (v >= lo_edge && v <= hi_edge)
@@ -325,6 +336,17 @@ __global__ void k_chf_final(int64_t n, int64_t nchunks, const double* __restrict
   double a = 0.0;
   for (int64_t c = 0; c < nchunks; ++c) a += part[(rk * nchunks + c) * 2 + j];
   out[t] = a;
+}
+
+// Values counted by one histogram block.  Enough blocks to fill the card (2048,
+// 8 per CU) come before large chunks: the last row of 500,000 values takes 12
+// us in chunks of 4096 and 54 in 8 blocks of 65536.  Where the rows fill it
+// anyway, the flush of each block's counts is what more blocks cost: 253 rows
+// of 500,000 take 162 us in chunks of 4096, 136 of 8192, 108 of 65536.
+static int64_t hist_span(int64_t rows, int64_t n) {
+  const int64_t per = rows * n / 2048;
+  const int64_t span = (per + kMcHistMin - 1) / kMcHistMin * kMcHistMin;
+  return span < kMcHistMin ? kMcHistMin : span > kMcHistMax ? kMcHistMax : span;
 }
 
 struct McShape {
@@ -410,7 +432,7 @@ extern "C" int sdegpu_mc_minmax(const void* x, int32_t dtype, int64_t rows, int6
     hipLaunchKernelGGL(k_mc_minmax<double>, grid, dim3(kBlock), 0, st, (const double*)x, paths,
                        sh.n, sh.nchunks, use, part);
   if (int e = launch_status("k_mc_minmax")) return e;
-  hipLaunchKernelGGL(k_mc_minmax_final, dim3(blocks_for(rows)), dim3(kBlock), 0, st, rows,
+  hipLaunchKernelGGL(k_mc_minmax_final, dim3(blocks_for(rows, kBlock / 64)), dim3(kBlock), 0, st, rows,
                      sh.nchunks, (const double*)part, out);
   return launch_status("k_mc_minmax_final");
 }
@@ -434,8 +456,8 @@ extern "C" int sdegpu_mc_moments(const void* x, int32_t dtype, int64_t rows, int
     hipLaunchKernelGGL(k_mc_moments<double>, grid, dim3(kBlock), 0, st, (const double*)x, paths,
                        sh.n, sh.nchunks, use, center, part);
   if (int e = launch_status("k_mc_moments")) return e;
-  hipLaunchKernelGGL(k_mc_moments_final, dim3(blocks_for(rows * kMcMoments)), dim3(kBlock), 0, st,
-                     rows, sh.nchunks, (const double*)part, out);
+  hipLaunchKernelGGL(k_mc_moments_final, dim3(blocks_for(rows * kMcMoments, kBlock / 64)),
+                     dim3(kBlock), 0, st, rows, sh.nchunks, (const double*)part, out);
   return launch_status("k_mc_moments_final");
 }
 
@@ -450,7 +472,8 @@ extern "C" int sdegpu_mc_histogram(const void* x, int32_t dtype, int64_t rows, i
   const int64_t nc = rows * (int64_t)(nbins + 1);
   hipLaunchKernelGGL(k_zero_u64, dim3(blocks_for(nc)), dim3(kBlock), 0, st, counts, nc);
   if (int e = launch_status("k_zero_u64")) return e;
-  const dim3 grid((unsigned)((sh.n + kMcHistChunk - 1) / kMcHistChunk), (unsigned)rows);
+  const int64_t span = hist_span(rows, sh.n);
+  const dim3 grid((unsigned)((sh.n + span - 1) / span), (unsigned)rows);
   const bool lds = nbins <= kMcLdsBins;
   // counter copies: a power of two up to 16 within kMcLdsCounterWords words
   int copies = 1;
@@ -462,17 +485,17 @@ extern "C" int sdegpu_mc_histogram(const void* x, int32_t dtype, int64_t rows, i
   if (dtype == SDEGPU_F32) {
     if (lds)
       hipLaunchKernelGGL((k_mc_histogram<float, true>), grid, dim3(kBlock), lds_bytes, st,
-                         (const float*)x, paths, sh.n, use, edges, nbins, up, copies, counts);
+                         (const float*)x, paths, sh.n, span, use, edges, nbins, up, copies, counts);
     else
       hipLaunchKernelGGL((k_mc_histogram<float, false>), grid, dim3(kBlock), 0, st,
-                         (const float*)x, paths, sh.n, use, edges, nbins, up, 1, counts);
+                         (const float*)x, paths, sh.n, span, use, edges, nbins, up, 1, counts);
   } else {
     if (lds)
       hipLaunchKernelGGL((k_mc_histogram<double, true>), grid, dim3(kBlock), lds_bytes, st,
-                         (const double*)x, paths, sh.n, use, edges, nbins, up, copies, counts);
+                         (const double*)x, paths, sh.n, span, use, edges, nbins, up, copies, counts);
     else
       hipLaunchKernelGGL((k_mc_histogram<double, false>), grid, dim3(kBlock), 0, st,
-                         (const double*)x, paths, sh.n, use, edges, nbins, up, 1, counts);
+                         (const double*)x, paths, sh.n, span, use, edges, nbins, up, 1, counts);
   }
   return launch_status("k_mc_histogram");
 }
