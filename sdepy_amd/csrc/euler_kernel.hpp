@@ -165,6 +165,61 @@ __device__ __forceinline__ void heston_next(T& x, T& y, int& cnt, T mu, T sig, T
   y = y + (ayt * ds + ayw * dwy);
 }
 
+// The constants of one step of a single Heston pair, with ds, sqrt|ds|, the
+// correlation and the parameters multiplied out:
+//   log x += mu0 - h y+ + sqrt(y+) (s z0)
+//   y     += k0 - k y+ + sqrt(y+) (a z0 + b z1)
+template <typename T>
+struct alignas(16) HestonRow {
+  T mu0, h, s, k0, k, a, b, unused;
+};
+
+// The row of table row c, in FP64 and rounded once.
+template <typename T>
+__device__ __forceinline__ HestonRow<T> heston_row(const T* c, int poff, bool corr) {
+  const double ds = (double)c[0], sq = (double)c[1];
+  const T* p = c + poff;
+  const double mu = (double)p[0], sig = (double)p[1], th = (double)p[2], kk = (double)p[3],
+               xi = (double)p[4];
+  const double l0 = corr ? (double)c[2] : 1.0, l1 = corr ? (double)c[3] : 0.0,
+               l2 = corr ? (double)c[4] : 1.0;
+  HestonRow<T> r;
+  r.mu0 = (T)(mu * ds);
+  r.h = (T)(0.5 * sig * sig * ds);
+  r.s = (T)(sig * sq * l0);
+  r.k0 = (T)(kk * th * ds);
+  r.k = (T)(kk * ds);
+  r.a = (T)(xi * sq * l1);
+  r.b = (T)(xi * sq * l2);
+  r.unused = (T)0;
+  return r;
+}
+
+// max(y, 0), 0 for a NaN.  The median with a bound that the compiler cannot see
+// is one instruction; a maximum comes with another that quiets NaNs.
+__device__ __forceinline__ float positive_part(float y, float inf) {
+  return __builtin_amdgcn_fmed3f(y, 0.f, inf);
+}
+__device__ __forceinline__ double positive_part(double y, double) { return fmax(y, 0.0); }
+
+template <typename T>
+__device__ __forceinline__ T opaque_inf() {
+  T v = (T)__builtin_inff();
+  asm("" : "+v"(v));
+  return v;
+}
+
+// heston_next from the multiplied-out constants and two standard normals
+template <typename T>
+__device__ __forceinline__ void heston_next(T& x, T& y, int& cnt, const HestonRow<T>& r, T z0,
+                                            T z1, T inf) {
+  cnt += (y < (T)0) ? 1 : 0;
+  const T yp = positive_part(y, inf);
+  const T sy = fast_sqrt<T>(yp);
+  x = x + fma(sy, r.s * z0, fma(-r.h, yp, r.mu0));
+  y = y + fma(sy, fma(r.b, z1, r.a * z0), fma(-r.k, yp, r.k0));
+}
+
 // The word below which every Poisson word of a pass is a count of 0: a word w
 // draws 0 when (w + 0.5) 2^-32 <= exp(-lam |ds|), so every w below the smallest
 // exp(-lam |ds|) 2^32 of the n table rows does, whatever its step; words
@@ -417,6 +472,7 @@ __global__ __launch_bounds__(kBlock, MOM ? 8 : 1) void k_euler(const EulerArgs a
   constexpr bool kDefer = kJump && DEFER;
   constexpr bool kHeston = MODEL == SDEGPU_MODEL_HESTON;
   constexpr int N = kHeston ? M / 2 : M;
+  constexpr bool kRow = kHeston && M == 2 && !GEN && !PP;
 
   gauss_init<T>();
   // words below it are counts of 0 (per-path intensities: none are known to be)
@@ -539,10 +595,37 @@ __global__ __launch_bounds__(kBlock, MOM ? 8 : 1) void k_euler(const EulerArgs a
     njev = 0;
   };
 
+  // One Heston pair: the wave multiplies the constants of its next steps
+  // out, a lane a step, into LDS of its own, and each step reads them from there
+  // into vector registers (an instruction takes one scalar operand only).  The
+  // kernel is bound by the issue of its vector instructions: a Heston step takes
+  // 44 of them so and took 57 from the table's rows.  FP32, 2 rows: Heston 2M x
+  // 730 1790 -> 1435 us (FP64 1M x 200 658 -> 623).
+  // With row moments the LDS columns leave room for 16 steps only at the same
+  // number of blocks per CU.
+  constexpr int kRowSteps = MOM ? 16 : 64;
+  __shared__ HestonRow<T> hrow[kRow ? kWaves : 1][kRow ? kRowSteps : 1];
+  const HestonRow<T>* hr = nullptr;
+  const T inf = kRow ? opaque_inf<T>() : (T)0;
+  auto fill_rows = [&](int s0) {
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int nw = MOM ? 64 : wave_paths(a, w);  // the lanes that are here
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    for (int i = threadIdx.x & 63; i < kRowSteps && s0 + i < a.nsteps; i += nw)
+      hrow[w][i] = heston_row<T>(coef + (int64_t)(s0 + i) * a.ncoef, a.poff, a.has_corr);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    hr = hrow[w];
+  };
+
   const bool replay = GEN && a.replay_dw != nullptr;
   const bool replay_j = GEN && a.replay_dj != nullptr;
 
   for (int s0 = 0; s0 < a.nsteps; s0 += CH) {
+    if constexpr (kRow) {
+      if (s0 % kRowSteps == 0) fill_rows(s0);
+    }
     T z[NZ];
     uint32_t upois[kJump ? NZ : 1];
     if (!replay) {
@@ -595,7 +678,9 @@ __global__ __launch_bounds__(kBlock, MOM ? 8 : 1) void k_euler(const EulerArgs a
       constexpr bool kOU = MODEL == SDEGPU_MODEL_OU;
       const bool ou_folded = kOU && a.has_corr && !replay && !PP;
       T dw[M];
-      if (replay) {
+      if constexpr (kRow) {
+        // from z
+      } else if (replay) {
         const T* rp = (const T*)a.replay_dw + ((int64_t)s * mt + c0) * P + gid;
 #pragma unroll
         for (int v = 0; v < M; ++v) dw[v] = rp[v * P];
@@ -663,6 +748,8 @@ __global__ __launch_bounds__(kBlock, MOM ? 8 : 1) void k_euler(const EulerArgs a
 #pragma unroll
         for (int v = 0; v < M; ++v)
           x[v] = cir_next<T>(x[v], p[v], p[M + v], p[2 * M + v], ds, dw[v]);
+      } else if constexpr (kRow) {
+        heston_next<T>(x[0], x[1], cnt[0], hr[s0 % kRowSteps + k], z[2 * k], z[2 * k + 1], inf);
       } else if constexpr (kHeston) {
         using L = HestonLayout<D>;
 #pragma unroll
