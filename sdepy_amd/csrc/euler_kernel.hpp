@@ -25,6 +25,8 @@
 // correlated OU-4 kernel: 93 instead of 106), which lets 8 waves share a
 // SIMD instead of 7.
 #pragma once
+#include <type_traits>
+
 #include "common.hpp"
 #include "jumps.hpp"
 #include "philox.hpp"
@@ -165,8 +167,10 @@ __device__ __forceinline__ void heston_next(T& x, T& y, int& cnt, T mu, T sig, T
   y = y + (ayt * ds + ayw * dwy);
 }
 
-// The constants of one step of a single Heston pair, with ds, sqrt|ds|, the
-// correlation and the parameters multiplied out:
+// The constants of one step, multiplied out in FP64 and rounded once.
+//
+// For a single Heston pair, with ds, sqrt|ds|, the
+// correlation and the parameters:
 //   log x += mu0 - h y+ + sqrt(y+) (s z0)
 //   y     += k0 - k y+ + sqrt(y+) (a z0 + b z1)
 template <typename T>
@@ -174,16 +178,14 @@ struct alignas(16) HestonRow {
   T mu0, h, s, k0, k, a, b, unused;
 };
 
-// The row of table row c, in FP64 and rounded once.
 template <typename T>
-__device__ __forceinline__ HestonRow<T> heston_row(const T* c, int poff, bool corr) {
+__device__ __forceinline__ void fill_row(HestonRow<T>& r, const T* c, int poff, bool corr) {
   const double ds = (double)c[0], sq = (double)c[1];
   const T* p = c + poff;
   const double mu = (double)p[0], sig = (double)p[1], th = (double)p[2], kk = (double)p[3],
                xi = (double)p[4];
   const double l0 = corr ? (double)c[2] : 1.0, l1 = corr ? (double)c[3] : 0.0,
                l2 = corr ? (double)c[4] : 1.0;
-  HestonRow<T> r;
   r.mu0 = (T)(mu * ds);
   r.h = (T)(0.5 * sig * sig * ds);
   r.s = (T)(sig * sq * l0);
@@ -192,7 +194,18 @@ __device__ __forceinline__ HestonRow<T> heston_row(const T* c, int poff, bool co
   r.a = (T)(xi * sq * l1);
   r.b = (T)(xi * sq * l2);
   r.unused = (T)0;
-  return r;
+}
+
+// The same for one additive component: x += b + s z.
+template <typename T>
+struct alignas(2 * sizeof(T)) AddRow {
+  T b, s;
+};
+
+template <typename T>
+__device__ __forceinline__ void fill_row(AddRow<T>& r, const T* c, int poff, bool corr) {
+  r.b = (T)((double)c[poff] * (double)c[0]);
+  r.s = (T)((double)c[poff + 1] * (double)c[1] * (corr ? (double)c[2] : 1.0));
 }
 
 // max(y, 0), 0 for a NaN.  The median with a bound that the compiler cannot see
@@ -472,7 +485,10 @@ __global__ __launch_bounds__(kBlock, MOM ? 8 : 1) void k_euler(const EulerArgs a
   constexpr bool kDefer = kJump && DEFER;
   constexpr bool kHeston = MODEL == SDEGPU_MODEL_HESTON;
   constexpr int N = kHeston ? M / 2 : M;
-  constexpr bool kRow = kHeston && M == 2 && !GEN && !PP;
+  constexpr bool kAdd1 = (kJump || MODEL == SDEGPU_MODEL_WIENER || MODEL == SDEGPU_MODEL_LOGNORM) &&
+                         M == 1 && !GEN && !PP;
+  constexpr bool kRow = (kHeston && M == 2 && !GEN && !PP) || kAdd1;
+  using Row = std::conditional_t<kHeston, HestonRow<T>, AddRow<T>>;
 
   gauss_init<T>();
   // words below it are counts of 0 (per-path intensities: none are known to be)
@@ -595,25 +611,26 @@ __global__ __launch_bounds__(kBlock, MOM ? 8 : 1) void k_euler(const EulerArgs a
     njev = 0;
   };
 
-  // One Heston pair: the wave multiplies the constants of its next steps
+  // One Heston pair or one additive component: the wave multiplies the constants of its next steps
   // out, a lane a step, into LDS of its own, and each step reads them from there
   // into vector registers (an instruction takes one scalar operand only).  The
   // kernel is bound by the issue of its vector instructions: a Heston step takes
   // 44 of them so and took 57 from the table's rows.  FP32, 2 rows: Heston 2M x
-  // 730 1790 -> 1435 us (FP64 1M x 200 658 -> 623).
+  // 730 1790 -> 1435 us (FP64 1M x 200 658 -> 623), lognormal 1M x 252 160 -> 125, Merton
+  // 2M x 252 625 -> 580.
   // With row moments the LDS columns leave room for 16 steps only at the same
   // number of blocks per CU.
   constexpr int kRowSteps = MOM ? 16 : 64;
-  __shared__ HestonRow<T> hrow[kRow ? kWaves : 1][kRow ? kRowSteps : 1];
-  const HestonRow<T>* hr = nullptr;
-  const T inf = kRow ? opaque_inf<T>() : (T)0;
+  __shared__ Row hrow[kRow ? kWaves : 1][kRow ? kRowSteps : 1];
+  const Row* hr = nullptr;
+  const T inf = kHeston && kRow ? opaque_inf<T>() : (T)0;
   auto fill_rows = [&](int s0) {
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int nw = MOM ? 64 : wave_paths(a, w);  // the lanes that are here
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
     for (int i = threadIdx.x & 63; i < kRowSteps && s0 + i < a.nsteps; i += nw)
-      hrow[w][i] = heston_row<T>(coef + (int64_t)(s0 + i) * a.ncoef, a.poff, a.has_corr);
+      fill_row<T>(hrow[w][i], coef + (int64_t)(s0 + i) * a.ncoef, a.poff, a.has_corr);
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
     hr = hrow[w];
@@ -720,7 +737,10 @@ __global__ __launch_bounds__(kBlock, MOM ? 8 : 1) void k_euler(const EulerArgs a
         }
         p = prow;
       }
-      if constexpr (MODEL == SDEGPU_MODEL_WIENER || MODEL == SDEGPU_MODEL_LOGNORM) {
+      if constexpr (kAdd1 && !kJump) {
+        const Row r = hr[s0 % kRowSteps + k];
+        x[0] = x[0] + fma(r.s, z[k], r.b);
+      } else if constexpr (MODEL == SDEGPU_MODEL_WIENER || MODEL == SDEGPU_MODEL_LOGNORM) {
         // wiener_SDE: {'dt': mu, 'dw': sigma}; lognorm_SDE: {'dt': mu - sigma^2/2, 'dw': sigma}
 #pragma unroll
         for (int v = 0; v < M; ++v) x[v] = x[v] + (p[v] * ds + p[M + v] * dw[v]);
@@ -748,7 +768,7 @@ __global__ __launch_bounds__(kBlock, MOM ? 8 : 1) void k_euler(const EulerArgs a
 #pragma unroll
         for (int v = 0; v < M; ++v)
           x[v] = cir_next<T>(x[v], p[v], p[M + v], p[2 * M + v], ds, dw[v]);
-      } else if constexpr (kRow) {
+      } else if constexpr (kHeston && kRow) {
         heston_next<T>(x[0], x[1], cnt[0], hr[s0 % kRowSteps + k], z[2 * k], z[2 * k + 1], inf);
       } else if constexpr (kHeston) {
         using L = HestonLayout<D>;
@@ -763,8 +783,13 @@ __global__ __launch_bounds__(kBlock, MOM ? 8 : 1) void k_euler(const EulerArgs a
         // dj = sign(ds) * sum of n ~ Poisson(lam*|ds|) jump sizes of the law
         // jump_law (cpoisson_source.__call__; norm_rv(a, b) for Merton).
         T inc[M];
+        if constexpr (kAdd1) {
+          const Row r = hr[s0 % kRowSteps + k];
+          inc[0] = fma(r.s, z[k], r.b);
+        } else {
 #pragma unroll
-        for (int v = 0; v < M; ++v) inc[v] = p[v] * ds + p[M + v] * dw[v];
+          for (int v = 0; v < M; ++v) inc[v] = p[v] * ds + p[M + v] * dw[v];
+        }
         if (replay_j) {
           const T* rp = (const T*)a.replay_dj + ((int64_t)s * mt + c0) * P + gid;
 #pragma unroll
