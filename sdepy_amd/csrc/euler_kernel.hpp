@@ -173,9 +173,16 @@ __device__ __forceinline__ void heston_next(T& x, T& y, int& cnt, T mu, T sig, T
 // correlation and the parameters:
 //   log x += mu0 - h y+ + sqrt(y+) (s z0)
 //   y     += k0 - k y+ + sqrt(y+) (a z0 + b z1)
+// In FP32 y keeps heston_next's operations, from constants that are not
+// multiplied out: another rounding of y would move its sign, and with it the count of
+// negative values, now and then (one path of 300,000 in 200 steps).
 template <typename T>
 struct alignas(16) HestonRow {
   T mu0, h, s, k0, k, a, b, unused;
+};
+template <>
+struct alignas(16) HestonRow<float> {
+  float mu0, h, s, l1, l2, sq, xi, kk, th, ds, unused[2];
 };
 
 template <typename T>
@@ -189,11 +196,20 @@ __device__ __forceinline__ void fill_row(HestonRow<T>& r, const T* c, int poff, 
   r.mu0 = (T)(mu * ds);
   r.h = (T)(0.5 * sig * sig * ds);
   r.s = (T)(sig * sq * l0);
-  r.k0 = (T)(kk * th * ds);
-  r.k = (T)(kk * ds);
-  r.a = (T)(xi * sq * l1);
-  r.b = (T)(xi * sq * l2);
-  r.unused = (T)0;
+  if constexpr (sizeof(T) == 8) {
+    r.k0 = kk * th * ds;
+    r.k = kk * ds;
+    r.a = xi * sq * l1;
+    r.b = xi * sq * l2;
+  } else {
+    r.l1 = (T)l1;
+    r.l2 = (T)l2;
+    r.sq = (T)sq;
+    r.xi = (T)xi;
+    r.kk = (T)kk;
+    r.th = (T)th;
+    r.ds = (T)ds;
+  }
 }
 
 // The same for one additive component: x += b + s z.
@@ -230,7 +246,12 @@ __device__ __forceinline__ void heston_next(T& x, T& y, int& cnt, const HestonRo
   const T yp = positive_part(y, inf);
   const T sy = fast_sqrt<T>(yp);
   x = x + fma(sy, r.s * z0, fma(-r.h, yp, r.mu0));
-  y = y + fma(sy, fma(r.b, z1, r.a * z0), fma(-r.k, yp, r.k0));
+  if constexpr (sizeof(T) == 8) {
+    y = y + fma(sy, fma(r.b, z1, r.a * z0), fma(-r.k, yp, r.k0));
+  } else {
+    const T dwy = fma(r.l2, z1, r.l1 * z0) * r.sq;
+    y = y + fma(r.kk * (r.th - yp), r.ds, r.xi * sy * dwy);
+  }
 }
 
 // The word below which every Poisson word of a pass is a count of 0: a word w
@@ -485,7 +506,10 @@ __global__ __launch_bounds__(kBlock, MOM ? 8 : 1) void k_euler(const EulerArgs a
   constexpr bool kDefer = kJump && DEFER;
   constexpr bool kHeston = MODEL == SDEGPU_MODEL_HESTON;
   constexpr int N = kHeston ? M / 2 : M;
-  constexpr bool kAdd1 = (kJump || MODEL == SDEGPU_MODEL_WIENER || MODEL == SDEGPU_MODEL_LOGNORM) &&
+  // (FP32 Wiener and lognormal states keep p ds + sigma dw: rounded otherwise, a
+  // value in a million of theirs changes its bin in a histogram)
+  constexpr bool kAdd1 = (kJump || (sizeof(T) == 8 && (MODEL == SDEGPU_MODEL_WIENER ||
+                                                       MODEL == SDEGPU_MODEL_LOGNORM))) &&
                          M == 1 && !GEN && !PP;
   constexpr bool kRow = (kHeston && M == 2 && !GEN && !PP) || kAdd1;
   using Row = std::conditional_t<kHeston, HestonRow<T>, AddRow<T>>;
@@ -614,13 +638,14 @@ __global__ __launch_bounds__(kBlock, MOM ? 8 : 1) void k_euler(const EulerArgs a
   // One Heston pair or one additive component: the wave multiplies the constants of its next steps
   // out, a lane a step, into LDS of its own, and each step reads them from there
   // into vector registers (an instruction takes one scalar operand only).  The
-  // kernel is bound by the issue of its vector instructions: a Heston step takes
-  // 44 of them so and took 57 from the table's rows.  FP32, 2 rows: Heston 2M x
-  // 730 1790 -> 1435 us (FP64 1M x 200 658 -> 623), lognormal 1M x 252 160 -> 125, Merton
-  // 2M x 252 625 -> 580.
-  // With row moments the LDS columns leave room for 16 steps only at the same
-  // number of blocks per CU.
-  constexpr int kRowSteps = MOM ? 16 : 64;
+  // kernel is bound by the issue of its vector instructions: an FP64 Heston step takes
+  // 44 of them so and took 57 from the table's rows, an FP32 one 48.  2 rows:
+  // Heston FP32 4M x 365 1787 -> 1499 us (y's constants as scalars from the table,
+  // x's from LDS: 1640), FP64 1M x 200 658 -> 623; Merton FP32 2M x 252 625 -> 580;
+  // lognormal FP64 1M x 252 329 -> 300.
+  // With row moments the LDS columns leave room for 16 steps (8 of 48 bytes) only
+  // at the same number of blocks per CU.
+  constexpr int kRowSteps = !MOM ? 64 : sizeof(Row) > 32 ? 8 : 16;
   __shared__ Row hrow[kRow ? kWaves : 1][kRow ? kRowSteps : 1];
   const Row* hr = nullptr;
   const T inf = kHeston && kRow ? opaque_inf<T>() : (T)0;

@@ -66,3 +66,17 @@ def test_rows_equal_table(gpu, monkeypatch, name, nsteps, dtype):
     first = _stack(x)[0].astype(np.float64)
     mean = _stack(run.pmean())[0]
     assert np.allclose(np.squeeze(mean), first.mean(axis=-1), rtol=1e-6, atol=1e-12)
+
+
+@pytest.mark.parametrize('name', ['gbm', 'heston', 'heston_uncorrelated'])
+def test_f32_whole_numbers_as_from_the_table(gpu, name):
+    # FP32: the variance (its sign is counted) and lognormal values (histograms
+    # bin them) carry the rounding of the table's rows, bit for bit
+    nsteps, few = 131, 5000
+    tt = np.linspace(0., 1., nsteps + 1)[[0, 40, nsteps]]
+    ref_info, info = {}, {}
+    ref = _stack(_process(name, np.float32, few, nsteps, ref_info)(tt))[-1]
+    got = _stack(_process(name, np.float32, ALONE, nsteps, info)(tt))[-1]
+    assert np.array_equal(got[..., :few], ref)
+    if 'negative_y_count' in info:
+        assert np.array_equal(info['negative_y_count'][..., :few], ref_info['negative_y_count'])
