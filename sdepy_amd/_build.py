@@ -27,6 +27,11 @@ HIPCC_FLAGS = [
 ]
 
 
+# units whose kernels hold too many registers when the constants of exp and
+# of the normals are kept in them through the step loop
+UNIT_FLAGS = {'euler_wide_f64.hip': ['-mllvm', '-disable-machine-licm']}
+
+
 def hipcc():
     path = shutil.which('hipcc') or '/opt/rocm/bin/hipcc'
     if not os.path.exists(path):
@@ -42,7 +47,7 @@ def sources():
 
 def _compile(src, verbose):
     obj = os.path.join(OBJDIR, os.path.basename(src)[:-4] + '.o')
-    cmd = [hipcc(), *HIPCC_FLAGS, '-I', INCLUDE, '-c', src, '-o', obj]
+    cmd = [hipcc(), *HIPCC_FLAGS, *UNIT_FLAGS.get(os.path.basename(src), ()), '-I', INCLUDE, '-c', src, '-o', obj]
     if verbose:
         print(' '.join(cmd), flush=True)
     res = subprocess.run(cmd, capture_output=True, text=True)

@@ -236,7 +236,9 @@ extern "C" int sdegpu_euler(const sdegpu_euler_problem* pr, void* stream) {
                 "fused row moments with per-path parameters: reduce the output separately");
   const int block_paths = wide ? 64 : kBlock;
   const dim3 grid(blocks_for(pr->paths, block_paths));
-  const dim3 block(wide ? 64 * wide_shape(pr->model, m).waves : kBlock);
+  const dim3 block(!wide ? kBlock
+                   : pr->dtype == SDEGPU_F64 ? 64 * wide_shape<double>(pr->model, m).waves
+                                             : 64 * wide_shape<float>(pr->model, m).waves);
   const bool wide_gen = pr->replay_dw || pr->replay_dj || pp || (jump && pr->lam_paths);
   hipStream_t st = (hipStream_t)stream;
   // runs of few paths: several waves share 64 paths

@@ -5,20 +5,27 @@
 // (wiener_source.__call__, infrastructure.py:1524-1553) and steps it with the
 // same euler_next update as any other state (integration.py:707-723).
 //
-// W waves share 64 paths and split the components: wave w holds components
-// (Heston: pairs) w, w + W, w + 2 W, ..., at most R of them.  Per step the
-// waves draw the block's normals together, one Philox block of 4 after the
-// other, into LDS, and after a barrier each applies its rows of the
-// correlation and steps its components; the cyclic rows give every wave about
-// the same share of the triangle.  The step's table row is fetched a step ahead and
-// spread out in LDS as a square with zeros above the diagonal, so that a wave
-// reads its coefficients as 16-byte broadcasts at fixed offsets (with scalar
-// loads and a wait per piece of a row the kernel took twice as long).  Bound
-// by LDS reads and VALU about equally.  One lane per path with the whole
-// state, which this replaces, took up to 256 registers, one or two waves
-// per SIMD, and its FP64 jump instances spilled: 100,000 paths x 252 steps of
-// 20 correlated lognormals FP64 2.54 ms, 1.64 ms now; 64 of them, 20,000 x
-// 100, 4.88 and 1.12 ms; FP32 12 of them, 200,000 x 100, 0.68 and 0.28 ms.
+// W waves share 64 paths.  Per step they draw the block's normals together, one
+// Philox block of 4 after the other, into LDS, and after a barrier each applies
+// the correlation and steps the components that it holds, at most R per lane.
+// The step's table row is fetched a step ahead and spread out in LDS as a square
+// with zeros above the diagonal.
+//
+// FP64: a wave holds 16 paths, a lane one component in four of one path, and
+// v_mfma_f64_4x4x4 multiplies four rows of the square by four normals of the 16
+// paths.  Its operands are one 8-byte LDS read each, 512 bytes for 256
+// multiply-adds; as 16-byte broadcasts to lanes of 64 paths the coefficients
+// took 1024 bytes for 128, and the kernel was bound by those reads (the LDS at
+// work 56% of the time, the vector units 48%).  Now half of what is left is
+// normals, and the waits at the two barriers of a step.
+// FP32: a wave holds components (Heston: pairs) w, w + W, w + 2 W, ... of all 64
+// paths and reads its coefficients as 16-byte broadcasts, four at a time, at
+// fixed offsets (with scalar loads and a wait per piece of a row it took
+// twice as long).
+// One lane per path with the whole state, which both replace, took up to
+// 256 registers, one or two waves per SIMD.  100 steps: 20 correlated lognormals
+// FP64, 100,000 paths, 1010 us so, 680 with broadcasts, 553 now; 64 of
+// them, 20,000 paths, 4880, 1140 and 656; FP32 12 of them, 200,000 paths, 680 and 280.
 //
 // The block's width m is a run-time value.  The kernel does everything the
 // general k_euler instance does (component groups, recorded increments,
@@ -28,7 +35,7 @@
 // in sdepy's order.
 //
 // Correlation: dw = L z sqrt|ds| with the packed Cholesky rows of the step,
-// row i summed over j = 0..i in order, as in k_euler; the sum runs on over the zeros
+// row i summed over j = 0..i in order (FP64: four at a time), as in k_euler; the sum runs on over the zeros
 // of the square (of the coefficients and of the normals past the width).
 #pragma once
 #include "euler_kernel.hpp"
@@ -40,18 +47,39 @@ struct Flag {
   static constexpr bool value = B;
 };
 
+// FP64 applies the correlation on the matrix cores, with v_mfma_f64_4x4x4: four
+// components by 16 paths, of four normals each.
+template <typename T>
+constexpr bool kWideMat = sizeof(T) == 8;
+
 // The square of one row's coefficients: N rows and columns, the columns
-// padded to whole 16-byte reads.
+// padded to whole 16-byte reads (FP64: against bank conflicts of its 4 x 4
+// pieces, whose rows must not lie a multiple of 128 bytes apart).
 template <typename T, int N>
 struct WideSquare {
   static constexpr int CK = 16 / sizeof(T);  // coefficients per LDS read
-  static constexpr int COLS = (N + CK - 1) / CK * CK;
+  static constexpr int COLS = kWideMat<T> ? N + (N % 16 == 0 ? 4 : 0) : (N + CK - 1) / CK * CK;
   static constexpr int SIZE = N * COLS;
 };
 
+// Waves per SIMD that the compiler has to leave registers for.  A wave waits at
+// two barriers a step, and what hides that are the other blocks of the CU: as
+// many as the LDS has room for, or fewer where the registers would be
+// spilled.  20 correlated lognormals FP64, 100,000 x 100: 4, 5, 6, 7 waves 593, 593, 599, 560
+// us; 40 of them, 40,000 x 100: 685, 683, 603, (no room) 687; FP32 4
+// and 6 waves: 502 and 412.  Jumps FP64, 40 of 40,000 x 100: 4, 5 waves 1601, 2159.
+template <int MODEL, typename T, int W, int R, bool GEN>
+constexpr int wide_occupancy() {
+  constexpr bool jump = MODEL == SDEGPU_MODEL_JUMPDIFF, heston = MODEL == SDEGPU_MODEL_HESTON;
+  if (!kWideMat<T>) return W == 6 ? (jump ? 5 : 6) : W == 3 && (heston || (jump && R == 7)) ? 5 : 4;
+  if (jump) return W == 4 && !GEN ? 5 : R == 8 ? 2 : 4;
+  if (GEN || (heston ? W * R == 32 : W * R == 64)) return 4;
+  return W == 4 && R < 6 && !heston ? 7 : 6;
+}
+
 // GEN: recorded increments, per-path parameters and per-path intensities.
 template <int MODEL, typename T, int W, int R, bool GEN>
-__global__ __launch_bounds__(64 * W) void k_euler_wide(const EulerArgs a,
+__global__ __launch_bounds__(64 * W, (wide_occupancy<MODEL, T, W, R, GEN>())) void k_euler_wide(const EulerArgs a,
                                                        const T* __restrict__ coef,
                                                        const int32_t* __restrict__ store_row,
                                                        const double* __restrict__ pois,
@@ -59,19 +87,28 @@ __global__ __launch_bounds__(64 * W) void k_euler_wide(const EulerArgs a,
   constexpr bool kJump = MODEL == SDEGPU_MODEL_JUMPDIFF;
   constexpr bool kHeston = MODEL == SDEGPU_MODEL_HESTON;
   constexpr bool kOU = MODEL == SDEGPU_MODEL_OU;
+  constexpr bool kMat = kWideMat<T>;
   constexpr int N = R * W;
   using Sq = WideSquare<T, N>;
   constexpr int CK = Sq::CK, COLS = Sq::COLS;
   constexpr int NS = kHeston ? 3 : 1;  // squares: of log x (or all); y by x, y by y
   constexpr int NB = kHeston ? 2 : 1;  // normals' buffers: of log x (or all), of y
   constexpr int NPAR = 5 * N;
-  __shared__ __align__(16) T chol[NS * Sq::SIZE];
-  __shared__ __align__(16) T par_lds[2 + NPAR];  // ds, sqrt|ds|, the parameter blocks
+  // the squares, then ds, sqrt|ds| and the parameter blocks
+  constexpr int NTAB = NS * Sq::SIZE + 2 + NPAR;
+  __shared__ __align__(16) T chol[NTAB];
+  T* const par_lds = chol + NS * Sq::SIZE;
   __shared__ T z[NB][COLS][64];
   __shared__ uint32_t words[kJump ? N : 1][kJump ? 64 : 1];
 
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // A lane draws for path `lane` of the block and steps the state of path `pl`.
+  const int quad = lane >> 4;
+  const int pl = kMat ? 16 * (w & 3) + (lane & 15) : lane;
+  // where a row of z holds a path's value (FP64: two of the four rows that the
+  // matrix instruction reads at once would meet in the same banks)
+  auto col = [&](int v, int p) { return kMat ? p ^ ((v & 1) << 4) : p; };
   const int m = a.nvars;
   const int n = kHeston ? m / 2 : m;  // width of a parameter block
   gauss_init<T>(64 * W);
@@ -81,22 +118,25 @@ __global__ __launch_bounds__(64 * W) void k_euler_wide(const EulerArgs a,
   const uint32_t zero_below = kJump && !(GEN && (a.replay_dj || a.lamp))
                                   ? zero_count_bound(pois, (int64_t)a.nsteps * m, 64 * W)
                                   : 0u;
-  for (int i = threadIdx.x; i < NS * Sq::SIZE; i += 64 * W) chol[i] = (T)0;
+  for (int i = threadIdx.x; i < NTAB; i += 64 * W) chol[i] = (T)0;
   for (int i = threadIdx.x; i < NB * COLS * 64; i += 64 * W) (&z[0][0][0])[i] = (T)0;
 
   // Table element e of a step: the header and the parameters go to par_lds, the
   // triangle's (i, j) to its square.  Thread t moves elements t, t + 64 W, ...
   constexpr int MAXC = 2 + (kHeston ? 2 * N * (2 * N + 1) / 2 : N * (N + 1) / 2) + NPAR;
   constexpr int NE = (MAXC + 64 * W - 1) / (64 * W);
-  const int ncoef = a.ncoef < 2 + NPAR + (a.poff - 2) ? a.ncoef : 2 + NPAR + (a.poff - 2);
-  T* dst[NE];
+  const int ncoef = a.ncoef < a.poff + 5 * n ? a.ncoef : a.poff + 5 * n;
+  int dst[NE];  // its place in chol (-1: none)
 #pragma unroll
   for (int k = 0; k < NE; ++k) {
     const int e = k * 64 * W + (int)threadIdx.x;
-    dst[k] = nullptr;
+    dst[k] = -1;
     if (e >= ncoef) continue;
-    if (e < 2 || e >= a.poff) {
-      dst[k] = par_lds + (e < 2 ? e : e - (a.poff - 2));
+    if (e < 2) {
+      dst[k] = NS * Sq::SIZE + e;
+    } else if (e >= a.poff) {
+      const int b = (e - a.poff) / n;
+      dst[k] = NS * Sq::SIZE + 2 + b * N + (e - a.poff - b * n);
     } else {
       // row i holds elements i (i + 1) / 2 .. of the packed triangle
       const int q = e - 2;
@@ -105,29 +145,34 @@ __global__ __launch_bounds__(64 * W) void k_euler_wide(const EulerArgs a,
       while (i * (i + 1) / 2 > q) --i;
       const int j = q - i * (i + 1) / 2;
       if (!kHeston || i < n)
-        dst[k] = chol + i * COLS + j;
+        dst[k] = i * COLS + j;
       else if (j < n)
-        dst[k] = chol + Sq::SIZE + (i - n) * COLS + j;
+        dst[k] = Sq::SIZE + (i - n) * COLS + j;
       else
-        dst[k] = chol + 2 * Sq::SIZE + (i - n) * COLS + (j - n);
+        dst[k] = 2 * Sq::SIZE + (i - n) * COLS + (j - n);
     }
   }
   T ahead[NE];
   auto fetch = [&](int s) {
 #pragma unroll
     for (int k = 0; k < NE; ++k)
-      if (dst[k]) ahead[k] = coef[(int64_t)s * a.ncoef + k * 64 * W + (int)threadIdx.x];
+      if (dst[k] >= 0) ahead[k] = coef[(int64_t)s * a.ncoef + k * 64 * W + (int)threadIdx.x];
   };
 
   const int64_t P = a.paths;
-  const int64_t tid = (int64_t)blockIdx.x * 64 + lane;
+  const int64_t tid = (int64_t)blockIdx.x * 64 + pl;
   // lanes beyond the last path step a copy of it and store nothing
   const bool live = tid < P;
   const int64_t gid = live ? tid : P - 1;
-  const uint32_t path = (uint32_t)gid;
-  const bool flip_w = a.anti_w > 0 && gid >= a.anti_w;
-  const uint32_t path_w = flip_w ? (uint32_t)(gid - a.anti_w) : path;
-  const uint32_t path_j = (a.anti_j > 0 && gid >= a.anti_j) ? (uint32_t)(gid - a.anti_j) : path;
+  auto jump_path = [&](int64_t i) {
+    return (uint32_t)(a.anti_j > 0 && i >= a.anti_j ? i - a.anti_j : i);
+  };
+  const uint32_t path_j = jump_path(gid);
+  // the path that the lane draws for
+  const int64_t did = min((int64_t)blockIdx.x * 64 + lane, P - 1);
+  const bool flip_w = a.anti_w > 0 && did >= a.anti_w;
+  const uint32_t path_w = (uint32_t)(flip_w ? did - a.anti_w : did);
+  const uint32_t path_p = jump_path(did);
   const int64_t mt = a.m_total, c0 = a.comp0;
   const int64_t mtb = kHeston ? mt / 2 : mt, c0b = kHeston ? c0 / 2 : c0;
   const T* __restrict__ ppar = (const T*)a.ppar;
@@ -135,16 +180,16 @@ __global__ __launch_bounds__(64 * W) void k_euler_wide(const EulerArgs a,
   auto x0_of = [&](int v) -> T {
     return x0p ? x0p[(c0 + v) * P + gid] : (T)a.x0[v];
   };
-  // the wave's r-th component, and whether it has one (uniform over the wave);
-  // rows without one step zeros
-  auto comp = [&](int r) { return r * W + w; };
-  auto has = [&](int r) { return r * W + w < n; };
+  // the r-th component of the wave (FP64: of the lane), and whether there is one; rows
+  // without one step zeros
+  auto comp = [&](int r) { return kMat ? r * W + (w >> 2) * 4 + quad : r * W + w; };
+  auto has = [&](int r) { return comp(r) < n; };
   // parameter block b of component (Heston: pair) v at a step (per path: at the
   // step's offset pbase into ppar)
   int64_t pbase = 0;
   auto par = [&](int b, int v) -> T {
     if (pp) return v < n ? ppar[pbase + ((int64_t)b * mtb + c0b + v) * P + gid] : (T)0;
-    return par_lds[2 + (v < n ? b * n + v : 0)];
+    return par_lds[2 + b * N + v];
   };
 
   T x[R];  // log x for Heston
@@ -168,39 +213,43 @@ __global__ __launch_bounds__(64 * W) void k_euler_wide(const EulerArgs a,
       __syncthreads();
 #pragma unroll
       for (int r = 0; r < R; ++r)
-        if (has(r)) z[0][comp(r)][lane] = x[r];
+        if (has(r)) z[0][comp(r)][pl] = x[r];
       __syncthreads();
-      if (w == 0 && live) {
+      if (w == 0 && (int64_t)blockIdx.x * 64 + lane < P) {
         T val = (T)0;
         for (int v = 0; v < m; ++v) val = val + z[0][v][lane];
-        __builtin_nontemporal_store(val, o_row);
+        __builtin_nontemporal_store(val, o_row - gid + did);
       }
       return;
     }
     if (!live) return;
+    T* o = o_row + comp(0) * P;  // row r of the wave is r W components further on
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       if (!has(r)) break;
-      const int v = comp(r);
       if constexpr (kHeston) {
-        __builtin_nontemporal_store((T)exp(x[r]), o_row + v * P);
-        if (a.nout == m) __builtin_nontemporal_store(vy[r], o_row + (n + v) * P);
-      } else if (v < a.nout) {
+        __builtin_nontemporal_store((T)exp(x[r]), o);
+        if (a.nout == m) __builtin_nontemporal_store(vy[r], o + n * P);
+      } else if (comp(r) < a.nout) {
         T val = x[r];
         if constexpr (OutRule<MODEL>::exp_all) val = exp(val);
-        __builtin_nontemporal_store(val, o_row + v * P);
+        __builtin_nontemporal_store(val, o);
       }
+      o += W * P;
     }
   };
 
   // The flat indices g .. g+m-1 of a stream lie in Philox blocks g/4 ...; f
-  // gets a block and the component of its first value, wave w every W-th one.
-  auto each_block = [&](uint64_t g, auto f) {
+  // gets a block and the component of its first value, every wave each W-th one.
+  // FP32: the waves take turns at the first, as those that draw one more would
+  // otherwise run on the same SIMD (3 to 10% faster; FP64 is 1 to 3% slower so).
+    int turn = kMat ? w : (int)((blockIdx.x + (unsigned)w) % (unsigned)W);
+  auto each_block = [&](uint64_t g, int first, auto f) {
     const uint32_t b0 = (uint32_t)(g >> 2);
     const int off = (int)(g & 3u);
     const int nb = (off + m + 3) >> 2;
     for (int i = 0; i * W < nb; ++i) {
-      const int q = i * W + w;
+      const int q = i * W + first;
       if (q >= nb) break;
       f(b0 + q, 4 * q - off);
     }
@@ -209,6 +258,24 @@ __global__ __launch_bounds__(64 * W) void k_euler_wide(const EulerArgs a,
   // acc[r] += sum over columns of square[row of r][column] zz[column]; of a
   // triangle only the columns up to the rows r of any wave.
   auto apply = [&](T(&acc)[R], const T* square, const T(*zz)[64], auto triangle) {
+    if constexpr (kMat) {
+      // lane 16 k + 4 b + i holds element (i, k) of the four rows' piece, for
+      // each b, and the normal k of path 16 k + 4 b + j; the sum of component i
+      // of a path comes out in lane 16 i + 4 b + j
+      constexpr int H = W / 4;
+      const T* mine = square + ((w >> 2) * 4 + (lane & 3)) * COLS + quad;
+#pragma unroll
+      for (int c = 0; c < N / 4; ++c) {
+        const T zc = zz[4 * c + quad][col(quad, pl)];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          if (decltype(triangle)::value && (r + 1) * H <= c) continue;
+          acc[r] = __builtin_amdgcn_mfma_f64_4x4x4f64(mine[r * W * COLS + 4 * c], zc, acc[r], 0,
+                                                      0, 0);
+        }
+      }
+      return;
+    }
     const T* mine = square + w * COLS;
 #pragma unroll
     for (int q = 0; q < COLS / CK; ++q) {
@@ -239,9 +306,9 @@ __global__ __launch_bounds__(64 * W) void k_euler_wide(const EulerArgs a,
     // the step's table row, normals and Poisson words into LDS
 #pragma unroll
     for (int k = 0; k < NE; ++k)
-      if (dst[k]) *dst[k] = ahead[k];
+      if (dst[k] >= 0) chol[dst[k]] = ahead[k];
     if (!replay) {
-      each_block(g, [&](uint32_t blk, int v0) {
+      each_block(g, turn, [&](uint32_t blk, int v0) {
         T zz[4];
         normals4<T>(blk, path_w, a.c2w, a.ew, a.kw0, a.kw1, zz);
 #pragma unroll
@@ -250,17 +317,17 @@ __global__ __launch_bounds__(64 * W) void k_euler_wide(const EulerArgs a,
           const T val = flip_w ? -zz[l] : zz[l];
           if (v >= 0 && v < m) {
             if (!kHeston || v < n)
-              z[0][v][lane] = val;
+              z[0][v][col(v, lane)] = val;
             else
-              z[NB - 1][v - n][lane] = val;
+              z[NB - 1][v - n][col(v - n, lane)] = val;
           }
         }
       });
     }
     if constexpr (kJump) {
       if (!replay_j) {
-        each_block(g, [&](uint32_t blk, int v0) {
-          const ctr4 u = philox4x32_10(ctr4{blk, path_j, a.c2p, a.ej}, a.kj0, a.kj1);
+        each_block(g, kMat ? w : W - 1 - turn, [&](uint32_t blk, int v0) {
+          const ctr4 u = philox4x32_10(ctr4{blk, path_p, a.c2p, a.ej}, a.kj0, a.kj1);
           const uint32_t uu[4] = {u.x, u.y, u.z, u.w};
 #pragma unroll
           for (int l = 0; l < 4; ++l)
@@ -268,6 +335,7 @@ __global__ __launch_bounds__(64 * W) void k_euler_wide(const EulerArgs a,
         });
       }
     }
+    if constexpr (!kMat) turn = turn + 1 < W ? turn + 1 : 0;
     __syncthreads();
     if (s + 1 < a.nsteps) fetch(s + 1);
     const int row = store_row[s];
@@ -295,8 +363,8 @@ __global__ __launch_bounds__(64 * W) void k_euler_wide(const EulerArgs a,
         } else {
 #pragma unroll
           for (int r = 0; r < R; ++r) {
-            zx[r] = z[0][comp(r)][lane];
-            zy[r] = z[NB - 1][comp(r)][lane];
+            zx[r] = z[0][comp(r)][col(comp(r), pl)];
+            zy[r] = z[NB - 1][comp(r)][col(comp(r), pl)];
           }
         }
 #pragma unroll
@@ -331,7 +399,7 @@ __global__ __launch_bounds__(64 * W) void k_euler_wide(const EulerArgs a,
         }
       } else {
 #pragma unroll
-        for (int r = 0; r < R; ++r) dw[r] = z[0][comp(r)][lane] * sq;
+        for (int r = 0; r < R; ++r) dw[r] = z[0][comp(r)][col(comp(r), pl)] * sq;
       }
 #pragma unroll
       for (int r = 0; r < R; ++r) {
@@ -353,7 +421,7 @@ __global__ __launch_bounds__(64 * W) void k_euler_wide(const EulerArgs a,
           if (replay_j) {
             if (has(r)) inc = inc + ((const T*)a.replay_dj)[((int64_t)g + v) * P + gid];
           } else if (has(r)) {
-            const uint32_t word = words[v][lane];
+            const uint32_t word = words[v][pl];
             if (word >= zero_below) {
               const double* pq = pois + ((int64_t)s * m + v) * 2;
               double lamds = pq[0], p0 = pq[1];
@@ -366,9 +434,9 @@ __global__ __launch_bounds__(64 * W) void k_euler_wide(const EulerArgs a,
               if (nj > 0) {
                 const bool neg = ds < (T)0;
                 const T* pj = par_lds + 2;
-                const T p2 = a.jump_law == SDEGPU_JUMP_NORMAL ? (T)0 : pj[4 * m + v];
+                const T p2 = a.jump_law == SDEGPU_JUMP_NORMAL ? (T)0 : pj[4 * N + v];
                 const T acc = jump_total<T>(a.jump_law, nj, (uint32_t)(g + v), path_j, a.c2j,
-                                            a.ej, a.kj0, a.kj1, pj[2 * m + v], pj[3 * m + v],
+                                            a.ej, a.kj0, a.kj1, pj[2 * N + v], pj[3 * N + v],
                                             p2);
                 inc = inc + (neg ? -acc : acc);
                 cnt[r] += neg ? -nj : nj;
@@ -440,9 +508,17 @@ __global__ __launch_bounds__(kBlock) void k_wiener_fill_wide(
 struct WideShape {
   int waves, rows;
 };
+template <typename T>
 inline WideShape wide_shape(int model, int m) {
   const bool h = model == SDEGPU_MODEL_HESTON;
   const int n = h ? m / 2 : m;
+  if (kWideMat<T>) {
+    // 4 waves hold 4 components of 16 paths each per row, 8 waves twice that
+    const int rows = (n + 3) / 4, most = h ? 4 : 6;
+    if (rows > 16 || (h && rows > 8)) return WideShape{0, 0};
+    if (rows <= most) return WideShape{4, rows < (h ? 2 : 3) ? (h ? 2 : 3) : rows};
+    return WideShape{8, h ? (rows + 1) / 2 : rows <= 8 ? 4 : rows <= 12 ? 6 : 8};
+  }
   const WideShape all[2][7] = {{{2, 6}, {2, 8}, {3, 7}, {3, 8}, {4, 8}, {6, 8}, {8, 8}},
                                {{2, 3}, {2, 4}, {3, 4}, {4, 4}, {6, 4}, {8, 4}, {8, 4}}};
   for (const WideShape& s : all[h ? 1 : 0])
@@ -452,7 +528,7 @@ inline WideShape wide_shape(int model, int m) {
 
 // k_euler_wide and k_wiener_fill_wide instances (euler_wide_f32.hip,
 // euler_wide_f64.hip): the kernel for a model and a width of 9..64, or null.
-// Blocks of 64 * wide_shape(model, m).waves threads, one per 64 paths; gen: recorded
+// Blocks of 64 * wide_shape<T>(model, m).waves threads, one per 64 paths; gen: recorded
 // increments, per-path parameters or intensities.
 template <typename T>
 EulerKernel<T> euler_wide_kernel(int model, int m, bool gen);
@@ -473,9 +549,19 @@ WienerFillWide<double> wiener_fill_wide_kernel<double>(int m);
 
 template <int MODEL, typename T, bool GEN>
 EulerKernel<T> pick_wide(int m) {
-  const WideShape s = wide_shape(MODEL, m);
-  if constexpr (MODEL == SDEGPU_MODEL_HESTON) {
-    switch (s.waves * 16 + s.rows) {
+  const WideShape s = wide_shape<T>(MODEL, m);
+  const int key = s.waves * 16 + s.rows;
+  if constexpr (MODEL == SDEGPU_MODEL_HESTON && kWideMat<T>) {
+    switch (key) {
+      case 4 * 16 + 2: return k_euler_wide<MODEL, T, 4, 2, GEN>;
+      case 4 * 16 + 3: return k_euler_wide<MODEL, T, 4, 3, GEN>;
+      case 4 * 16 + 4: return k_euler_wide<MODEL, T, 4, 4, GEN>;
+      case 8 * 16 + 3: return k_euler_wide<MODEL, T, 8, 3, GEN>;
+      case 8 * 16 + 4: return k_euler_wide<MODEL, T, 8, 4, GEN>;
+      default: return nullptr;
+    }
+  } else if constexpr (MODEL == SDEGPU_MODEL_HESTON) {
+    switch (key) {
       case 2 * 16 + 3: return k_euler_wide<MODEL, T, 2, 3, GEN>;
       case 2 * 16 + 4: return k_euler_wide<MODEL, T, 2, 4, GEN>;
       case 3 * 16 + 4: return k_euler_wide<MODEL, T, 3, 4, GEN>;
@@ -484,8 +570,19 @@ EulerKernel<T> pick_wide(int m) {
       case 8 * 16 + 4: return k_euler_wide<MODEL, T, 8, 4, GEN>;
       default: return nullptr;
     }
+  } else if constexpr (kWideMat<T>) {
+    switch (key) {
+      case 4 * 16 + 3: return k_euler_wide<MODEL, T, 4, 3, GEN>;
+      case 4 * 16 + 4: return k_euler_wide<MODEL, T, 4, 4, GEN>;
+      case 4 * 16 + 5: return k_euler_wide<MODEL, T, 4, 5, GEN>;
+      case 4 * 16 + 6: return k_euler_wide<MODEL, T, 4, 6, GEN>;
+      case 8 * 16 + 4: return k_euler_wide<MODEL, T, 8, 4, GEN>;
+      case 8 * 16 + 6: return k_euler_wide<MODEL, T, 8, 6, GEN>;
+      case 8 * 16 + 8: return k_euler_wide<MODEL, T, 8, 8, GEN>;
+      default: return nullptr;
+    }
   } else {
-    switch (s.waves * 16 + s.rows) {
+    switch (key) {
       case 2 * 16 + 6: return k_euler_wide<MODEL, T, 2, 6, GEN>;
       case 2 * 16 + 8: return k_euler_wide<MODEL, T, 2, 8, GEN>;
       case 3 * 16 + 7: return k_euler_wide<MODEL, T, 3, 7, GEN>;

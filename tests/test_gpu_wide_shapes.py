@@ -41,3 +41,21 @@ def test_heston_widths(gpu, n):
                         **kw)
     for got, want in zip(p(tt), ref):
         assert np.max(np.abs(got / want - 1)) < 1e-12
+
+
+@pytest.mark.parametrize('P', [1, 15, 16, 17, 48, 63, 81])
+@pytest.mark.parametrize('m', [10, 20, 21, 40])
+def test_sixteen_path_groups(gpu, m, P):
+    # FP64 steps 16 paths in a wave: groups that are full, partial and without a path
+    n, tt = 3, np.linspace(0., 1., 4)
+    info, ref_info = {}, {}
+    jump = dict(lam=6., a=-.05, b=.1)
+    p = sa.merton_jumpdiff_process(paths=P, vshape=m, steps=n, corr=_corr(m), info=info, x0=1.,
+                                   mu=.03, sigma=.2, rng=np.random.default_rng(5), **jump)
+    src = {'dw': ora.PhiloxWiener(p.sources['dw'].key, 0, P, (m,), corr=_corr(m)),
+           'dj': ora.PhiloxCPoisson(p.sources['dj'].key, 0, P, (m,), **jump)}
+    got = p(tt)
+    ref = ora.integrate('jumpdiff', tt, paths=P, vshape=(m,), steps=n, sources=src,
+                        info=ref_info, x0=1., mu=.03, sigma=.2)
+    assert np.array_equal(info['jump_count'], ref_info['jump_count'])
+    assert np.max(np.abs(got / ref - 1)) < 1e-12
