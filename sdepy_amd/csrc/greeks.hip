@@ -617,7 +617,7 @@ __global__ __launch_bounds__(kBlock) void k_loglin_greeks(const LogArgs a,
     int nev = 0;
     for (int s0 = 0; s0 < n; s0 += 4) {
       T z[4];
-      normals4<T>((uint32_t)(s0 >> 2), path, kStreamNormal, a.ew, a.kw0, a.kw1, z);
+      normals4<T, false>((uint32_t)(s0 >> 2), path, kStreamNormal, a.ew, a.kw0, a.kw1, z);
       uint32_t up[4] = {0u, 0u, 0u, 0u};
       if (a.pois) {
         const ctr4 r = philox4x32_10(ctr4{(uint32_t)(s0 >> 2), path, kStreamPoisson, a.ej}, a.kj0, a.kj1);
