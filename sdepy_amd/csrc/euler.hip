@@ -248,12 +248,12 @@ extern "C" int sdegpu_euler(const sdegpu_euler_problem* pr, void* stream) {
   if (share > 1) {
     const dim3 sgrid(blocks_for(pr->paths, 64)), sblock(64 * share);
     if (pr->dtype == SDEGPU_F32) {
-      if (EulerKernel<float> k = euler_split_kernel<float>(pr->model, m, hd)) {
+      if (EulerKernel<float> k = euler_split_kernel<float>(pr->model, m, hd, sgrid.x)) {
         hipLaunchKernelGGL(k, sgrid, sblock, 0, st, a, (const float*)pr->coef, pr->store_row,
                            pr->pois, (float*)pr->out);
         return launch_status("k_euler_split");
       }
-    } else if (EulerKernel<double> k = euler_split_kernel<double>(pr->model, m, hd)) {
+    } else if (EulerKernel<double> k = euler_split_kernel<double>(pr->model, m, hd, sgrid.x)) {
       hipLaunchKernelGGL(k, sgrid, sblock, 0, st, a, (const double*)pr->coef, pr->store_row,
                          pr->pois, (double*)pr->out);
       return launch_status("k_euler_split");

@@ -24,13 +24,15 @@
 
 namespace sdegpu {
 
-constexpr int kSplitWaves = 8;  // most waves that share 64 paths
-
-// Units of CH steps (whole Philox blocks) per chunk: 8, so that 8 waves have
-// one each (4 for the 3-component states, whose unit is 4 steps of 3 blocks).
-template <int M>
+// Units of CH steps (whole Philox blocks) per chunk, MOST of them (4 for the
+// 3-component states, whose unit is 4 steps of 3 blocks): 8, so that 8 waves have
+// one each.  FP64 jumps take 52 KB of LDS so, three blocks per CU: grids of
+// more than three, whose blocks have 4 waves at most, run with 4 units and 28 KB.  FP64, 250
+// steps, 251 rows: Kou of 60,000 paths 159 -> 142 us, two Mertons 310 -> 278; of
+// 40,000 paths (2.4 blocks per CU) 114 with 8 units, 121 with 4.
+template <int M, int MOST>
 struct SplitChunk {
-  static constexpr int U = Chunking<M>::NZ > 4 ? 4 : 8;
+  static constexpr int U = Chunking<M>::NZ > 4 ? 4 : MOST;
   static constexpr int L = U * Chunking<M>::CH;
 };
 
@@ -39,12 +41,12 @@ struct Count {
   static constexpr int value = K;
 };
 
-template <int MODEL, typename T, int M, int D>
-__global__ __launch_bounds__(64 * kSplitWaves) void k_euler_split(
+template <int MODEL, typename T, int M, int D, int MOST = 8>
+__global__ __launch_bounds__(64 * MOST) void k_euler_split(
     const EulerArgs a, const T* __restrict__ coef, const int32_t* __restrict__ store_row,
     const double* __restrict__ pois, T* __restrict__ out) {
   constexpr int CH = Chunking<M>::CH, NZ = Chunking<M>::NZ;
-  constexpr int U = SplitChunk<M>::U, L = SplitChunk<M>::L;
+  constexpr int U = SplitChunk<M, MOST>::U, L = SplitChunk<M, MOST>::L;
   constexpr bool kJump = MODEL == SDEGPU_MODEL_JUMPDIFF;
   constexpr bool kHeston = MODEL == SDEGPU_MODEL_HESTON;
   constexpr bool kOU = MODEL == SDEGPU_MODEL_OU;
@@ -273,34 +275,41 @@ __global__ __launch_bounds__(64 * kSplitWaves) void k_euler_split(
 }
 
 template <typename T>
-EulerKernel<T> euler_split_kernel(int model, int m, int d);
+EulerKernel<T> euler_split_kernel(int model, int m, int d, int64_t blocks);
 template <>
-EulerKernel<float> euler_split_kernel<float>(int model, int m, int d);
+EulerKernel<float> euler_split_kernel<float>(int model, int m, int d, int64_t blocks);
 template <>
-EulerKernel<double> euler_split_kernel<double>(int model, int m, int d);
+EulerKernel<double> euler_split_kernel<double>(int model, int m, int d, int64_t blocks);
 
-template <int MODEL, typename T, int MAX>
+template <int MODEL, typename T, int MAX, int MOST = 8>
 EulerKernel<T> pick_split(int m) {
-  if (m == 1) return k_euler_split<MODEL, T, 1, 1>;
-  if (m == 2) return k_euler_split<MODEL, T, 2, 1>;
+  if (m == 1) return k_euler_split<MODEL, T, 1, 1, MOST>;
+  if (m == 2) return k_euler_split<MODEL, T, 2, 1, MOST>;
   if constexpr (MAX > 2) {
-    if (m == 3) return k_euler_split<MODEL, T, 3, 1>;
-    if (m == 4) return k_euler_split<MODEL, T, 4, 1>;
+    if (m == 3) return k_euler_split<MODEL, T, 3, 1, MOST>;
+    if (m == 4) return k_euler_split<MODEL, T, 4, 1, MOST>;
   }
   return nullptr;
 }
 
-// The kernel for a model, its components m and Heston's group width d, or
-// null (euler_split_f32.hip, euler_split_f64.hip).
+template <typename T>
+EulerKernel<T> pick_split_jump(int m, int64_t blocks) {
+  // (split_waves gives such grids 4 waves a block at most)
+  if (sizeof(T) == 8 && blocks > 3 * 256) return pick_split<SDEGPU_MODEL_JUMPDIFF, T, 2, 4>(m);
+  return pick_split<SDEGPU_MODEL_JUMPDIFF, T, 2>(m);
+}
+
+// The kernel for a model, its components m, Heston's group width d and the
+// blocks of the grid, or null (euler_split_f32.hip, euler_split_f64.hip).
 #define SDEGPU_EULER_SPLIT_SET(T)                                                       \
   template <>                                                                           \
-  EulerKernel<T> euler_split_kernel<T>(int model, int m, int d) {                       \
+  EulerKernel<T> euler_split_kernel<T>(int model, int m, int d, int64_t blocks) {       \
     switch (model) {                                                                    \
       case SDEGPU_MODEL_WIENER: return pick_split<SDEGPU_MODEL_WIENER, T, 4>(m);        \
       case SDEGPU_MODEL_LOGNORM: return pick_split<SDEGPU_MODEL_LOGNORM, T, 4>(m);      \
       case SDEGPU_MODEL_OU: return pick_split<SDEGPU_MODEL_OU, T, 4>(m);                \
       case SDEGPU_MODEL_CIR: return pick_split<SDEGPU_MODEL_CIR, T, 4>(m);              \
-      case SDEGPU_MODEL_JUMPDIFF: return pick_split<SDEGPU_MODEL_JUMPDIFF, T, 2>(m);    \
+      case SDEGPU_MODEL_JUMPDIFF: return pick_split_jump<T>(m, blocks);                 \
       case SDEGPU_MODEL_HESTON:                                                         \
         if (m == 2) return k_euler_split<SDEGPU_MODEL_HESTON, T, 2, 1>;                 \
         if (m == 4 && d == 1) return k_euler_split<SDEGPU_MODEL_HESTON, T, 4, 1>;       \
