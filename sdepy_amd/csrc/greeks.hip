@@ -20,6 +20,8 @@
 // the order of the FP32 operations shows: where the variance reaches 0, single
 // paths dominate the sums of 1 / sqrt(v), and the segment form moves the
 // variance's Greeks of 4M paths by 6e-7.
+#include <type_traits>
+
 #include "common.hpp"
 #include "philox.hpp"
 
@@ -533,19 +535,22 @@ __global__ __launch_bounds__(kBlock, (heston_waves<T, TV>())) void k_heston_tang
 
   if (live) {
     HestonPath<T, TV> p = heston_start<T, TV>(a);
-    for (int s0 = 0; s0 < n; s0 += 2) {
+    auto pair = [&](int s0, int most) {
       T z[4];
       normals4_folded<T>((uint32_t)(s0 >> 1), path, kStreamNormal, a.epoch, a.k0, a.k1, z);
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
-        if (s0 + j < n) {
+        if (j < most) {
           const int64_t row = (int64_t)(s0 + j) * kHestonTab;
           const HestonPartials<TV> d = heston_step<false, T, TV>(p, tb + row, tv + row, z[2 * j],
                                                           z[2 * j + 1], rho, rhoc, rho_r);
           heston_tangent_step(p, d, tv[row]);
         }
       }
-    }
+    };
+    int s0 = 0;
+    for (; s0 + 2 <= n; s0 += 2) pair(s0, 2);
+    if (s0 < n) pair(s0, 1);
     heston_greeks_of(a, p, *sum_ds, acc);
   }
   block_reduce_store<kHestonNS>(acc, a.part);
@@ -615,7 +620,8 @@ __global__ __launch_bounds__(kBlock) void k_loglin_greeks(const LogArgs a,
     // at a lane-computed address, not a select into each register
     __shared__ uint32_t ev[kLogEvents][kBlock];
     int nev = 0;
-    for (int s0 = 0; s0 < n; s0 += 4) {
+    // four steps; groups that are whole run without a test for the last step
+    auto group = [&](int s0, auto whole) {
       T z[4];
       normals4<T, false>((uint32_t)(s0 >> 2), path, kStreamNormal, a.ew, a.kw0, a.kw1, z);
       uint32_t up[4] = {0u, 0u, 0u, 0u};
@@ -629,7 +635,7 @@ __global__ __launch_bounds__(kBlock) void k_loglin_greeks(const LogArgs a,
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const int s = s0 + j;
-        if (s < n) {
+        if (decltype(whole)::value || s < n) {
           const T dw = z[j] * st[2 * s + 1];
           // a word below the step's bound (the low word of pois[s][2]) is a
           // count of 0: one integer compare in place of forming the FP64
@@ -653,7 +659,10 @@ __global__ __launch_bounds__(kBlock) void k_loglin_greeks(const LogArgs a,
           sdw = sdw + dw;
         }
       }
-    }
+    };
+    int s0 = 0;
+    for (; s0 + 4 <= n; s0 += 4) group(s0, std::true_type{});
+    if (s0 < n) group(s0, std::false_type{});
 #pragma unroll
     for (int k = 0; k < kLogEvents; ++k) {
       if (k < nev) {
