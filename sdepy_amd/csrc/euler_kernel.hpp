@@ -597,6 +597,17 @@ __global__ __launch_bounds__(kBlock, MOM ? 8 : 1) void k_euler(const EulerArgs a
   for (int v = 0; v < M; ++v) cnt[v] = 0;
   int interval_jumps = 0;
 
+  // the count of component v at step s from its Poisson word
+  auto jump_count = [&](int s, int v, uint32_t word) {
+    const double* pq = pois + ((int64_t)s * M + v) * 2;
+    double lamds = pq[0], p0 = pq[1];
+    if (GEN && a.lamp) {
+      // per-path intensity: pois holds |ds|
+      lamds = a.lamp[(int64_t)s * a.lamp_step + (c0 + v) * P + gid] * lamds;
+      p0 = exp(-lamds);
+    }
+    return poisson_inv(u01_f64(word), lamds, p0, kPoissonCap);
+  };
   // jumpdiff with DEFER: x moves by (drift + diffusion) + dj with
   // state-independent coefficients, so the jump sizes of a step only have to
   // be in x when x is next stored.  On steps that are not stored, up to kJumpEvents jump draws
@@ -609,7 +620,15 @@ __global__ __launch_bounds__(kBlock, MOM ? 8 : 1) void k_euler(const EulerArgs a
   // the same terms, rounded in another order.  The host asks for it when
   // stored steps are sparse; with a store at most steps the bookkeeping
   // costs more than it saves.
+  // Late (without row moments, whose LDS is full): an event records its word in
+  // place of the count, which is inverted with the sizes, as long as the
+  // pass's bound says that no count comes near 256 (1 or more means
+  // intensities below 22.2 per step).  Merton 2M x 252 FP32, 5 rows 580 -> 533 us;
+  // FP64 1M x 60, 2 rows 245 -> 212 (two of them 556 -> 571: not so in FP64).
   constexpr int kJumpEvents = 4;
+  constexpr bool kLate = kDefer && !MOM && (M == 1 || sizeof(T) == 4);
+  const bool late = kLate && zero_below > 0u;
+  __shared__ uint32_t jword[kLate ? kJumpEvents : 1][kLate ? kBlock : 1];
   // one LDS column per lane: recording an event is a store at a lane-computed
   // address, not a select into each of 4 registers
   __shared__ uint32_t jev[kDefer ? kJumpEvents : 1][kDefer ? kBlock : 1];
@@ -625,10 +644,20 @@ __global__ __launch_bounds__(kBlock, MOM ? 8 : 1) void k_euler(const EulerArgs a
   auto flush_jumps = [&]() {
     for (int q = 0; q < njev; ++q) {
       const uint32_t e = jev[q][threadIdx.x];
-      const int s = (int)(e >> 12), v = (int)((e >> 8) & 7u), n = (int)(e & 255u);
+      const int s = (int)(e >> 12), v = (int)((e >> 8) & 7u);
+      const bool neg = ((e >> 11) & 1u) != 0u;
+      int n = (int)(e & 255u);
+      if constexpr (kLate) {
+        if (late) {
+          n = jump_count(s, v, jword[q][threadIdx.x]);
+#pragma unroll
+          for (int w = 0; w < M; ++w) cnt[w] += w == v ? (neg ? -n : n) : 0;
+          interval_jumps += neg ? -n : n;
+        }
+      }
       const T* pr = coef + (int64_t)s * a.ncoef + a.poff;
       T acc = jump_sum(s, v, n, pr);
-      acc = (e >> 11) & 1u ? -acc : acc;
+      acc = neg ? -acc : acc;
 #pragma unroll
       for (int w = 0; w < M; ++w) x[w] = x[w] + (w == v ? acc : (T)0);
     }
@@ -821,7 +850,6 @@ __global__ __launch_bounds__(kBlock, MOM ? 8 : 1) void k_euler(const EulerArgs a
 #pragma unroll
           for (int v = 0; v < M; ++v) inc[v] = inc[v] + rp[v * P];
         } else {
-          const double* pq = pois + (int64_t)s * M * 2;
           const bool neg = ds < (T)0;
           // a stored step takes its own jumps in place (its state is written
           // now); the steps in between defer theirs
@@ -829,15 +857,18 @@ __global__ __launch_bounds__(kBlock, MOM ? 8 : 1) void k_euler(const EulerArgs a
 #pragma unroll
           for (int v = 0; v < M; ++v) {
             if (upois[k * M + v] < zero_below) continue;
-            double lamds = pq[2 * v], p0 = pq[2 * v + 1];
-            if (GEN && a.lamp) {
-              // per-path intensity: pois holds |ds|
-              lamds = a.lamp[(int64_t)s * a.lamp_step + (c0 + v) * P + gid] * lamds;
-              p0 = exp(-lamds);
+            if constexpr (kLate) {
+              if (late && !stored && njev < kJumpEvents && s < (1 << 20)) {
+                jev[njev][threadIdx.x] =
+                    ((uint32_t)s << 12) | ((neg ? 1u : 0u) << 11) | ((uint32_t)v << 8);
+                jword[njev][threadIdx.x] = upois[k * M + v];
+                ++njev;
+                continue;
+              }
             }
-            const int n = poisson_inv(u01_f64(upois[k * M + v]), lamds, p0, kPoissonCap);
+            const int n = jump_count(s, v, upois[k * M + v]);
             if (n > 0) {
-              if (kDefer && !stored && njev < kJumpEvents && n < 256 && s < (1 << 20)) {
+              if (kDefer && !late && !stored && njev < kJumpEvents && n < 256 && s < (1 << 20)) {
                 jev[njev][threadIdx.x] = ((uint32_t)s << 12) | ((neg ? 1u : 0u) << 11) |
                                          ((uint32_t)v << 8) | (uint32_t)n;
                 ++njev;
@@ -868,6 +899,9 @@ __global__ __launch_bounds__(kBlock, MOM ? 8 : 1) void k_euler(const EulerArgs a
 
   if constexpr (MOM) {
     if (mk > 0) flush_row_moments<T>(a, moment_columns<T>(), mres, mrows, mk * a.nout, mphase);
+  }
+  if constexpr (kLate) {
+    if (late) flush_jumps();  // the counts after the last row
   }
   if (a.info_paths && (kHeston || kJump) && live) {
     // Heston counts per log-x value (the group's first is comp0 / 2), jump

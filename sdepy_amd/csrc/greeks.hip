@@ -612,14 +612,22 @@ __global__ __launch_bounds__(kBlock) void k_loglin_greeks(const LogArgs a,
     // The log-space recursion is linear with state-independent
     // coefficients and only x_T is needed, so the jump sizes can be added
     // after the step loop: up to kLogEvents jump steps per path are recorded
-    // as (s << 8 | count) and drawn afterwards, when every lane of the wave
-    // draws its own (at lambda ds = 1/252 a wave otherwise draws a Philox
-    // block at about one step in five for a single jumping lane).  Further
-    // jump steps, counts above 255 and steps beyond 2^24 are drawn in place.
+    // and drawn afterwards, when every lane of the wave draws its own (at lambda
+    // ds = 1/252 a wave otherwise draws a Philox block at about one step in five
+    // for a single jumping lane).  Further jump steps, counts above 255 and
+    // steps beyond 2^24 are drawn in place.  An event is (s << 8 | count); in FP32
+    // the step and its Poisson word, which is inverted afterwards too (2M x
+    // 252 514 -> 489 us; FP64 was 3% slower so): a bound of 1 or more means
+    // a lambda ds below 22.2, whose counts never come near 256.
     // the events live in LDS, one column per lane: recording one is a store
     // at a lane-computed address, not a select into each register
-    __shared__ uint32_t ev[kLogEvents][kBlock];
+    constexpr bool kLate = sizeof(T) == 4;
+    using Event = std::conditional_t<kLate, uint2, uint32_t>;
+    __shared__ Event ev[kLogEvents][kBlock];
     int nev = 0;
+    auto count = [&](int s, uint32_t word) {
+      return poisson_inv(u01_f64(word), pois[3 * s], pois[3 * s + 1], 4096);
+    };
     // four steps; groups that are whole run without a test for the last step
     auto group = [&](int s0, auto whole) {
       T z[4];
@@ -642,13 +650,27 @@ __global__ __launch_bounds__(kBlock) void k_loglin_greeks(const LogArgs a,
           // uniform; words at or above it take the inversion, which
           // re-checks against exp(-lam ds)
           if (a.pois && up[j] >= reinterpret_cast<const uint32_t*>(pois)[6 * s + 4]) {
-            const int cnt = poisson_inv(u01_f64(up[j]), pois[3 * s], pois[3 * s + 1], 4096);
+            bool kept = false;
+            if constexpr (kLate) {
+              if (reinterpret_cast<const uint32_t*>(pois)[6 * s + 4] > 0u && nev < kLogEvents &&
+                  s < (1 << 24)) {
+                ev[nev][threadIdx.x] = make_uint2((uint32_t)s, up[j]);
+                ++nev;
+                kept = true;
+              }
+            }
+            const int cnt = kept ? 0 : count(s, up[j]);
             if (cnt > 0) {
-              njump += cnt;
               if (nev < kLogEvents && cnt < 256 && s < (1 << 24)) {
-                ev[nev][threadIdx.x] = ((uint32_t)s << 8) | (uint32_t)cnt;
+                if constexpr (kLate) {
+                  ev[nev][threadIdx.x] = make_uint2((uint32_t)s, up[j]);
+                } else {
+                  njump += cnt;
+                  ev[nev][threadIdx.x] = ((uint32_t)s << 8) | (uint32_t)cnt;
+                }
                 ++nev;
               } else {
+                njump += cnt;
                 T dj = (T)0, zsum = (T)0;
                 jumps(s, cnt, dj, zsum);
                 sj = sj + dj;
@@ -667,8 +689,14 @@ __global__ __launch_bounds__(kBlock) void k_loglin_greeks(const LogArgs a,
     for (int k = 0; k < kLogEvents; ++k) {
       if (k < nev) {
         T dj = (T)0, zsum = (T)0;
-        const uint32_t e = ev[k][threadIdx.x];
-        jumps((int)(e >> 8), (int)(e & 255u), dj, zsum);
+        const Event e = ev[k][threadIdx.x];
+        if constexpr (kLate) {
+          const int cnt = count((int)e.x, e.y);
+          njump += cnt;
+          jumps((int)e.x, cnt, dj, zsum);
+        } else {
+          jumps((int)(e >> 8), (int)(e & 255u), dj, zsum);
+        }
         sj = sj + dj;
         szeta = szeta + zsum;
       }
