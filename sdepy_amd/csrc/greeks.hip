@@ -723,25 +723,49 @@ __global__ __launch_bounds__(kBlock) void k_loglin_greeks(const LogArgs a,
   block_reduce_store<kLogNS>(acc, a.part);
 }
 
-// out[c] = sum_r part[r][c]: one block per column, fixed-order tree, so the
-// result does not depend on scheduling.  A latency chain: 16 blocks read the
-// 2 MB that 4M paths leave, so each of the 1024 threads keeps 16 loads in flight (256
-// threads with one load at a time took 30 us).
+// The columns' sums of part[rows][ncol], in a fixed order that does not depend on
+// scheduling.  Above kSumRows rows the rows are first summed in place, slice by
+// slice: a block per slice reads its rows in whole lines and leaves their sum in
+// the first.  One block per column reads 8 bytes of every line of all rows, 27
+// us for the 15,625 rows of 4M paths, however many loads are in flight; the
+// two kernels take 15.  For the 7,813 rows of 2M paths it is 12 and 10, for 1,172 the second
+// launch costs 2 more than it saves.
+constexpr int kSumRows = 4096, kSumSlices = 64;
+
+__global__ __launch_bounds__(kBlock) void k_sum_slices(double* __restrict__ part, int64_t rows,
+                                                       int ncol, int64_t per) {
+  __shared__ double sh[kBlock];
+  const int64_t lo = blockIdx.x * per, hi = lo + per < rows ? lo + per : rows;
+  const int deep = kBlock / ncol;  // rows read at a time
+  const int t = threadIdx.x, c = t % ncol, r = t / ncol;
+  double v = 0.0;
+  if (r < deep)
+    for (int64_t i = lo + r; i < hi; i += deep) v += part[i * ncol + c];
+  sh[t] = v;
+  __syncthreads();
+  if (t < ncol) {
+    double s = 0.0;
+    for (int k = 0; k < deep; ++k) s += sh[k * ncol + t];
+    part[lo * ncol + t] = s;
+  }
+}
+
+// out[c]: the sum of part[r step][c], r < rows, one block per column; each thread
+// keeps 4 loads in flight
 constexpr int kSumThreads = 1024;
 
 __global__ __launch_bounds__(kSumThreads) void k_sum_columns(const double* __restrict__ part,
-                                                             int64_t rows, int ncol,
+                                                             int64_t rows, int64_t step, int ncol,
                                                              double* __restrict__ out) {
-  constexpr int kAhead = 16;
+  constexpr int kAhead = kSumRows / kSumThreads;
   __shared__ double sh[kSumThreads / 64];
-  const int c = blockIdx.x;
   double v = 0.0;
   for (int64_t r0 = threadIdx.x; r0 < rows; r0 += kAhead * kSumThreads) {
     double q[kAhead];
 #pragma unroll
     for (int i = 0; i < kAhead; ++i) {
       const int64_t r = r0 + i * kSumThreads;
-      q[i] = r < rows ? part[r * ncol + c] : 0.0;
+      q[i] = r < rows ? part[r * step * ncol + blockIdx.x] : 0.0;
     }
 #pragma unroll
     for (int i = 0; i < kAhead; ++i) v += q[i];
@@ -754,8 +778,23 @@ __global__ __launch_bounds__(kSumThreads) void k_sum_columns(const double* __res
     double s = 0.0;
 #pragma unroll
     for (int w = 0; w < kSumThreads / 64; ++w) s += sh[w];
-    out[c] = s;
+    out[blockIdx.x] = s;
   }
+}
+
+static int sum_columns(double* part, int64_t rows, int ncol, double* out, hipStream_t st) {
+  int64_t step = 1;
+  if (rows > kSumRows) {
+    step = (rows + kSumSlices - 1) / kSumSlices;
+    const int64_t slices = (rows + step - 1) / step;
+    hipLaunchKernelGGL(k_sum_slices, dim3((unsigned)slices), dim3(kBlock), 0, st, part, rows, ncol,
+                       step);
+    if (int e = launch_status("k_sum_slices")) return e;
+    rows = slices;
+  }
+  hipLaunchKernelGGL(k_sum_columns, dim3(ncol), dim3(kSumThreads), 0, st, (const double*)part, rows, step,
+                     ncol, out);
+  return launch_status("k_sum_columns");
 }
 
 // Workspace of one Heston Greeks launch, in this order (each part 256-byte
@@ -885,9 +924,7 @@ extern "C" int sdegpu_heston_greeks_run(const sdegpu_heston_greeks* g, double* o
                          (const double*)sum_ds);
   }
   if (int e = launch_status(g->method == 1 ? "k_heston_tangent" : "k_heston_adjoint")) return e;
-  hipLaunchKernelGGL(k_sum_columns, dim3(kHestonNS), dim3(kSumThreads), 0, st, (const double*)a.part,
-                     (int64_t)nb, kHestonNS, out);
-  return launch_status("k_sum_columns");
+  return sum_columns(a.part, (int64_t)nb, kHestonNS, out, st);
 }
 
 extern "C" size_t sdegpu_loglin_greeks_workspace(int64_t paths) {
@@ -940,7 +977,5 @@ extern "C" int sdegpu_loglin_greeks_run(const sdegpu_loglin_greeks* g, double* o
     hipLaunchKernelGGL(k_loglin_greeks<double>, dim3(nb), dim3(kBlock), 0, st, a,
                        (const double*)a.steps, a.pois);
   if (int e = launch_status("k_loglin_greeks")) return e;
-  hipLaunchKernelGGL(k_sum_columns, dim3(kLogNS), dim3(kSumThreads), 0, st, (const double*)a.part,
-                     (int64_t)nb, kLogNS, out);
-  return launch_status("k_sum_columns");
+  return sum_columns(a.part, (int64_t)nb, kLogNS, out, st);
 }
