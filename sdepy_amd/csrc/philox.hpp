@@ -71,7 +71,8 @@ __host__ __device__ __forceinline__ ctr4 philox_round(ctr4 c, uint32_t k0, uint3
 // key first, on the scalar unit, they save a move each, 3 of some 53
 // instructions of four FP32 normals: batched run of 256 2190 -> 2136 us,
 // Heston 4M x 365 1596 -> 1561.  Kernels that draw FP64 normals or Poisson words are
-// 1% slower so.
+// 1% slower so, and those of k_euler that read their rows as scalars 1 to 2%
+// (lognormal 1M x 200 147 against 143.5).
 template <bool KEY1ST>
 __device__ __forceinline__ ctr4 philox_round_v(ctr4 c, uint32_t k0, uint32_t k1, int round) {
   const uint64_t p0 = (uint64_t)kPhiloxM0 * c.x;
