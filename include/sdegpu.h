@@ -430,7 +430,9 @@ int sdegpu_cpoisson_fill_paths(int32_t dtype, const uint32_t key[2], uint32_t ep
  *
  * Heston (NG = 7): d/d(x0, r, k, theta, xi, rho, y0); r is both the drift mu
  * of log x and the discount rate.  The workspace holds the expanded step
- * table and block partials.
+ * table, block partials and, for SDEGPU_F32 without variance_f64, variance
+ * checkpoints of method 0: ceil(nsteps/8) floats per path.  Its size does not
+ * depend on method, so that one workspace serves both.
  * steps: device [nsteps][2] = (ds, sqrt(ds)) in dtype.  Scalar rho builds
  * corr = [[1, rho], [rho, 1]] as sdepy does (infrastructure.py:128-150).
  */

@@ -829,7 +829,8 @@ using namespace sdegpu;
 
 extern "C" size_t sdegpu_heston_greeks_workspace(const sdegpu_heston_greeks* g) {
   if (!g || g->paths < 1) return 0;
-  return heston_ws(g->dtype, g->variance_f64 != 0, g->method, g->paths, g->nsteps).total;
+  // (method 0's, which is the larger: one workspace serves both methods)
+  return heston_ws(g->dtype, g->variance_f64 != 0, 0, g->paths, g->nsteps).total;
 }
 
 extern "C" int sdegpu_heston_greeks_run(const sdegpu_heston_greeks* g, double* out, void* ws,
@@ -851,12 +852,12 @@ extern "C" int sdegpu_heston_greeks_run(const sdegpu_heston_greeks* g, double* o
     return fail(SDEGPU_EINVAL, "heston_greeks: variance_f64 %d", g->variance_f64);
   // an FP64 variance state with FP32 normals (FP64 runs carry it anyway)
   const bool v64 = g->variance_f64 != 0 && g->dtype == SDEGPU_F32;
-  const size_t need = sdegpu_heston_greeks_workspace(g);
-  if (!ws || ws_bytes < need)
-    return fail(SDEGPU_ENOMEM, "heston_greeks: workspace of %zu bytes, %zu needed", ws_bytes, need);
+  const HestonWs lay = heston_ws(g->dtype, v64, g->method, g->paths, g->nsteps);
+  if (!ws || ws_bytes < lay.total)
+    return fail(SDEGPU_ENOMEM, "heston_greeks: workspace of %zu bytes, %zu needed", ws_bytes,
+                lay.total);
   HestonArgs a = {};
   a.steps = g->steps;
-  const HestonWs lay = heston_ws(g->dtype, v64, g->method, g->paths, g->nsteps);
   char* base = (char*)ws;
   a.ckpt = base + lay.ckpt;
   a.part = (double*)(base + lay.part);

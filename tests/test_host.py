@@ -505,3 +505,19 @@ def test_montecarlo_pdf_and_cdf_from_a_histogram():
     mid = (bins[:-1] + bins[1:]) / 2
     assert np.allclose(M._histogram_interp(mid, density, bins, 'linear', False), density)
     assert M._histogram_interp(np.array([-5., 5.]), density, bins, 'linear', False).tolist() == [0., 0.]
+
+
+@pytest.mark.parametrize('dtype,v64', [(_lib.F32, 0), (_lib.F32, 1), (_lib.F64, 0)])
+def test_heston_greeks_workspace_serves_both_methods(dtype, v64):
+    """A workspace sized for one method is large enough for the other, and an
+    FP32 one has room for method 0's checkpoints (every 8 steps)."""
+    lib = G._bind()
+    pr = G.HestonGreeksProblem()
+    pr.dtype, pr.variance_f64, pr.paths, pr.nsteps = dtype, v64, 1000, 365
+    sizes = []
+    for method in (0, 1):
+        pr.method = method
+        sizes.append(lib.sdegpu_heston_greeks_workspace(pr))
+    assert sizes[0] == sizes[1]
+    if dtype == _lib.F32 and not v64:
+        assert sizes[0] > 46 * 1000 * 4
