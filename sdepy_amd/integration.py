@@ -354,7 +354,7 @@ class _gpu_sde:
         z = self._args[name]
         n = math.prod(shape)
         if not callable(z) and np.ndim(z) == 0:
-            return np.full((len(t0s), n), float(z))
+            return np.full((len(t0s), n), np.asarray(z, dtype=float))
         if callable(z):
             return np.stack([per_component(z(t), shape, name) for t in t0s]) \
                 if len(t0s) else np.zeros((0, n))

@@ -521,3 +521,20 @@ def test_heston_greeks_workspace_serves_both_methods(dtype, v64):
     assert sizes[0] == sizes[1]
     if dtype == _lib.F32 and not v64:
         assert sizes[0] > 46 * 1000 * 4
+
+
+@pytest.mark.parametrize('value,want', [
+    (None, np.nan), (np.array(None), np.nan), ('0.25', .25), (True, 1.),
+    (np.float32(.25), .25), (np.array(.25), .25), (np.ma.masked, 0.),
+    (np.datetime64(3, 'D'), 3.)])
+def test_scalar_parameters_convert_as_arrays_do(value, want):
+    """Whatever NumPy converts to one double is a scalar parameter (None is NaN),
+    as it is inside an array."""
+    t0s = np.array([0., .5])
+    p = sa.lognorm_process(paths=4, mu=value, steps=4)
+    assert p._path_params(t0s) is None
+    got = p._eval('mu', t0s, (1,))
+    assert got.dtype == np.float64 and got.shape == (2, 1)
+    assert np.array_equal(got, np.full((2, 1), want), equal_nan=True)
+    with pytest.raises(TypeError):
+        sa.lognorm_process(paths=4, mu=1j, steps=4)._eval('mu', t0s, (1,))
