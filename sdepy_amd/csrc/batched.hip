@@ -147,7 +147,7 @@ __device__ __forceinline__ float run_tile(const sdegpu_batch_instance& d, const 
     const uint32_t b0 = (uint32_t)(((int64_t)s0 * M) >> 2);
 #pragma unroll
     for (int j = 0; j < NZ / 4; ++j)
-      normals4<float>(b0 + j, path, kStreamNormal, d.epoch, d.key[0], d.key[1], z + 4 * j);
+      normals4<float, true>(b0 + j, path, kStreamNormal, d.epoch, d.key[0], d.key[1], z + 4 * j);
   };
   for (int c0 = 0; c0 < n; c0 += kRowSteps) {
     if constexpr (kRows) fill(c0);

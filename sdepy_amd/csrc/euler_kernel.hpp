@@ -710,8 +710,8 @@ __global__ __launch_bounds__(kBlock, MOM ? 8 : 1) void k_euler(const EulerArgs a
         const uint32_t b0 = (uint32_t)(((int64_t)s0 * M) >> 2);
 #pragma unroll
         for (int j = 0; j < NZ / 4; ++j)
-          normals4<T, sizeof(T) == 4 && kHeston>(b0 + j, path_w, a.c2w, a.ew, a.kw0, a.kw1,
-                                                z + 4 * j);
+          normals4<T, sizeof(T) == 4 && kHeston && kRow>(b0 + j, path_w, a.c2w, a.ew, a.kw0,
+                                                        a.kw1, z + 4 * j);
       }
       if (flip_w) {
 #pragma unroll

@@ -302,7 +302,7 @@ struct HestonRev {
 // variances and normals from its checkpoint and the Philox counters into
 // registers, then walk its steps backwards.  FULL segments hold C steps.
 // rho, rhoc and rho_r as in heston_step.
-template <int C, bool FULL>
+template <int C, bool FULL, bool KEY1ST>
 __device__ __forceinline__ void heston_segment(const HestonArgs& a, const float* __restrict__ tb,
                                                const float* __restrict__ ck, int64_t gid,
                                                uint32_t path, int c, int n, float rho, float rhoc,
@@ -315,8 +315,8 @@ __device__ __forceinline__ void heston_segment(const HestonArgs& a, const float*
     if (FULL || s0 + j < n) {
       __asm__ volatile("" ::: "memory");
       float z[4];
-      normals4_folded<float>((uint32_t)((s0 + j) >> 1), path, kStreamNormal, a.epoch, a.k0, a.k1,
-                             z);
+      normals4_folded<float, KEY1ST>((uint32_t)((s0 + j) >> 1), path, kStreamNormal, a.epoch,
+                                     a.k0, a.k1, z);
 #pragma unroll
       for (int q = 0; q < 2; ++q) {
         const int s = s0 + j + q;
@@ -361,7 +361,7 @@ __device__ __forceinline__ void heston_segment(const HestonArgs& a, const float*
 // adjoint of V carries U = Vbar / Xbar; k and theta need the sums of U ds and
 // U y+ ds, xi and rho those of U sv sq w and U sv sq (z0 - rho w): the
 // derivatives of X_T along the same directions.
-template <int C>
+template <int C, bool KEY1ST>
 __global__ __launch_bounds__(kBlock, (heston_waves<float, float>())) void k_heston_adjoint(
     const HestonArgs a, const float* __restrict__ tb, float* __restrict__ ck,
     const double* __restrict__ sum_ds) {
@@ -383,7 +383,8 @@ __global__ __launch_bounds__(kBlock, (heston_waves<float, float>())) void k_hest
     // ---- pass 1: forward, variance checkpoints every C steps ----
     for (int s0 = 0; s0 < n; s0 += 2) {
       float z[4];
-      normals4_folded<float>((uint32_t)(s0 >> 1), path, kStreamNormal, a.epoch, a.k0, a.k1, z);
+      normals4_folded<float, KEY1ST>((uint32_t)(s0 >> 1), path, kStreamNormal, a.epoch, a.k0,
+                                     a.k1, z);
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
         const int s = s0 + j;
@@ -405,9 +406,9 @@ __global__ __launch_bounds__(kBlock, (heston_waves<float, float>())) void k_hest
     HestonRev rv{0.f, 0.f, 0.f, 0.f, 0.f};
     const int nfull = n / C;
     if (nfull * C < n)
-      heston_segment<C, false>(a, tb, ck, gid, path, nfull, n, rho, rhoc, rho_r, rv);
+      heston_segment<C, false, KEY1ST>(a, tb, ck, gid, path, nfull, n, rho, rhoc, rho_r, rv);
     for (int c = nfull - 1; c >= 0; --c)
-      heston_segment<C, true>(a, tb, ck, gid, path, c, n, rho, rhoc, rho_r, rv);
+      heston_segment<C, true, KEY1ST>(a, tb, ck, gid, path, c, n, rho, rhoc, rho_r, rv);
     p.x1 = rv.s1;
     p.x2 = rv.s2;
     p.xx = rv.sx;
@@ -631,7 +632,7 @@ __global__ __launch_bounds__(kBlock) void k_loglin_greeks(const LogArgs a,
     // four steps; groups that are whole run without a test for the last step
     auto group = [&](int s0, auto whole) {
       T z[4];
-      normals4<T, false>((uint32_t)(s0 >> 2), path, kStreamNormal, a.ew, a.kw0, a.kw1, z);
+      normals4<T>((uint32_t)(s0 >> 2), path, kStreamNormal, a.ew, a.kw0, a.kw1, z);
       uint32_t up[4] = {0u, 0u, 0u, 0u};
       if (a.pois) {
         const ctr4 r = philox4x32_10(ctr4{(uint32_t)(s0 >> 2), path, kStreamPoisson, a.ej}, a.kj0, a.kj1);
@@ -907,8 +908,12 @@ extern "C" int sdegpu_heston_greeks_run(const sdegpu_heston_greeks* g, double* o
       hipLaunchKernelGGL((k_heston_tangent<float, float>), dim3(nb), dim3(kBlock), 0, st, a,
                          (const float*)tab, (const float*)tab, (const double*)sum_ds);
     } else {
-      hipLaunchKernelGGL(k_heston_adjoint<kHestonSeg>, dim3(nb), dim3(kBlock), 0, st, a,
-                         (const float*)tab, (float*)a.ckpt, (const double*)sum_ds);
+      // KEY1ST pays where the grid refills every SIMD (256 CUs of 8 blocks): 1M paths
+      // as fast either way, 4M x 365 3.16 ms so and 3.19 without, 30,000 x 660 341 us so
+      // and 325 without
+      auto kernel = nb > 8192 ? k_heston_adjoint<kHestonSeg, true> : k_heston_adjoint<kHestonSeg, false>;
+      hipLaunchKernelGGL(kernel, dim3(nb), dim3(kBlock), 0, st, a, (const float*)tab,
+                         (float*)a.ckpt, (const double*)sum_ds);
     }
   } else {
     double* tab = (double*)(base + lay.tab);

@@ -69,10 +69,13 @@ __host__ __device__ __forceinline__ ctr4 philox_round(ctr4 c, uint32_t k0, uint3
 // KEY1ST: in the third round y and w, in the fourth w meet the key while they
 // are wave-uniform still.  An instruction reads one scalar register, so xored with the
 // key first, on the scalar unit, they save a move each, 3 of some 53
-// instructions of four FP32 normals: batched run of 256 2190 -> 2136 us,
-// Heston 4M x 365 1596 -> 1561.  Kernels that draw FP64 normals or Poisson words are
-// 1% slower so, and those of k_euler that read their rows as scalars 1 to 2%
-// (lognormal 1M x 200 147 against 143.5).
+// instructions of four FP32 normals: batched run of 256 2190 -> 2136 us, one
+// Heston pair 4M x 365 1596 -> 1561, Heston adjoint 4M x 365 3186 -> 3159.  Only those
+// ask for it.  Kernels that draw FP64 normals or Poisson words are 1% slower
+// so, and those that read their rows as scalars or run few waves per SIMD,
+// which wait for the scalar xors, up to 5% (lognormal 1M x 200 147
+// against 143.5 us; three Heston pairs of 1000 paths x 250 170 and 161; Heston
+// adjoint of 30,000 x 660 341 and 325, tangent 289 and 279).
 template <bool KEY1ST>
 __device__ __forceinline__ ctr4 philox_round_v(ctr4 c, uint32_t k0, uint32_t k1, int round) {
   const uint64_t p0 = (uint64_t)kPhiloxM0 * c.x;
@@ -242,7 +245,7 @@ struct Gauss<double> {
 };
 
 // Four normals from one Philox block.
-template <typename T, bool KEY1ST = sizeof(T) == 4>
+template <typename T, bool KEY1ST = false>
 __device__ __forceinline__ void normals4(uint32_t blk, uint32_t path, uint32_t c2, uint32_t epoch,
                                          uint32_t k0, uint32_t k1, T* z) {
   const ctr4 r = philox4x32_10<KEY1ST>(ctr4{blk, path, c2, epoch}, k0, k1);
@@ -258,11 +261,11 @@ __device__ __forceinline__ void normals4(uint32_t blk, uint32_t path, uint32_t c
 template <typename T>
 constexpr double kGaussFold = sizeof(T) == 4 ? 1.1774100225154747 : 1.0;
 
-template <typename T>
+template <typename T, bool KEY1ST = false>
 __device__ __forceinline__ void normals4_folded(uint32_t blk, uint32_t path, uint32_t c2,
                                                 uint32_t epoch, uint32_t k0, uint32_t k1, T* z) {
   if constexpr (sizeof(T) == 4) {
-    const ctr4 r = philox4x32_10<true>(ctr4{blk, path, c2, epoch}, k0, k1);
+    const ctr4 r = philox4x32_10<KEY1ST>(ctr4{blk, path, c2, epoch}, k0, k1);
     const uint32_t a[2] = {r.x, r.z}, b[2] = {r.y, r.w};
 #pragma unroll
     for (int q = 0; q < 2; ++q) {
