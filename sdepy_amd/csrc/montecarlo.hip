@@ -342,9 +342,12 @@ __global__ void k_chf_final(int64_t n, int64_t nchunks, const double* __restrict
 // 8 per CU) come before large chunks: the last row of 500,000 values takes 12
 // us in chunks of 4096 and 54 in 8 blocks of 65536.  Where the rows fill it
 // anyway, the flush of each block's counts is what more blocks cost: 253 rows
-// of 500,000 take 162 us in chunks of 4096, 136 of 8192, 108 of 65536.
-static int64_t hist_span(int64_t rows, int64_t n) {
-  const int64_t per = rows * n / 2048;
+// of 500,000 take 162 us in chunks of 4096, 136 of 8192, 108 of 65536.  The flush grows
+// with the bins, so above 1024 of them fewer blocks do: 253 rows of 100,000 in
+// 4096 bins 88 us with 7 blocks a row, 60 with 2.
+static int64_t hist_span(int64_t rows, int64_t n, int nbins) {
+  const int64_t blocks = nbins <= 1024 || nbins > kMcLdsBins ? 2048 : 2048 * 1024 / nbins;
+  const int64_t per = rows * n / blocks;
   const int64_t span = (per + kMcHistMin - 1) / kMcHistMin * kMcHistMin;
   return span < kMcHistMin ? kMcHistMin : span > kMcHistMax ? kMcHistMax : span;
 }
@@ -472,7 +475,7 @@ extern "C" int sdegpu_mc_histogram(const void* x, int32_t dtype, int64_t rows, i
   const int64_t nc = rows * (int64_t)(nbins + 1);
   hipLaunchKernelGGL(k_zero_u64, dim3(blocks_for(nc)), dim3(kBlock), 0, st, counts, nc);
   if (int e = launch_status("k_zero_u64")) return e;
-  const int64_t span = hist_span(rows, sh.n);
+  const int64_t span = hist_span(rows, sh.n, nbins);
   const dim3 grid((unsigned)((sh.n + span - 1) / span), (unsigned)rows);
   const bool lds = nbins <= kMcLdsBins;
   // counter copies: a power of two up to 16 within kMcLdsCounterWords words

@@ -78,3 +78,10 @@ def test_along_axis_groups(n, cols, dtype):
         _lib.check(lib.sdegpu_axis_reduce(_lib.ptr(x), code, 1, n, cols, 0, cols, None, op, code,
                                           0, _lib.ptr(out), _lib.stream()))
         assert np.array_equal(out.cpu().numpy(), ref)
+
+
+@pytest.mark.parametrize('rows,n', [(1, 4096), (60, 40_001), (253, 9000)])
+@pytest.mark.parametrize('bins', [1024, 1025, 3000, 4096, 4097])
+def test_histogram_chunks_of_many_bins(rows, n, bins):
+    """Bin counts around the bounds at which the number of blocks changes."""
+    test_histogram_chunks(rows, n, bins)
