@@ -2,6 +2,9 @@
 ahead and around its groups of 4 (one component) and 2 steps (two factors), with and
 without correlations, against the presets on their own; one path more than a
 wave has."""
+import hashlib
+import json
+
 import numpy as np
 import pytest
 
@@ -34,3 +37,23 @@ def test_rows_ahead(gpu, i):
         scale = max(abs(x.mean()), x.std(), 1e-3)
         assert abs(mean[j] - x.mean()) < 1e-5 * scale, n
         assert abs(var[j] - x.var()) < 1e-4 * x.var() + 1e-12, n
+
+
+def test_points_tuned_for_the_previous_kernel_are_not_used(gpu, tmp_path, monkeypatch):
+    """A batch does not take up the launch point that the cache holds for the same
+    shape under the tag of the kernel before."""
+    path = tmp_path / 'tune.json'
+    monkeypatch.setenv('SDEPY_AMD_TUNE_CACHE', str(path))
+
+    def batch():
+        specs = [(sa.lognorm_process(paths=1000, steps=20, dtype=np.float32,
+                                     rng=np.random.default_rng(3)), (0., 1.))]
+        return B.BatchedTerminalMoments(specs, autotune=False, graph=False)
+    b = batch()
+    old = hashlib.sha1(b'v2' + b.nsteps.tobytes() + b.paths.tobytes() +
+                       b.nvars.tobytes()).hexdigest()[:16]
+    point = {'blocks': b.cu * 12, 'tile_waves': 16, 'order': 'interleave'}
+    path.write_text(json.dumps({old: point}))
+    assert batch().tile_waves == 1
+    path.write_text(json.dumps({b.sig: point}))
+    assert batch().tile_waves == 16
