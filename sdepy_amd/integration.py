@@ -372,10 +372,10 @@ class _gpu_sde:
         allocate the device output; returns a ``PreparedRun`` whose
         ``launch()`` issues the kernels and ``result()`` returns the
         process(es).  ``__call__`` is ``prepare(timeline).run()``.
-        With ``moments=True`` the kernels also reduce every stored row to
-        its FP64 moments as they store it, so that the run's ``pmean``,
-        ``pvar``, ``psum`` and ``pstd`` need no further pass over the
-        output."""
+        With ``moments=True`` every launch also reduces every stored row to
+        its FP64 moments, so that the run's ``pmean``, ``pvar``, ``psum`` and
+        ``pstd`` only read them back: the kernels as they store the row, or, for
+        few paths, a pass over the rows right after them."""
         run = self._prepare(timeline)
         if moments:
             run._fuse_moments()
@@ -714,11 +714,28 @@ class _Pass:
 
 
 # Paths up to which prepare(moments=True) reduces the rows by a pass after the
-# kernels: there several waves share 64 paths (k_euler_split, up to 1024 waves
-# of paths), which the kernels with the moments fused in do not, and the rows
-# are still in the caches.  10,000 x 252 lognormal FP64, launch and both moments
-# read back: 110 us, 172 us with the moments fused in.
+# kernels, at most: there several waves share 64 paths (k_euler_split, up to 1024
+# waves of paths), which the kernels with the moments fused in do not.  10,000 x
+# 252 lognormal FP64, launch and both moments read back: 110 us, 172 us fused.
 _SEPARATE_PATHS = 65536
+
+
+def _separate_paths(prob):
+    """Paths up to which a launch of ``prob`` and a pass over its rows take less
+    than the launch with the moments fused in.
+
+    Wherever several waves share 64 paths, the two take 0.3 to 1.0 of the fused
+    launch's time (CIR of 65,000 paths the least).  Jump models that they do not share
+    (3 components or more): 0.65 to 1.05.  The others gain
+    only where the fused kernel's lower occupancy shows: 0.65 to 1.05 up to 16,384
+    paths, 0.95 to 1.35 at 32,000 and above (3 Heston pairs FP32 65,000 x
+    1000, 13 rows: 761 us fused, 931 not)."""
+    jump = prob.model == _lib.MODEL_JUMPDIFF
+    recorded = prob.replay_dw or prob.replay_dj
+    shared = prob.nvars <= (2 if jump else 4) and not (
+        recorded or prob.lam_paths or prob.nvars_total)
+    return _SEPARATE_PATHS if shared or (jump and not recorded) \
+        else min(_SEPARATE_PATHS, 16384)
 
 
 class PreparedRun:
@@ -736,7 +753,7 @@ class PreparedRun:
         """Have every pass reduce its stored rows as it stores them: block
         partials [ceil(paths/256)][rows][2], merged after each launch into
         the FP64 (mean, m2) of every row.  Runs of few paths are reduced by
-        a pass of its own within the launch (_SEPARATE_PATHS)."""
+        a pass of its own within the launch (_separate_paths)."""
         if any(prob.param_paths or prob.nvars > _lib.MAX_VARS
                for p in self.passes for prob in p.probs):
             # per-path parameters or a wide coupled block: the separate
@@ -745,7 +762,7 @@ class PreparedRun:
         n_t, nout, P = self.xx_dev.shape
         rows = n_t * nout
         self._mom_mean, self._mom_m2 = _lib.empty((2, rows), np.float64)
-        if P <= _SEPARATE_PATHS:
+        if P <= min(_separate_paths(prob) for p in self.passes for prob in p.probs):
             self._mom_nbytes = _lib.lib().sdegpu_moments_workspace(rows, P)
             self._mom_ws = _lib.workspace(self._mom_nbytes)
             return

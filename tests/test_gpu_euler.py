@@ -678,6 +678,61 @@ def test_fused_row_moments_match_numpy(gpu, case):
             assert np.allclose(got_v, np.asarray(pvi, np.float64).reshape(mean.shape),
                                rtol=1e-12, atol=1e-15)
 
+C4 = np.array([[1., .3, -.2, .1], [.3, 1., .25, 0.], [-.2, .25, 1., .4], [.1, 0., .4, 1.]])
+
+
+@pytest.mark.parametrize('points,steps,cls,kw', [
+    (21, 61, sa.ornstein_uhlenbeck_process, dict(paths=3000, vshape=4, k=1.5, sigma=.3, corr=C4)),
+    (21, 61, sa.ornstein_uhlenbeck_process, dict(paths=3000, vshape=4, k=1.5, sigma=.3, corr=C4,
+                                                 dtype=np.float32)),
+    (21, 21, sa.lognorm_process, dict(paths=1, mu=.1, sigma=.3)),
+    (21, 21, sa.wiener_process, dict(paths=257, vshape=3)),
+    (9, 33, sa.full_heston_process, dict(paths=1000, vshape=2, i0=3, rho=[-.5, -.3])),
+    (21, 21, sa.lognorm_process, dict(paths=700, vshape=(3, 4), mu=.05, sigma=.2)),
+    (3, 101, sa.kou_jumpdiff_process, dict(paths=2000, lam=5.)),
+    (3, 101, sa.merton_jumpdiff_process, dict(paths=2000, vshape=2, lam=5., dtype=np.float32))])
+def test_row_moments_fused_at_any_path_count(gpu, monkeypatch, points, steps, cls, kw):
+    """prepare(moments=True) with the moments fused into the kernels, as for more
+    paths: a correlated and a ragged state, two passes, component groups, deferred
+    jumps."""
+    from sdepy_amd import integration
+    monkeypatch.setattr(integration, '_SEPARATE_PATHS', 0)
+    run = cls(**dict(dict(dtype=np.float64, steps=steps, rng=np.random.default_rng(5)),
+                     **kw)).prepare(np.linspace(0., 1., points), moments=True)
+    assert run._row_mom is not None
+    _check_row_moments(run)
+
+
+def _check_row_moments(run):
+    x, m, v = run.run(), run.pmean(dtype=np.float64), run.pvar(dtype=np.float64)
+    for xi, mi, vi in zip(*(z if isinstance(z, tuple) else (z,) for z in (x, m, v))):
+        mean, m2 = _np_moments(xi)
+        var = m2 / xi.shape[-1]
+        assert np.abs(np.asarray(mi).reshape(mean.shape) - mean).max() < \
+            1e-12 * max(1., np.abs(mean).max())
+        assert np.abs(np.asarray(vi).reshape(mean.shape) - var).max() < \
+            1e-12 * max(1., var.max())
+
+
+@pytest.mark.parametrize('fused,cls,kw', [
+    (True, sa.ornstein_uhlenbeck_process, dict(paths=16_385, vshape=5, rho=None)),
+    (False, sa.ornstein_uhlenbeck_process, dict(paths=16_384, vshape=5, rho=None)),
+    (True, sa.full_heston_process, dict(paths=16_500, vshape=3, rho=[-.5, -.3, .1])),
+    (True, sa.lognorm_process, dict(paths=20_000, vshape=8, sigma=.2)),
+    (True, sa.merton_jumpdiff_process, dict(paths=65_700, vshape=2, lam=3.)),
+    (True, sa.merton_jumpdiff_process, dict(paths=65_700, lam=3.)),
+    (True, sa.lognorm_process, dict(paths=65_537, sigma=.2)),
+    (False, sa.lognorm_process, dict(paths=65_536, sigma=.2)),
+    (False, sa.kou_jumpdiff_process, dict(paths=20_001, vshape=3, lam=3., dtype=np.float64))])
+def test_row_moments_by_the_default_rule(gpu, fused, cls, kw):
+    """Moments fused into the kernels or reduced after them, around the path counts at
+    which that changes, with partial last blocks."""
+    tt = np.linspace(0., 1., 9)
+    kw = dict(dict(dtype=np.float32, steps=17, rng=np.random.default_rng(12)), **kw)
+    run = cls(**kw).prepare(tt, moments=True)
+    assert (run._row_mom is not None) == fused
+    _check_row_moments(run)
+
 
 @pytest.mark.parametrize('dtype', [np.float32, np.float64])
 def test_fill_rows(gpu, dtype):

@@ -538,3 +538,21 @@ def test_scalar_parameters_convert_as_arrays_do(value, want):
     assert np.array_equal(got, np.full((2, 1), want), equal_nan=True)
     with pytest.raises(TypeError):
         sa.lognorm_process(paths=4, mu=1j, steps=4)._eval('mu', t0s, (1,))
+
+
+@pytest.mark.parametrize('model,nvars,field,want', [
+    (_lib.MODEL_OU, 4, None, 65536), (_lib.MODEL_OU, 5, None, 16384),
+    (_lib.MODEL_HESTON, 4, None, 65536), (_lib.MODEL_HESTON, 6, None, 16384),
+    (_lib.MODEL_CIR, 1, 'replay_dw', 16384), (_lib.MODEL_LOGNORM, 4, 'nvars_total', 16384),
+    (_lib.MODEL_JUMPDIFF, 2, None, 65536), (_lib.MODEL_JUMPDIFF, 8, None, 65536),
+    (_lib.MODEL_JUMPDIFF, 1, 'lam_paths', 65536), (_lib.MODEL_JUMPDIFF, 1, 'replay_dj', 16384)])
+def test_row_moments_are_separate_where_that_is_faster(model, nvars, field, want, monkeypatch):
+    """prepare(moments=True) gives up the fused moments of small runs only where
+    several waves share paths, or where the two kernels take less."""
+    prob = _lib.EulerProblem()
+    prob.model, prob.nvars = model, nvars
+    if field:
+        setattr(prob, field, 16)
+    assert integ._separate_paths(prob) == want
+    monkeypatch.setattr(integ, '_SEPARATE_PATHS', 0)
+    assert integ._separate_paths(prob) == 0
