@@ -729,13 +729,15 @@ def _separate_paths(prob):
     (3 components or more): 0.65 to 1.05.  The others gain
     only where the fused kernel's lower occupancy shows: 0.65 to 1.05 up to 16,384
     paths, 0.95 to 1.35 at 32,000 and above (3 Heston pairs FP32 65,000 x
-    1000, 13 rows: 761 us fused, 931 not)."""
+    1000, 13 rows: 761 us fused, 931 not), FP32 OU states 0.85 to 1.02 at 32,000."""
     jump = prob.model == _lib.MODEL_JUMPDIFF
     recorded = prob.replay_dw or prob.replay_dj
     shared = prob.nvars <= (2 if jump else 4) and not (
         recorded or prob.lam_paths or prob.nvars_total)
-    return _SEPARATE_PATHS if shared or (jump and not recorded) \
-        else min(_SEPARATE_PATHS, 16384)
+    if shared or (jump and not recorded):
+        return _SEPARATE_PATHS
+    ou = prob.model == _lib.MODEL_OU and prob.dtype == _lib.F32
+    return min(_SEPARATE_PATHS, 32768 if ou else 16384)
 
 
 class PreparedRun:

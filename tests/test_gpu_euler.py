@@ -715,8 +715,9 @@ def _check_row_moments(run):
 
 
 @pytest.mark.parametrize('fused,cls,kw', [
-    (True, sa.ornstein_uhlenbeck_process, dict(paths=16_385, vshape=5, rho=None)),
-    (False, sa.ornstein_uhlenbeck_process, dict(paths=16_384, vshape=5, rho=None)),
+    (True, sa.ornstein_uhlenbeck_process, dict(paths=32_769, vshape=5)),
+    (False, sa.ornstein_uhlenbeck_process, dict(paths=32_768, vshape=5)),
+    (True, sa.cox_ingersoll_ross_process, dict(paths=16_385, vshape=5)),
     (True, sa.full_heston_process, dict(paths=16_500, vshape=3, rho=[-.5, -.3, .1])),
     (True, sa.lognorm_process, dict(paths=20_000, vshape=8, sigma=.2)),
     (True, sa.merton_jumpdiff_process, dict(paths=65_700, vshape=2, lam=3.)),

@@ -541,7 +541,7 @@ def test_scalar_parameters_convert_as_arrays_do(value, want):
 
 
 @pytest.mark.parametrize('model,nvars,field,want', [
-    (_lib.MODEL_OU, 4, None, 65536), (_lib.MODEL_OU, 5, None, 16384),
+    (_lib.MODEL_OU, 4, None, 65536), (_lib.MODEL_OU, 5, None, 32768),
     (_lib.MODEL_HESTON, 4, None, 65536), (_lib.MODEL_HESTON, 6, None, 16384),
     (_lib.MODEL_CIR, 1, 'replay_dw', 16384), (_lib.MODEL_LOGNORM, 4, 'nvars_total', 16384),
     (_lib.MODEL_JUMPDIFF, 2, None, 65536), (_lib.MODEL_JUMPDIFF, 8, None, 65536),
