@@ -10,22 +10,22 @@ namespace sdegpu {
 // antithetic halves or component groups are involved, with or without fused
 // row moments.
 template <typename T>
-static EulerKernel<T> choose(bool plain, bool mom, bool pp, int model, int m, int d, bool defer);
+static EulerKernel<T> choose(bool plain, bool mom, bool pp, int model, int m, int d, JumpForm form);
 template <>
 EulerKernel<float> choose<float>(bool plain, bool mom, bool pp, int model, int m, int d,
-                                 bool defer) {
-  if (pp) return euler_set_pp_f32(model, m, d, defer);
-  if (plain) return mom ? euler_set_plain_mom_f32(model, m, d, defer)
-                        : euler_set_plain_f32(model, m, d, defer);
-  return mom ? euler_set_gen_mom_f32(model, m, d, defer) : euler_set_gen_f32(model, m, d, defer);
+                                 JumpForm form) {
+  if (pp) return euler_set_pp_f32(model, m, d, form);
+  if (plain) return mom ? euler_set_plain_mom_f32(model, m, d, form)
+                        : euler_set_plain_f32(model, m, d, form);
+  return mom ? euler_set_gen_mom_f32(model, m, d, form) : euler_set_gen_f32(model, m, d, form);
 }
 template <>
 EulerKernel<double> choose<double>(bool plain, bool mom, bool pp, int model, int m, int d,
-                                   bool defer) {
-  if (pp) return euler_set_pp_f64(model, m, d, defer);
-  if (plain) return mom ? euler_set_plain_mom_f64(model, m, d, defer)
-                        : euler_set_plain_f64(model, m, d, defer);
-  return mom ? euler_set_gen_mom_f64(model, m, d, defer) : euler_set_gen_f64(model, m, d, defer);
+                                   JumpForm form) {
+  if (pp) return euler_set_pp_f64(model, m, d, form);
+  if (plain) return mom ? euler_set_plain_mom_f64(model, m, d, form)
+                        : euler_set_plain_f64(model, m, d, form);
+  return mom ? euler_set_gen_mom_f64(model, m, d, form) : euler_set_gen_f64(model, m, d, form);
 }
 
 // exp_mask the model implies for nout stored values (see OutRule and
@@ -228,7 +228,7 @@ extern "C" int sdegpu_euler(const sdegpu_euler_problem* pr, void* stream) {
   // no recorded increments and no antithetic halves: the plain instance
   const bool plain = !pr->replay_dw && !pr->replay_dj && pr->anti_w == 0 && pr->anti_j == 0 &&
                      !grouped && !(jump && pr->lam_paths);
-  const bool defer = jump && pr->jump_defer != 0 && !wide;
+  const JumpForm form = jump_form(jump && pr->jump_defer != 0 && !wide, pr->nsteps, m);
   const bool mom = pr->row_moments != nullptr;
   const bool pp = pr->param_paths != nullptr;
   if (pp && mom)
@@ -261,13 +261,13 @@ extern "C" int sdegpu_euler(const sdegpu_euler_problem* pr, void* stream) {
   }
   if (pr->dtype == SDEGPU_F32) {
     EulerKernel<float> k = wide ? euler_wide_kernel<float>(pr->model, m, wide_gen)
-                                : choose<float>(plain, mom, pp, pr->model, m, hd, defer);
+                                : choose<float>(plain, mom, pp, pr->model, m, hd, form);
     if (!k) return fail(SDEGPU_EUNSUPPORTED, "no kernel for model %d with %d components", pr->model, m);
     hipLaunchKernelGGL(k, grid, block, 0, st, a, (const float*)pr->coef, pr->store_row,
                        pr->pois, (float*)pr->out);
   } else {
     EulerKernel<double> k = wide ? euler_wide_kernel<double>(pr->model, m, wide_gen)
-                                 : choose<double>(plain, mom, pp, pr->model, m, hd, defer);
+                                 : choose<double>(plain, mom, pp, pr->model, m, hd, form);
     if (!k) return fail(SDEGPU_EUNSUPPORTED, "no kernel for model %d with %d components", pr->model, m);
     hipLaunchKernelGGL(k, grid, block, 0, st, a, (const double*)pr->coef, pr->store_row,
                        pr->pois, (double*)pr->out);

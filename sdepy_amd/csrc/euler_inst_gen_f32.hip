@@ -4,7 +4,7 @@
 namespace sdegpu {
 
 SDEGPU_EULER_SET(euler_set_gen_f32, true, float, false) {
-  return pick_kernel_mom<true, float, false>(model, m, d, defer);
+  return pick_kernel_mom<true, float, false>(model, m, d, form);
 }
 
 }  // namespace sdegpu

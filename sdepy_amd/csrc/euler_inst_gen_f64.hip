@@ -4,7 +4,7 @@
 namespace sdegpu {
 
 SDEGPU_EULER_SET(euler_set_gen_f64, true, double, false) {
-  return pick_kernel_mom<true, double, false>(model, m, d, defer);
+  return pick_kernel_mom<true, double, false>(model, m, d, form);
 }
 
 }  // namespace sdegpu

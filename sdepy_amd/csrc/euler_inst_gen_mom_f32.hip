@@ -4,7 +4,7 @@
 namespace sdegpu {
 
 SDEGPU_EULER_SET(euler_set_gen_mom_f32, true, float, true) {
-  return pick_kernel_mom<true, float, true>(model, m, d, defer);
+  return pick_kernel_mom<true, float, true>(model, m, d, form);
 }
 
 }  // namespace sdegpu

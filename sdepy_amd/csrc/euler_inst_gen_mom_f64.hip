@@ -4,7 +4,7 @@
 namespace sdegpu {
 
 SDEGPU_EULER_SET(euler_set_gen_mom_f64, true, double, true) {
-  return pick_kernel_mom<true, double, true>(model, m, d, defer);
+  return pick_kernel_mom<true, double, true>(model, m, d, form);
 }
 
 }  // namespace sdegpu

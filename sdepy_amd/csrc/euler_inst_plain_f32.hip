@@ -4,7 +4,7 @@
 namespace sdegpu {
 
 SDEGPU_EULER_SET(euler_set_plain_f32, false, float, false) {
-  return pick_kernel_mom<false, float, false>(model, m, d, defer);
+  return pick_kernel_mom<false, float, false>(model, m, d, form);
 }
 
 }  // namespace sdegpu

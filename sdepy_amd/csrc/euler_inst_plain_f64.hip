@@ -4,7 +4,7 @@
 namespace sdegpu {
 
 SDEGPU_EULER_SET(euler_set_plain_f64, false, double, false) {
-  return pick_kernel_mom<false, double, false>(model, m, d, defer);
+  return pick_kernel_mom<false, double, false>(model, m, d, form);
 }
 
 }  // namespace sdegpu

@@ -4,7 +4,7 @@
 namespace sdegpu {
 
 SDEGPU_EULER_SET(euler_set_plain_mom_f32, false, float, true) {
-  return pick_kernel_mom<false, float, true>(model, m, d, defer);
+  return pick_kernel_mom<false, float, true>(model, m, d, form);
 }
 
 }  // namespace sdegpu

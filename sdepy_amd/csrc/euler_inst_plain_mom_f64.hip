@@ -4,7 +4,7 @@
 namespace sdegpu {
 
 SDEGPU_EULER_SET(euler_set_plain_mom_f64, false, double, true) {
-  return pick_kernel_mom<false, double, true>(model, m, d, defer);
+  return pick_kernel_mom<false, double, true>(model, m, d, form);
 }
 
 }  // namespace sdegpu

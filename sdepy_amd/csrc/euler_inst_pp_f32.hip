@@ -5,7 +5,7 @@
 namespace sdegpu {
 
 SDEGPU_EULER_SET(euler_set_pp_f32, true, float, false) {
-  return pick_kernel_mom<true, float, false, true>(model, m, d, defer);
+  return pick_kernel_mom<true, float, false, true>(model, m, d, form);
 }
 
 }  // namespace sdegpu

@@ -5,7 +5,7 @@
 namespace sdegpu {
 
 SDEGPU_EULER_SET(euler_set_pp_f64, true, double, false) {
-  return pick_kernel_mom<true, double, false, true>(model, m, d, defer);
+  return pick_kernel_mom<true, double, false, true>(model, m, d, form);
 }
 
 }  // namespace sdegpu

@@ -254,6 +254,22 @@ __device__ __forceinline__ void heston_next(T& x, T& y, int& cnt, const HestonRo
   }
 }
 
+// The least of v over a wave whose lanes are all active.
+__device__ __forceinline__ uint32_t wave_least(uint32_t v) {
+  auto step = [&](auto ctrl) {
+    const uint32_t other = (uint32_t)__builtin_amdgcn_update_dpp(
+        -1, (int)v, decltype(ctrl)::value, 0xf, 0xf, false);
+    v = other < v ? other : v;
+  };
+  step(std::integral_constant<int, 0x111>{});  // row_shr:1, 2, 4, 8
+  step(std::integral_constant<int, 0x112>{});
+  step(std::integral_constant<int, 0x114>{});
+  step(std::integral_constant<int, 0x118>{});
+  step(std::integral_constant<int, 0x142>{});  // row_bcast:15, 31
+  step(std::integral_constant<int, 0x143>{});
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+
 // The word below which every Poisson word of a pass is a count of 0: a word w
 // draws 0 when (w + 0.5) 2^-32 <= exp(-lam |ds|), so every w below the smallest
 // exp(-lam |ds|) 2^32 of the n table rows does, whatever its step; words
@@ -262,20 +278,30 @@ __device__ __forceinline__ void heston_next(T& x, T& y, int& cnt, const HestonRo
 // uniform, selecting the sum and counting took a dozen instructions: Merton
 // 2M x 252 FP32, 2 rows 691 -> 562 us, 253 rows 1087 -> 964 us (a bound per
 // step, from the table or beside it, cost more than it saved).  Every thread
-// of the block must call it.
+// of the block must call it.  Up to 256 rows each wave reads them all, four loads at
+// once and no barrier: 12 to 24 steps 1 to 2% faster than with FP64 shuffles and a
+// barrier.
 __device__ __forceinline__ uint32_t zero_count_bound(const double* __restrict__ pois, int64_t n,
                                                      unsigned threads = kBlock) {
-  __shared__ double sh[16];
-  double p = 1.0;
-  for (int64_t i = threadIdx.x; i < n; i += threads) p = fmin(p, pois[2 * i + 1]);
+  auto of_row = [&](int64_t i) -> uint32_t {
+    const double b = pois[2 * i + 1] * 0x1p32;
+    return b < 0x1p32 ? (uint32_t)b : 0xFFFFFFFFu;
+  };
+  uint32_t least = 0xFFFFFFFFu;
+  if (n <= 256) {
+    const int64_t lane = threadIdx.x & 63;
 #pragma unroll
-  for (int off = 32; off > 0; off >>= 1) p = fmin(p, __shfl_xor(p, off, 64));
-  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = p;
+    for (int k = 0; k < 4; ++k)
+      if (lane + 64 * k < n) least = min(least, of_row(lane + 64 * k));
+    return wave_least(least);
+  }
+  __shared__ uint32_t sh[16];
+  for (int64_t i = threadIdx.x; i < n; i += threads) least = min(least, of_row(i));
+  least = wave_least(least);
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = least;
   __syncthreads();
-  for (unsigned w = 0; w < threads >> 6; ++w) p = fmin(p, sh[w]);
-  const double b = p * 0x1p32;
-  const uint32_t bound = b < 0x1p32 ? (uint32_t)b : 0xFFFFFFFFu;
-  return __builtin_amdgcn_readfirstlane(bound);
+  for (unsigned w = 0; w < threads >> 6; ++w) least = min(least, sh[w]);
+  return __builtin_amdgcn_readfirstlane(least);
 }
 
 // Heston working state (SDEs.pack, integration.py:1759-1783, with the two
@@ -494,8 +520,11 @@ __device__ __forceinline__ void flush_row_moments(const EulerArgs& a, T* cols, d
   }
 }
 
+// BOUND (jump models): counts of 0 by the pass's bound, and with one component
+// the step's constants from LDS; without, every word is inverted in place.  FP64: always.
+// FP32 in place, without row moments: JumpForm.
 template <int MODEL, typename T, int M, int D, bool GEN, bool DEFER = false, bool MOM = false,
-          bool PP = false>
+          bool PP = false, bool BOUND = true>
 __global__ __launch_bounds__(kBlock, MOM ? 8 : 1) void k_euler(const EulerArgs a, const T* __restrict__ coef,
                                                   const int32_t* __restrict__ store_row,
                                                   const double* __restrict__ pois,
@@ -508,7 +537,7 @@ __global__ __launch_bounds__(kBlock, MOM ? 8 : 1) void k_euler(const EulerArgs a
   constexpr int N = kHeston ? M / 2 : M;
   // (FP32 Wiener and lognormal states keep p ds + sigma dw: rounded otherwise, a
   // value in a million of theirs changes its bin in a histogram)
-  constexpr bool kAdd1 = (kJump || (sizeof(T) == 8 && (MODEL == SDEGPU_MODEL_WIENER ||
+  constexpr bool kAdd1 = ((kJump && BOUND) || (sizeof(T) == 8 && (MODEL == SDEGPU_MODEL_WIENER ||
                                                        MODEL == SDEGPU_MODEL_LOGNORM))) &&
                          M == 1 && !GEN && !PP;
   constexpr bool kRow = (kHeston && M == 2 && !GEN && !PP) || kAdd1;
@@ -516,7 +545,7 @@ __global__ __launch_bounds__(kBlock, MOM ? 8 : 1) void k_euler(const EulerArgs a
 
   gauss_init<T>();
   // words below it are counts of 0 (per-path intensities: none are known to be)
-  const uint32_t zero_below = kJump && !(GEN && (a.replay_dj || a.lamp))
+  const uint32_t zero_below = kJump && BOUND && !(GEN && (a.replay_dj || a.lamp))
                                   ? zero_count_bound(pois, (int64_t)a.nsteps * M)
                                   : 0u;
   // With fused row moments every thread of the block takes part in the LDS
@@ -856,7 +885,7 @@ __global__ __launch_bounds__(kBlock, MOM ? 8 : 1) void k_euler(const EulerArgs a
           const bool stored = store_row[s] >= 0;
 #pragma unroll
           for (int v = 0; v < M; ++v) {
-            if (upois[k * M + v] < zero_below) continue;
+            if (BOUND && upois[k * M + v] < zero_below) continue;
             if constexpr (kLate) {
               if (late && !stored && njev < kJumpEvents && s < (1 << 20)) {
                 jev[njev][threadIdx.x] =
@@ -915,19 +944,38 @@ __global__ __launch_bounds__(kBlock, MOM ? 8 : 1) void k_euler(const EulerArgs a
 template <typename T>
 using EulerKernel = void (*)(const EulerArgs, const T*, const int32_t*, const double*, T*);
 
-template <bool GEN, int MODEL, typename T, bool DEFER, bool MOM, bool PP = false>
+template <bool GEN, int MODEL, typename T, bool DEFER, bool MOM, bool PP = false, bool BOUND = true>
 EulerKernel<T> pick_m(int m) {
+  // (JumpForm: no bound in FP32 with row moments of 2 and more components)
+  constexpr bool B = BOUND && !(MODEL == SDEGPU_MODEL_JUMPDIFF && MOM && sizeof(T) == 4);
   switch (m) {
-    case 1: return k_euler<MODEL, T, 1, 1, GEN, DEFER, MOM, PP>;
-    case 2: return k_euler<MODEL, T, 2, 1, GEN, DEFER, MOM, PP>;
-    case 3: return k_euler<MODEL, T, 3, 1, GEN, DEFER, MOM, PP>;
-    case 4: return k_euler<MODEL, T, 4, 1, GEN, DEFER, MOM, PP>;
-    case 5: return k_euler<MODEL, T, 5, 1, GEN, DEFER, MOM, PP>;
-    case 6: return k_euler<MODEL, T, 6, 1, GEN, DEFER, MOM, PP>;
-    case 7: return k_euler<MODEL, T, 7, 1, GEN, DEFER, MOM, PP>;
-    case 8: return k_euler<MODEL, T, 8, 1, GEN, DEFER, MOM, PP>;
+    case 1: return k_euler<MODEL, T, 1, 1, GEN, DEFER, MOM, PP, BOUND>;
+    case 2: return k_euler<MODEL, T, 2, 1, GEN, DEFER, MOM, PP, B>;
+    case 3: return k_euler<MODEL, T, 3, 1, GEN, DEFER, MOM, PP, B>;
+    case 4: return k_euler<MODEL, T, 4, 1, GEN, DEFER, MOM, PP, B>;
+    case 5: return k_euler<MODEL, T, 5, 1, GEN, DEFER, MOM, PP, B>;
+    case 6: return k_euler<MODEL, T, 6, 1, GEN, DEFER, MOM, PP, B>;
+    case 7: return k_euler<MODEL, T, 7, 1, GEN, DEFER, MOM, PP, B>;
+    case 8: return k_euler<MODEL, T, 8, 1, GEN, DEFER, MOM, PP, B>;
     default: return nullptr;
   }
+}
+
+// How a jump model's kernel takes its jumps.
+//
+// In FP32 without row moments the bound pays in place (kInPlaceBound) where
+// most waves pass a step without a jump: 1 component from 96 steps on, more from
+// 160, at some 1 to 2 jumps a pass.  Below, nearly every step has a lane that enters
+// the inversion behind one more branch, and the prologue is not paid back.
+// 100,000 paths, every step stored, us without / with it: 1 component 12 steps 18.0 / 20.5,
+// 64 steps 56 / 58, 96 steps 72 / 73, 128 steps 86 / 85, 252 steps 135 / 124; 2 components
+// 64 steps 101 / 105, 160 steps 180 / 179, 252 steps 243 / 234.
+// With row moments, of 2 and more components it never does: their LDS is full and
+// the scalar registers spill (2 Kous 1.5M x 252, 13 rows 1249 us with it, 1101
+// without).
+enum JumpForm { kInPlace, kDeferred, kInPlaceBound };
+inline JumpForm jump_form(bool defer, int nsteps, int m) {
+  return defer ? kDeferred : nsteps >= (m == 1 ? 96 : 160) ? kInPlaceBound : kInPlace;
 }
 
 // Heston kernels by (M, D): D log-x components per group of 2D.
@@ -947,9 +995,8 @@ EulerKernel<T> pick_heston(int m, int d) {
   }
 }
 
-// defer: jumpdiff draws jump sizes at the next stored step (see k_euler)
 template <bool GEN, typename T, bool MOM, bool PP = false>
-EulerKernel<T> pick_kernel_mom(int model, int m, int d, bool defer) {
+EulerKernel<T> pick_kernel_mom(int model, int m, int d, JumpForm form) {
   switch (model) {
     case SDEGPU_MODEL_WIENER: return pick_m<GEN, SDEGPU_MODEL_WIENER, T, false, MOM, PP>(m);
     case SDEGPU_MODEL_LOGNORM: return pick_m<GEN, SDEGPU_MODEL_LOGNORM, T, false, MOM, PP>(m);
@@ -957,8 +1004,12 @@ EulerKernel<T> pick_kernel_mom(int model, int m, int d, bool defer) {
     case SDEGPU_MODEL_CIR: return pick_m<GEN, SDEGPU_MODEL_CIR, T, false, MOM, PP>(m);
     case SDEGPU_MODEL_HESTON: return pick_heston<GEN, T, MOM, PP>(m, d);
     case SDEGPU_MODEL_JUMPDIFF:
-      return defer ? pick_m<GEN, SDEGPU_MODEL_JUMPDIFF, T, true, MOM, PP>(m)
-                   : pick_m<GEN, SDEGPU_MODEL_JUMPDIFF, T, false, MOM, PP>(m);
+      if constexpr (sizeof(T) == 4 && !MOM) {
+        if (form == kInPlace)
+          return pick_m<GEN, SDEGPU_MODEL_JUMPDIFF, T, false, MOM, PP, false>(m);
+      }
+      return form == kDeferred ? pick_m<GEN, SDEGPU_MODEL_JUMPDIFF, T, true, MOM, PP>(m)
+                               : pick_m<GEN, SDEGPU_MODEL_JUMPDIFF, T, false, MOM, PP>(m);
     default: return nullptr;
   }
 }
@@ -967,7 +1018,7 @@ EulerKernel<T> pick_kernel_mom(int model, int m, int d, bool defer) {
 // they build in parallel), one per (GEN, T, MOM) and the two with per-path
 // parameters (general, no fused moments): euler_inst_*.hip.
 #define SDEGPU_EULER_SET(NAME, GEN, T, MOM) \
-  EulerKernel<T> NAME(int model, int m, int d, bool defer)
+  EulerKernel<T> NAME(int model, int m, int d, JumpForm form)
 SDEGPU_EULER_SET(euler_set_pp_f32, true, float, false);
 SDEGPU_EULER_SET(euler_set_pp_f64, true, double, false);
 SDEGPU_EULER_SET(euler_set_gen_f32, true, float, false);
