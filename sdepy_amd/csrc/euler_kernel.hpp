@@ -522,7 +522,7 @@ __device__ __forceinline__ void flush_row_moments(const EulerArgs& a, T* cols, d
 
 // BOUND (jump models): counts of 0 by the pass's bound, and with one component
 // the step's constants from LDS; without, every word is inverted in place.  FP64: always.
-// FP32 in place, without row moments: JumpForm.
+// FP32 without row moments: JumpForm.
 template <int MODEL, typename T, int M, int D, bool GEN, bool DEFER = false, bool MOM = false,
           bool PP = false, bool BOUND = true>
 __global__ __launch_bounds__(kBlock, MOM ? 8 : 1) void k_euler(const EulerArgs a, const T* __restrict__ coef,
@@ -970,12 +970,16 @@ EulerKernel<T> pick_m(int m) {
 // 100,000 paths, every step stored, us without / with it: 1 component 12 steps 18.0 / 20.5,
 // 64 steps 56 / 58, 96 steps 72 / 73, 128 steps 86 / 85, 252 steps 135 / 124; 2 components
 // 64 steps 101 / 105, 160 steps 180 / 179, 252 steps 243 / 234.
+// Deferred jumps, rows at the ends: from 24 steps on (40 with 3 and more components); 70,000
+// paths, 1 component 12 steps 12.9 / 13.8, 24 steps 17.6 / 17.4, 32 steps 20.1 / 19.2; 3
+// components 24 steps 53.6 / 57.6; 4 of 40 steps, 5 rows 76 (before the bound) / 69.
 // With row moments, of 2 and more components it never does: their LDS is full and
 // the scalar registers spill (2 Kous 1.5M x 252, 13 rows 1249 us with it, 1101
 // without).
-enum JumpForm { kInPlace, kDeferred, kInPlaceBound };
+enum JumpForm { kInPlace, kDeferred, kInPlaceBound, kDeferredBound };
 inline JumpForm jump_form(bool defer, int nsteps, int m) {
-  return defer ? kDeferred : nsteps >= (m == 1 ? 96 : 160) ? kInPlaceBound : kInPlace;
+  if (defer) return nsteps >= (m <= 2 ? 24 : 40) ? kDeferredBound : kDeferred;
+  return nsteps >= (m == 1 ? 96 : 160) ? kInPlaceBound : kInPlace;
 }
 
 // Heston kernels by (M, D): D log-x components per group of 2D.
@@ -1007,9 +1011,12 @@ EulerKernel<T> pick_kernel_mom(int model, int m, int d, JumpForm form) {
       if constexpr (sizeof(T) == 4 && !MOM) {
         if (form == kInPlace)
           return pick_m<GEN, SDEGPU_MODEL_JUMPDIFF, T, false, MOM, PP, false>(m);
+        if (form == kDeferred)
+          return pick_m<GEN, SDEGPU_MODEL_JUMPDIFF, T, true, MOM, PP, false>(m);
       }
-      return form == kDeferred ? pick_m<GEN, SDEGPU_MODEL_JUMPDIFF, T, true, MOM, PP>(m)
-                               : pick_m<GEN, SDEGPU_MODEL_JUMPDIFF, T, false, MOM, PP>(m);
+      return form == kDeferred || form == kDeferredBound
+                 ? pick_m<GEN, SDEGPU_MODEL_JUMPDIFF, T, true, MOM, PP>(m)
+                 : pick_m<GEN, SDEGPU_MODEL_JUMPDIFF, T, false, MOM, PP>(m);
     default: return nullptr;
   }
 }

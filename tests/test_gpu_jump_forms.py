@@ -1,5 +1,5 @@
 """FP32 jump models on either side of the step counts from which zero counts are decided by
-the pass's bound where jumps are summed in place, with antithetic halves and with fused
+the pass's bound, where jumps are summed in place and where they are deferred, with antithetic halves and with fused
 row moments too; counts and values against the oracle, jump by jump."""
 import numpy as np
 import pytest
@@ -17,9 +17,21 @@ PATHS = 65_602
                                          (3, 157), (3, 163)])
 @pytest.mark.parametrize('lam', [.5, 40.])
 def test_forms_match_oracle(gpu, how, nvar, nsteps, lam):
-    vshape = () if nvar == 1 else (nvar,)
     grid = np.linspace(0., 1., nsteps + 1)
     tt = np.unique(np.r_[grid[::5], grid[-1]])      # too many rows to defer jumps
+    _check(how, nvar, grid, tt, lam, 0)
+
+
+@pytest.mark.parametrize('how', ['plain', 'antithetic', 'moments'])
+@pytest.mark.parametrize('nvar,nsteps', [(1, 8), (1, 23), (1, 24), (2, 22), (2, 24), (3, 39),
+                                         (3, 40)])
+@pytest.mark.parametrize('lam', [.5, 40.])
+def test_deferred_forms_match_oracle(gpu, how, nvar, nsteps, lam):
+    _check(how, nvar, np.linspace(0., 1., nsteps + 1), np.array([0., 1.]), lam, 1)
+
+
+def _check(how, nvar, grid, tt, lam, deferred):
+    vshape = () if nvar == 1 else (nvar,)
     jump = dict(lam=lam, a=-.01, b=.02)
     anti = how == 'antithetic'
     info, ref_info = {}, {}
@@ -28,7 +40,7 @@ def test_forms_match_oracle(gpu, how, nvar, nsteps, lam):
         dw=sa.odd_wiener_source if anti else None, rng=np.random.default_rng(9), **jump)
     dw, dj = p.sources['dw'], p.sources['dj']
     run = p.prepare(tt, moments=how == 'moments')
-    assert all(q.jump_defer == 0 for ps in run.passes for q in ps.probs)
+    assert all(q.jump_defer == deferred for ps in run.passes for q in ps.probs)
     assert (run._row_mom is not None) == (how == 'moments')
     x = run.run()
     # of antithetic paths the leading half, whose normals and jumps are a plain run's
