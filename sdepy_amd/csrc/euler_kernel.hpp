@@ -254,22 +254,6 @@ __device__ __forceinline__ void heston_next(T& x, T& y, int& cnt, const HestonRo
   }
 }
 
-// The least of v over a wave whose lanes are all active.
-__device__ __forceinline__ uint32_t wave_least(uint32_t v) {
-  auto step = [&](auto ctrl) {
-    const uint32_t other = (uint32_t)__builtin_amdgcn_update_dpp(
-        -1, (int)v, decltype(ctrl)::value, 0xf, 0xf, false);
-    v = other < v ? other : v;
-  };
-  step(std::integral_constant<int, 0x111>{});  // row_shr:1, 2, 4, 8
-  step(std::integral_constant<int, 0x112>{});
-  step(std::integral_constant<int, 0x114>{});
-  step(std::integral_constant<int, 0x118>{});
-  step(std::integral_constant<int, 0x142>{});  // row_bcast:15, 31
-  step(std::integral_constant<int, 0x143>{});
-  return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
-}
-
 // The word below which every Poisson word of a pass is a count of 0: a word w
 // draws 0 when (w + 0.5) 2^-32 <= exp(-lam |ds|), so every w below the smallest
 // exp(-lam |ds|) 2^32 of the n table rows does, whatever its step; words
@@ -278,30 +262,20 @@ __device__ __forceinline__ uint32_t wave_least(uint32_t v) {
 // uniform, selecting the sum and counting took a dozen instructions: Merton
 // 2M x 252 FP32, 2 rows 691 -> 562 us, 253 rows 1087 -> 964 us (a bound per
 // step, from the table or beside it, cost more than it saved).  Every thread
-// of the block must call it.  Up to 256 rows each wave reads them all, four loads at
-// once and no barrier: 12 to 24 steps 1 to 2% faster than with FP64 shuffles and a
-// barrier.
+// of the block must call it.
 __device__ __forceinline__ uint32_t zero_count_bound(const double* __restrict__ pois, int64_t n,
                                                      unsigned threads = kBlock) {
-  auto of_row = [&](int64_t i) -> uint32_t {
-    const double b = pois[2 * i + 1] * 0x1p32;
-    return b < 0x1p32 ? (uint32_t)b : 0xFFFFFFFFu;
-  };
-  uint32_t least = 0xFFFFFFFFu;
-  if (n <= 256) {
-    const int64_t lane = threadIdx.x & 63;
+  __shared__ double sh[16];
+  double p = 1.0;
+  for (int64_t i = threadIdx.x; i < n; i += threads) p = fmin(p, pois[2 * i + 1]);
 #pragma unroll
-    for (int k = 0; k < 4; ++k)
-      if (lane + 64 * k < n) least = min(least, of_row(lane + 64 * k));
-    return wave_least(least);
-  }
-  __shared__ uint32_t sh[16];
-  for (int64_t i = threadIdx.x; i < n; i += threads) least = min(least, of_row(i));
-  least = wave_least(least);
-  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = least;
+  for (int off = 32; off > 0; off >>= 1) p = fmin(p, __shfl_xor(p, off, 64));
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = p;
   __syncthreads();
-  for (unsigned w = 0; w < threads >> 6; ++w) least = min(least, sh[w]);
-  return __builtin_amdgcn_readfirstlane(least);
+  for (unsigned w = 0; w < threads >> 6; ++w) p = fmin(p, sh[w]);
+  const double b = p * 0x1p32;
+  const uint32_t bound = b < 0x1p32 ? (uint32_t)b : 0xFFFFFFFFu;
+  return __builtin_amdgcn_readfirstlane(bound);
 }
 
 // Heston working state (SDEs.pack, integration.py:1759-1783, with the two
