@@ -240,6 +240,8 @@ extern "C" int sdegpu_euler(const sdegpu_euler_problem* pr, void* stream) {
                    : pr->dtype == SDEGPU_F64 ? 64 * wide_shape<double>(pr->model, m).waves
                                              : 64 * wide_shape<float>(pr->model, m).waves);
   const bool wide_gen = pr->replay_dw || pr->replay_dj || pp || (jump && pr->lam_paths);
+  const bool wide_stream =
+      (pr->paths * (pr->dtype == SDEGPU_F64 ? 8 : 4)) % 64 == 0 && (uintptr_t)pr->out % 64 == 0;
   hipStream_t st = (hipStream_t)stream;
   // runs of few paths: several waves share 64 paths
   const bool can_split = !wide && !mom && !pp && !grouped && !pr->replay_dw && !pr->replay_dj &&
@@ -260,13 +262,13 @@ extern "C" int sdegpu_euler(const sdegpu_euler_problem* pr, void* stream) {
     }
   }
   if (pr->dtype == SDEGPU_F32) {
-    EulerKernel<float> k = wide ? euler_wide_kernel<float>(pr->model, m, wide_gen)
+    EulerKernel<float> k = wide ? euler_wide_kernel<float>(pr->model, m, wide_gen, wide_stream)
                                 : choose<float>(plain, mom, pp, pr->model, m, hd, form);
     if (!k) return fail(SDEGPU_EUNSUPPORTED, "no kernel for model %d with %d components", pr->model, m);
     hipLaunchKernelGGL(k, grid, block, 0, st, a, (const float*)pr->coef, pr->store_row,
                        pr->pois, (float*)pr->out);
   } else {
-    EulerKernel<double> k = wide ? euler_wide_kernel<double>(pr->model, m, wide_gen)
+    EulerKernel<double> k = wide ? euler_wide_kernel<double>(pr->model, m, wide_gen, wide_stream)
                                  : choose<double>(plain, mom, pp, pr->model, m, hd, form);
     if (!k) return fail(SDEGPU_EUNSUPPORTED, "no kernel for model %d with %d components", pr->model, m);
     hipLaunchKernelGGL(k, grid, block, 0, st, a, (const double*)pr->coef, pr->store_row,

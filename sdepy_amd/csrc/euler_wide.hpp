@@ -78,7 +78,15 @@ constexpr int wide_occupancy() {
 }
 
 // GEN: recorded increments, per-path parameters and per-path intensities.
-template <int MODEL, typename T, int W, int R, bool GEN>
+//
+// STREAM: rows begin on 64-byte lines, and the stores stream past the L2.
+// Where they don't, every wave's 64 values share their first and last line with the
+// neighbouring blocks', and streamed one by one those halves are
+// written back alone: 400,003 paths of 12 FP32 OU components x 13, 14 rows 161 us, 81 by
+// plain stores that the L2 joins (400,000 paths: 81 and 83; 1,636,947: 631 and 307).  So that
+// neighbours meet in one L2, XCD x (blockIdx.x mod 8) steps the x-th eighth of the blocks;
+// without that the 1,636,947 paths take 492.  Streamed rows are 1 to 2% slower in that order.
+template <int MODEL, typename T, int W, int R, bool GEN, bool STREAM>
 __global__ __launch_bounds__(64 * W, (wide_occupancy<MODEL, T, W, R, GEN>())) void k_euler_wide(const EulerArgs a,
                                                        const T* __restrict__ coef,
                                                        const int32_t* __restrict__ store_row,
@@ -103,6 +111,10 @@ __global__ __launch_bounds__(64 * W, (wide_occupancy<MODEL, T, W, R, GEN>())) vo
 
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // the block's place among the paths (the last few, past whole eighths, keep theirs)
+  const unsigned eighth = STREAM ? 0u : gridDim.x >> 3;
+  const unsigned blk = blockIdx.x < 8u * eighth ? (blockIdx.x & 7u) * eighth + (blockIdx.x >> 3)
+                                                : blockIdx.x;
   // A lane draws for path `lane` of the block and steps the state of path `pl`.
   const int quad = lane >> 4;
   const int pl = kMat ? 16 * (w & 3) + (lane & 15) : lane;
@@ -160,7 +172,7 @@ __global__ __launch_bounds__(64 * W, (wide_occupancy<MODEL, T, W, R, GEN>())) vo
   };
 
   const int64_t P = a.paths;
-  const int64_t tid = (int64_t)blockIdx.x * 64 + pl;
+  const int64_t tid = (int64_t)blk * 64 + pl;
   // lanes beyond the last path step a copy of it and store nothing
   const bool live = tid < P;
   const int64_t gid = live ? tid : P - 1;
@@ -169,7 +181,7 @@ __global__ __launch_bounds__(64 * W, (wide_occupancy<MODEL, T, W, R, GEN>())) vo
   };
   const uint32_t path_j = jump_path(gid);
   // the path that the lane draws for
-  const int64_t did = min((int64_t)blockIdx.x * 64 + lane, P - 1);
+  const int64_t did = min((int64_t)blk * 64 + lane, P - 1);
   const bool flip_w = a.anti_w > 0 && did >= a.anti_w;
   const uint32_t path_w = (uint32_t)(flip_w ? did - a.anti_w : did);
   const uint32_t path_p = jump_path(did);
@@ -204,6 +216,12 @@ __global__ __launch_bounds__(64 * W, (wide_occupancy<MODEL, T, W, R, GEN>())) vo
   for (int r = 0; r < R; ++r) cnt[r] = 0;
   int interval_jumps = 0;
 
+  auto put = [&](T v, T* at) {
+    if constexpr (STREAM)
+      __builtin_nontemporal_store(v, at);
+    else
+      *at = v;
+  };
   // Every thread of the block must call it.
   auto store = [&](int row) {
     T* o_row = out + ((int64_t)row * a.out_stride + a.out0) * P + gid;
@@ -215,10 +233,10 @@ __global__ __launch_bounds__(64 * W, (wide_occupancy<MODEL, T, W, R, GEN>())) vo
       for (int r = 0; r < R; ++r)
         if (has(r)) z[0][comp(r)][pl] = x[r];
       __syncthreads();
-      if (w == 0 && (int64_t)blockIdx.x * 64 + lane < P) {
+      if (w == 0 && (int64_t)blk * 64 + lane < P) {
         T val = (T)0;
         for (int v = 0; v < m; ++v) val = val + z[0][v][lane];
-        __builtin_nontemporal_store(val, o_row - gid + did);
+        put(val, o_row - gid + did);
       }
       return;
     }
@@ -228,12 +246,12 @@ __global__ __launch_bounds__(64 * W, (wide_occupancy<MODEL, T, W, R, GEN>())) vo
     for (int r = 0; r < R; ++r) {
       if (!has(r)) break;
       if constexpr (kHeston) {
-        __builtin_nontemporal_store((T)exp(x[r]), o);
-        if (a.nout == m) __builtin_nontemporal_store(vy[r], o + n * P);
+        put((T)exp(x[r]), o);
+        if (a.nout == m) put(vy[r], o + n * P);
       } else if (comp(r) < a.nout) {
         T val = x[r];
         if constexpr (OutRule<MODEL>::exp_all) val = exp(val);
-        __builtin_nontemporal_store(val, o);
+        put(val, o);
       }
       o += W * P;
     }
@@ -529,9 +547,9 @@ inline WideShape wide_shape(int model, int m) {
 // k_euler_wide and k_wiener_fill_wide instances (euler_wide_f32.hip,
 // euler_wide_f64.hip): the kernel for a model and a width of 9..64, or null.
 // Blocks of 64 * wide_shape<T>(model, m).waves threads, one per 64 paths; gen: recorded
-// increments, per-path parameters or intensities.
+// increments, per-path parameters or intensities (plain stores only); stream: rows of whole 64-byte lines.
 template <typename T>
-EulerKernel<T> euler_wide_kernel(int model, int m, bool gen);
+EulerKernel<T> euler_wide_kernel(int model, int m, bool gen, bool stream);
 
 template <typename T>
 using WienerFillWide = void (*)(uint32_t, uint32_t, uint32_t, uint32_t, int64_t, int64_t,
@@ -539,78 +557,79 @@ using WienerFillWide = void (*)(uint32_t, uint32_t, uint32_t, uint32_t, int64_t,
 template <typename T>
 WienerFillWide<T> wiener_fill_wide_kernel(int m);
 template <>
-EulerKernel<float> euler_wide_kernel<float>(int model, int m, bool gen);
+EulerKernel<float> euler_wide_kernel<float>(int model, int m, bool gen, bool stream);
 template <>
-EulerKernel<double> euler_wide_kernel<double>(int model, int m, bool gen);
+EulerKernel<double> euler_wide_kernel<double>(int model, int m, bool gen, bool stream);
 template <>
 WienerFillWide<float> wiener_fill_wide_kernel<float>(int m);
 template <>
 WienerFillWide<double> wiener_fill_wide_kernel<double>(int m);
 
-template <int MODEL, typename T, bool GEN>
+template <int MODEL, typename T, bool GEN, bool STREAM>
 EulerKernel<T> pick_wide(int m) {
   const WideShape s = wide_shape<T>(MODEL, m);
   const int key = s.waves * 16 + s.rows;
   if constexpr (MODEL == SDEGPU_MODEL_HESTON && kWideMat<T>) {
     switch (key) {
-      case 4 * 16 + 2: return k_euler_wide<MODEL, T, 4, 2, GEN>;
-      case 4 * 16 + 3: return k_euler_wide<MODEL, T, 4, 3, GEN>;
-      case 4 * 16 + 4: return k_euler_wide<MODEL, T, 4, 4, GEN>;
-      case 8 * 16 + 3: return k_euler_wide<MODEL, T, 8, 3, GEN>;
-      case 8 * 16 + 4: return k_euler_wide<MODEL, T, 8, 4, GEN>;
+      case 4 * 16 + 2: return k_euler_wide<MODEL, T, 4, 2, GEN, STREAM>;
+      case 4 * 16 + 3: return k_euler_wide<MODEL, T, 4, 3, GEN, STREAM>;
+      case 4 * 16 + 4: return k_euler_wide<MODEL, T, 4, 4, GEN, STREAM>;
+      case 8 * 16 + 3: return k_euler_wide<MODEL, T, 8, 3, GEN, STREAM>;
+      case 8 * 16 + 4: return k_euler_wide<MODEL, T, 8, 4, GEN, STREAM>;
       default: return nullptr;
     }
   } else if constexpr (MODEL == SDEGPU_MODEL_HESTON) {
     switch (key) {
-      case 2 * 16 + 3: return k_euler_wide<MODEL, T, 2, 3, GEN>;
-      case 2 * 16 + 4: return k_euler_wide<MODEL, T, 2, 4, GEN>;
-      case 3 * 16 + 4: return k_euler_wide<MODEL, T, 3, 4, GEN>;
-      case 4 * 16 + 4: return k_euler_wide<MODEL, T, 4, 4, GEN>;
-      case 6 * 16 + 4: return k_euler_wide<MODEL, T, 6, 4, GEN>;
-      case 8 * 16 + 4: return k_euler_wide<MODEL, T, 8, 4, GEN>;
+      case 2 * 16 + 3: return k_euler_wide<MODEL, T, 2, 3, GEN, STREAM>;
+      case 2 * 16 + 4: return k_euler_wide<MODEL, T, 2, 4, GEN, STREAM>;
+      case 3 * 16 + 4: return k_euler_wide<MODEL, T, 3, 4, GEN, STREAM>;
+      case 4 * 16 + 4: return k_euler_wide<MODEL, T, 4, 4, GEN, STREAM>;
+      case 6 * 16 + 4: return k_euler_wide<MODEL, T, 6, 4, GEN, STREAM>;
+      case 8 * 16 + 4: return k_euler_wide<MODEL, T, 8, 4, GEN, STREAM>;
       default: return nullptr;
     }
   } else if constexpr (kWideMat<T>) {
     switch (key) {
-      case 4 * 16 + 3: return k_euler_wide<MODEL, T, 4, 3, GEN>;
-      case 4 * 16 + 4: return k_euler_wide<MODEL, T, 4, 4, GEN>;
-      case 4 * 16 + 5: return k_euler_wide<MODEL, T, 4, 5, GEN>;
-      case 4 * 16 + 6: return k_euler_wide<MODEL, T, 4, 6, GEN>;
-      case 8 * 16 + 4: return k_euler_wide<MODEL, T, 8, 4, GEN>;
-      case 8 * 16 + 6: return k_euler_wide<MODEL, T, 8, 6, GEN>;
-      case 8 * 16 + 8: return k_euler_wide<MODEL, T, 8, 8, GEN>;
+      case 4 * 16 + 3: return k_euler_wide<MODEL, T, 4, 3, GEN, STREAM>;
+      case 4 * 16 + 4: return k_euler_wide<MODEL, T, 4, 4, GEN, STREAM>;
+      case 4 * 16 + 5: return k_euler_wide<MODEL, T, 4, 5, GEN, STREAM>;
+      case 4 * 16 + 6: return k_euler_wide<MODEL, T, 4, 6, GEN, STREAM>;
+      case 8 * 16 + 4: return k_euler_wide<MODEL, T, 8, 4, GEN, STREAM>;
+      case 8 * 16 + 6: return k_euler_wide<MODEL, T, 8, 6, GEN, STREAM>;
+      case 8 * 16 + 8: return k_euler_wide<MODEL, T, 8, 8, GEN, STREAM>;
       default: return nullptr;
     }
   } else {
     switch (key) {
-      case 2 * 16 + 6: return k_euler_wide<MODEL, T, 2, 6, GEN>;
-      case 2 * 16 + 8: return k_euler_wide<MODEL, T, 2, 8, GEN>;
-      case 3 * 16 + 7: return k_euler_wide<MODEL, T, 3, 7, GEN>;
-      case 3 * 16 + 8: return k_euler_wide<MODEL, T, 3, 8, GEN>;
-      case 4 * 16 + 8: return k_euler_wide<MODEL, T, 4, 8, GEN>;
-      case 6 * 16 + 8: return k_euler_wide<MODEL, T, 6, 8, GEN>;
-      case 8 * 16 + 8: return k_euler_wide<MODEL, T, 8, 8, GEN>;
+      case 2 * 16 + 6: return k_euler_wide<MODEL, T, 2, 6, GEN, STREAM>;
+      case 2 * 16 + 8: return k_euler_wide<MODEL, T, 2, 8, GEN, STREAM>;
+      case 3 * 16 + 7: return k_euler_wide<MODEL, T, 3, 7, GEN, STREAM>;
+      case 3 * 16 + 8: return k_euler_wide<MODEL, T, 3, 8, GEN, STREAM>;
+      case 4 * 16 + 8: return k_euler_wide<MODEL, T, 4, 8, GEN, STREAM>;
+      case 6 * 16 + 8: return k_euler_wide<MODEL, T, 6, 8, GEN, STREAM>;
+      case 8 * 16 + 8: return k_euler_wide<MODEL, T, 8, 8, GEN, STREAM>;
       default: return nullptr;
     }
   }
 }
 
 template <int MODEL, typename T>
-EulerKernel<T> pick_wide(int m, bool gen) {
-  return gen ? pick_wide<MODEL, T, true>(m) : pick_wide<MODEL, T, false>(m);
+EulerKernel<T> pick_wide(int m, bool gen, bool stream) {
+  if (gen) return pick_wide<MODEL, T, true, false>(m);
+  return stream ? pick_wide<MODEL, T, false, true>(m) : pick_wide<MODEL, T, false, false>(m);
 }
 
 #define SDEGPU_EULER_WIDE_SET(T)                                                         \
   template <>                                                                            \
-  EulerKernel<T> euler_wide_kernel<T>(int model, int m, bool gen) {                      \
+  EulerKernel<T> euler_wide_kernel<T>(int model, int m, bool gen, bool stream) {         \
     if (m <= SDEGPU_MAX_VARS || m > SDEGPU_MAX_COUPLED) return nullptr;                  \
     switch (model) {                                                                     \
-      case SDEGPU_MODEL_WIENER: return pick_wide<SDEGPU_MODEL_WIENER, T>(m, gen);        \
-      case SDEGPU_MODEL_LOGNORM: return pick_wide<SDEGPU_MODEL_LOGNORM, T>(m, gen);      \
-      case SDEGPU_MODEL_OU: return pick_wide<SDEGPU_MODEL_OU, T>(m, gen);                \
-      case SDEGPU_MODEL_CIR: return pick_wide<SDEGPU_MODEL_CIR, T>(m, gen);              \
-      case SDEGPU_MODEL_HESTON: return pick_wide<SDEGPU_MODEL_HESTON, T>(m, gen);        \
-      case SDEGPU_MODEL_JUMPDIFF: return pick_wide<SDEGPU_MODEL_JUMPDIFF, T>(m, gen);    \
+      case SDEGPU_MODEL_WIENER: return pick_wide<SDEGPU_MODEL_WIENER, T>(m, gen, stream);\
+      case SDEGPU_MODEL_LOGNORM: return pick_wide<SDEGPU_MODEL_LOGNORM, T>(m, gen, stream);\
+      case SDEGPU_MODEL_OU: return pick_wide<SDEGPU_MODEL_OU, T>(m, gen, stream);        \
+      case SDEGPU_MODEL_CIR: return pick_wide<SDEGPU_MODEL_CIR, T>(m, gen, stream);      \
+      case SDEGPU_MODEL_HESTON: return pick_wide<SDEGPU_MODEL_HESTON, T>(m, gen, stream);\
+      case SDEGPU_MODEL_JUMPDIFF: return pick_wide<SDEGPU_MODEL_JUMPDIFF, T>(m, gen, stream);\
       default: return nullptr;                                                           \
     }                                                                                    \
   }                                                                                      \

@@ -59,3 +59,34 @@ def test_sixteen_path_groups(gpu, m, P):
                         info=ref_info, x0=1., mu=.03, sigma=.2)
     assert np.array_equal(info['jump_count'], ref_info['jump_count'])
     assert np.max(np.abs(got / ref - 1)) < 1e-12
+
+
+@pytest.mark.parametrize('dtype', [np.float64, np.float32])
+@pytest.mark.parametrize('cls,kw', [
+    (sa.lognorm_process, dict(vshape=9, mu=.05, sigma=.2)),
+    (sa.hull_white_process, dict(factors=12, k=.2, sigma=.01)),
+    (sa.full_heston_process, dict(vshape=5, y0=.04, theta=.05, k=2., xi=.3, rho=np.full(5, -.5))),
+    (sa.merton_jumpdiff_process, dict(vshape=10, lam=3., a=-.05, b=.1))])
+def test_order_of_blocks_and_rows_of_partial_lines(gpu, dtype, cls, kw):
+    """Block counts around the eights that share an L2, rows on and off 64-byte lines:
+    every path, and its counts, as in a run of more paths."""
+    tt = np.linspace(0., 1., 4)
+    m = kw.get('vshape', kw.get('factors'))
+    if cls is not sa.full_heston_process:
+        kw = dict(kw, corr=.9 * np.eye(m) + .1)
+
+    def run(paths):
+        info = {}
+        x = cls(paths=paths, dtype=dtype, steps=13, info=info, rng=np.random.default_rng(3),
+                **kw)(tt)
+        return (x if isinstance(x, tuple) else (x,)), info
+    ref, ref_info = run(1600)
+    for paths in (1, 63, 448, 511, 512, 513, 529, 1024, 1087):
+        got, info = run(paths)
+        for g, r in zip(got, ref):
+            r = r[..., :paths]
+            assert np.max(np.abs(g - r)) <= (1e-12 if dtype == np.float64 else 2e-5) * \
+                np.max(np.abs(r))
+        for key in ('negative_y_count', 'jump_count'):
+            if key in info:
+                assert np.array_equal(info[key], ref_info[key][..., :paths])
