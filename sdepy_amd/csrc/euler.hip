@@ -63,7 +63,7 @@ static int split_waves(int64_t paths, int model) {
   constexpr int64_t kSimds = 1024;
   const int64_t waves = (paths + 63) / 64;
   if (waves > kSimds) return 1;
-  const bool root = model == SDEGPU_MODEL_HESTON || model == SDEGPU_MODEL_CIR;
+  const bool root = split_root(model);
   const int64_t room = (root ? 2 : 4) * kSimds / waves;
   return room >= 8 ? 8 : room >= 4 ? 4 : 2;
 }
@@ -240,7 +240,8 @@ extern "C" int sdegpu_euler(const sdegpu_euler_problem* pr, void* stream) {
                    : pr->dtype == SDEGPU_F64 ? 64 * wide_shape<double>(pr->model, m).waves
                                              : 64 * wide_shape<float>(pr->model, m).waves);
   const bool wide_gen = pr->replay_dw || pr->replay_dj || pp || (jump && pr->lam_paths);
-  const bool wide_stream =
+  // every row of a value begins on a 64-byte line
+  const bool lines =
       (pr->paths * (pr->dtype == SDEGPU_F64 ? 8 : 4)) % 64 == 0 && (uintptr_t)pr->out % 64 == 0;
   hipStream_t st = (hipStream_t)stream;
   // runs of few paths: several waves share 64 paths
@@ -250,25 +251,25 @@ extern "C" int sdegpu_euler(const sdegpu_euler_problem* pr, void* stream) {
   if (share > 1) {
     const dim3 sgrid(blocks_for(pr->paths, 64)), sblock(64 * share);
     if (pr->dtype == SDEGPU_F32) {
-      if (EulerKernel<float> k = euler_split_kernel<float>(pr->model, m, hd, sgrid.x)) {
+      if (EulerKernel<float> k = euler_split_kernel<float>(pr->model, m, hd, sgrid.x, lines)) {
         hipLaunchKernelGGL(k, sgrid, sblock, 0, st, a, (const float*)pr->coef, pr->store_row,
                            pr->pois, (float*)pr->out);
         return launch_status("k_euler_split");
       }
-    } else if (EulerKernel<double> k = euler_split_kernel<double>(pr->model, m, hd, sgrid.x)) {
+    } else if (EulerKernel<double> k = euler_split_kernel<double>(pr->model, m, hd, sgrid.x, lines)) {
       hipLaunchKernelGGL(k, sgrid, sblock, 0, st, a, (const double*)pr->coef, pr->store_row,
                          pr->pois, (double*)pr->out);
       return launch_status("k_euler_split");
     }
   }
   if (pr->dtype == SDEGPU_F32) {
-    EulerKernel<float> k = wide ? euler_wide_kernel<float>(pr->model, m, wide_gen, wide_stream)
+    EulerKernel<float> k = wide ? euler_wide_kernel<float>(pr->model, m, wide_gen, lines)
                                 : choose<float>(plain, mom, pp, pr->model, m, hd, form);
     if (!k) return fail(SDEGPU_EUNSUPPORTED, "no kernel for model %d with %d components", pr->model, m);
     hipLaunchKernelGGL(k, grid, block, 0, st, a, (const float*)pr->coef, pr->store_row,
                        pr->pois, (float*)pr->out);
   } else {
-    EulerKernel<double> k = wide ? euler_wide_kernel<double>(pr->model, m, wide_gen, wide_stream)
+    EulerKernel<double> k = wide ? euler_wide_kernel<double>(pr->model, m, wide_gen, lines)
                                  : choose<double>(plain, mom, pp, pr->model, m, hd, form);
     if (!k) return fail(SDEGPU_EUNSUPPORTED, "no kernel for model %d with %d components", pr->model, m);
     hipLaunchKernelGGL(k, grid, block, 0, st, a, (const double*)pr->coef, pr->store_row,

@@ -322,7 +322,7 @@ __device__ __forceinline__ void store_lane_nt(T* base, uint32_t off, T v) {
 // Non-temporal stores: the output is not read again by this kernel.  Lanes
 // without a path (live false, MOM instances only) store nothing; with MOM
 // every stored value also goes to its LDS column (mcol + o * kMomStride).
-template <int MODEL, typename T, int M, int D, bool GRP, bool MOM>
+template <int MODEL, typename T, int M, int D, bool GRP, bool MOM, bool STREAM = true>
 __device__ __forceinline__ void store_state(T* __restrict__ out, const EulerArgs& a, int row,
                                             const T (&x)[M], int64_t gid, bool live, T* mcol) {
   const int64_t P = a.paths;
@@ -341,8 +341,10 @@ __device__ __forceinline__ void store_state(T* __restrict__ out, const EulerArgs
     if constexpr (MOM) {
       if (live) store_lane_nt(o_blk + o * P, lane_bytes, v);
       mcol[o * kMomStride] = v;
-    } else {
+    } else if constexpr (STREAM) {
       __builtin_nontemporal_store(v, o_row + o * P);
+    } else {
+      o_row[o * P] = v;
     }
   };
   if constexpr (MODEL == SDEGPU_MODEL_HESTON) {

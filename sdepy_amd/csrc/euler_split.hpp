@@ -41,7 +41,12 @@ struct Count {
   static constexpr int value = K;
 };
 
-template <int MODEL, typename T, int M, int D, int MOST = 8>
+// STREAM: rows begin on 64-byte lines, and the stores stream past the L2.
+// Where they don't, the halves of the lines that neighbouring blocks share are joined
+// in the L2 (as in k_euler_wide): 4 OU components FP32 64,999 x 250, every step stored,
+// 121 us alone, 162 streamed, 100 so; lognormal 162 and 98.  FP64 Heston and CIR, whose
+// lines are further apart in time, are up to 20% slower so and always stream.
+template <int MODEL, typename T, int M, int D, bool STREAM, int MOST = 8>
 __global__ __launch_bounds__(64 * MOST) void k_euler_split(
     const EulerArgs a, const T* __restrict__ coef, const int32_t* __restrict__ store_row,
     const double* __restrict__ pois, T* __restrict__ out) {
@@ -65,7 +70,12 @@ __global__ __launch_bounds__(64 * MOST) void k_euler_split(
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t P = a.paths;
-  const int64_t tid = (int64_t)blockIdx.x * 64 + lane;
+  // the block's place among the paths: XCD x takes the x-th eighth of the blocks (the last few,
+  // past whole eighths, keep theirs)
+  const unsigned eighth = STREAM ? 0u : gridDim.x >> 3;
+  const unsigned blk = blockIdx.x < 8u * eighth ? (blockIdx.x & 7u) * eighth + (blockIdx.x >> 3)
+                                                : blockIdx.x;
+  const int64_t tid = (int64_t)blk * 64 + lane;
   // lanes beyond the last path step a copy of it and store nothing
   const bool live = tid < P;
   const int64_t gid = live ? tid : P - 1;
@@ -88,7 +98,8 @@ __global__ __launch_bounds__(64 * MOST) void k_euler_split(
   for (int v = 0; v < M; ++v) cnt[v] = 0;
   int interval_jumps = 0;
   auto store = [&](int row) {
-    if (live) store_state<MODEL, T, M, D, false, false>(out, a, row, x, gid, true, (T*)nullptr);
+    if (live)
+      store_state<MODEL, T, M, D, false, false, STREAM>(out, a, row, x, gid, true, (T*)nullptr);
   };
   if (a.row0 >= 0 && w == 0) store(a.row0);
 
@@ -275,48 +286,60 @@ __global__ __launch_bounds__(64 * MOST) void k_euler_split(
 }
 
 template <typename T>
-EulerKernel<T> euler_split_kernel(int model, int m, int d, int64_t blocks);
+EulerKernel<T> euler_split_kernel(int model, int m, int d, int64_t blocks, bool stream);
 template <>
-EulerKernel<float> euler_split_kernel<float>(int model, int m, int d, int64_t blocks);
+EulerKernel<float> euler_split_kernel<float>(int model, int m, int d, int64_t blocks, bool stream);
 template <>
-EulerKernel<double> euler_split_kernel<double>(int model, int m, int d, int64_t blocks);
+EulerKernel<double> euler_split_kernel<double>(int model, int m, int d, int64_t blocks,
+                                               bool stream);
 
-template <int MODEL, typename T, int MAX, int MOST = 8>
+template <int MODEL, typename T, bool STREAM, int MAX, int MOST = 8>
 EulerKernel<T> pick_split(int m) {
-  if (m == 1) return k_euler_split<MODEL, T, 1, 1, MOST>;
-  if (m == 2) return k_euler_split<MODEL, T, 2, 1, MOST>;
+  if (m == 1) return k_euler_split<MODEL, T, 1, 1, STREAM, MOST>;
+  if (m == 2) return k_euler_split<MODEL, T, 2, 1, STREAM, MOST>;
   if constexpr (MAX > 2) {
-    if (m == 3) return k_euler_split<MODEL, T, 3, 1, MOST>;
-    if (m == 4) return k_euler_split<MODEL, T, 4, 1, MOST>;
+    if (m == 3) return k_euler_split<MODEL, T, 3, 1, STREAM, MOST>;
+    if (m == 4) return k_euler_split<MODEL, T, 4, 1, STREAM, MOST>;
   }
   return nullptr;
 }
 
-template <typename T>
-EulerKernel<T> pick_split_jump(int m, int64_t blocks) {
-  // (split_waves gives such grids 4 waves a block at most)
-  if (sizeof(T) == 8 && blocks > 3 * 256) return pick_split<SDEGPU_MODEL_JUMPDIFF, T, 2, 4>(m);
-  return pick_split<SDEGPU_MODEL_JUMPDIFF, T, 2>(m);
+// Models whose recursion takes a square root.
+constexpr bool split_root(int model) {
+  return model == SDEGPU_MODEL_CIR || model == SDEGPU_MODEL_HESTON;
 }
 
-// The kernel for a model, its components m, Heston's group width d and the
-// blocks of the grid, or null (euler_split_f32.hip, euler_split_f64.hip).
-#define SDEGPU_EULER_SPLIT_SET(T)                                                       \
-  template <>                                                                           \
-  EulerKernel<T> euler_split_kernel<T>(int model, int m, int d, int64_t blocks) {       \
-    switch (model) {                                                                    \
-      case SDEGPU_MODEL_WIENER: return pick_split<SDEGPU_MODEL_WIENER, T, 4>(m);        \
-      case SDEGPU_MODEL_LOGNORM: return pick_split<SDEGPU_MODEL_LOGNORM, T, 4>(m);      \
-      case SDEGPU_MODEL_OU: return pick_split<SDEGPU_MODEL_OU, T, 4>(m);                \
-      case SDEGPU_MODEL_CIR: return pick_split<SDEGPU_MODEL_CIR, T, 4>(m);              \
-      case SDEGPU_MODEL_JUMPDIFF: return pick_split_jump<T>(m, blocks);                 \
-      case SDEGPU_MODEL_HESTON:                                                         \
-        if (m == 2) return k_euler_split<SDEGPU_MODEL_HESTON, T, 2, 1>;                 \
-        if (m == 4 && d == 1) return k_euler_split<SDEGPU_MODEL_HESTON, T, 4, 1>;       \
-        if (m == 4 && d == 2) return k_euler_split<SDEGPU_MODEL_HESTON, T, 4, 2>;       \
-        return nullptr;                                                                 \
-      default: return nullptr;                                                          \
-    }                                                                                   \
+template <typename T, bool STREAM>
+EulerKernel<T> pick_split(int model, int m, int d, int64_t blocks) {
+  constexpr bool kRootStream = STREAM || sizeof(T) == 8;
+  switch (model) {
+    case SDEGPU_MODEL_WIENER: return pick_split<SDEGPU_MODEL_WIENER, T, STREAM, 4>(m);
+    case SDEGPU_MODEL_LOGNORM: return pick_split<SDEGPU_MODEL_LOGNORM, T, STREAM, 4>(m);
+    case SDEGPU_MODEL_OU: return pick_split<SDEGPU_MODEL_OU, T, STREAM, 4>(m);
+    case SDEGPU_MODEL_CIR: return pick_split<SDEGPU_MODEL_CIR, T, kRootStream, 4>(m);
+    case SDEGPU_MODEL_JUMPDIFF:
+      // (split_waves gives such grids 4 waves a block at most)
+      if (sizeof(T) == 8 && blocks > 3 * 256)
+        return pick_split<SDEGPU_MODEL_JUMPDIFF, T, STREAM, 2, 4>(m);
+      return pick_split<SDEGPU_MODEL_JUMPDIFF, T, STREAM, 2>(m);
+    case SDEGPU_MODEL_HESTON:
+      if (m == 2) return k_euler_split<SDEGPU_MODEL_HESTON, T, 2, 1, kRootStream>;
+      if (m == 4 && d == 1) return k_euler_split<SDEGPU_MODEL_HESTON, T, 4, 1, kRootStream>;
+      if (m == 4 && d == 2) return k_euler_split<SDEGPU_MODEL_HESTON, T, 4, 2, kRootStream>;
+      return nullptr;
+    default: return nullptr;
+  }
+}
+
+// The kernel for a model, its components m, Heston's group width d, the blocks of the
+// grid and rows that begin on 64-byte lines or don't, or null (euler_split_f32.hip,
+// euler_split_f64.hip).
+#define SDEGPU_EULER_SPLIT_SET(T)                                                         \
+  template <>                                                                             \
+  EulerKernel<T> euler_split_kernel<T>(int model, int m, int d, int64_t blocks,           \
+                                       bool stream) {                                     \
+    return stream ? pick_split<T, true>(model, m, d, blocks)                              \
+                  : pick_split<T, false>(model, m, d, blocks);                            \
   }
 
 }  // namespace sdegpu
