@@ -51,18 +51,25 @@ static uint32_t expected_exp_mask(int model, int m, int nout, int d) {
 // Twice the share for the models whose recursion is a sum or an FMA: 4096
 // waves for them, 2048 for Heston and CIR, whose every wave repeats a square
 // root per step.  Microseconds for 252 steps alone / with 2, 4, 8 waves:
-//   lognormal FP64, 253 rows   10,000 paths  79 / 53, 32, 25
-//                              32,768        79 / 67, 40, 36
-//                              65,536        78 / 66, 60, 63
-//   Heston FP64, 253 rows      10,000       160 / 115, 79, 77
-//                              32,768       159 / 141, 99, 119
-//                              65,536       160 / 142, 159, 223
-//   Kou FP32, 2 rows           10,000        62 / 52, 35, 28
-//                              65,536        63 / 59, 50, 56
-static int split_waves(int64_t paths, int model) {
+//   lognormal FP64, 253 rows   16,000 paths  64 / 53, 33, 26
+//                              32,000        65 / 66, 39, 35
+//                              65,000        64 / 66, 58, 61
+//   Heston FP64, 253 rows      16,000       120 / 115, 79, 77
+//                              32,000       119 / 141, 97, 118
+//                              65,000       120 / 141, 154, 221
+//   Merton FP32, 2 rows        16,000        53 / 55, 37, 29
+//                              65,000        54 / 62, 53, 59
+// (12, 20, 32, 60 and 120 steps give the same shares, less a launch of some 7 us.)
+// Heston of one pair is alone above 512 waves: k_euler reads its constants from
+// LDS.  So are three FP64 CIR components above 768 (53 KB of LDS, three
+// blocks per CU): 65,000 paths, 2 rows, 165 alone, 249 with 2 waves; 32,000 164 alone,
+// 117 with 4.
+static int split_waves(int64_t paths, int model, int dtype, int m) {
   constexpr int64_t kSimds = 1024;
   const int64_t waves = (paths + 63) / 64;
   if (waves > kSimds) return 1;
+  if (model == SDEGPU_MODEL_HESTON && m == 2 && waves > kSimds / 2) return 1;
+  if (model == SDEGPU_MODEL_CIR && dtype == SDEGPU_F64 && m == 3 && waves > 768) return 1;
   const bool root = split_root(model);
   const int64_t room = (root ? 2 : 4) * kSimds / waves;
   return room >= 8 ? 8 : room >= 4 ? 4 : 2;
@@ -247,7 +254,7 @@ extern "C" int sdegpu_euler(const sdegpu_euler_problem* pr, void* stream) {
   // runs of few paths: several waves share 64 paths
   const bool can_split = !wide && !mom && !pp && !grouped && !pr->replay_dw && !pr->replay_dj &&
                          !(jump && pr->lam_paths);
-  const int share = can_split ? split_waves(pr->paths, pr->model) : 1;
+  const int share = can_split ? split_waves(pr->paths, pr->model, pr->dtype, m) : 1;
   if (share > 1) {
     const dim3 sgrid(blocks_for(pr->paths, 64)), sblock(64 * share);
     if (pr->dtype == SDEGPU_F32) {

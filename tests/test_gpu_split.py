@@ -125,3 +125,14 @@ def test_moments_of_few_paths_fused_and_separate(gpu, monkeypatch, paths):
                       (v, fv, x.var(axis=-1, keepdims=True))):
         assert np.allclose(a, ref, rtol=1e-12, atol=1e-14)
         assert np.allclose(b, ref, rtol=1e-12, atol=1e-14)
+
+
+@pytest.mark.parametrize('paths', [49_152, 49_153])
+def test_three_fp64_cir_components(gpu, paths):
+    """On either side of the blocks that three per CU hold at once."""
+    tt, kw = np.array([0., .5, 1.]), dict(x0=.05, theta=.04, k=2., xi=.2)
+    p = sa.cox_ingersoll_ross_process(paths=paths, vshape=3, corr=CORR3, steps=17,
+                                      rng=np.random.default_rng(8), **kw)
+    src = ora.PhiloxWiener(p.sources['dw'].key, 0, 100, (3,), corr=CORR3)
+    ref = ora.integrate('cir', tt, paths=100, vshape=(3,), steps=17, sources={'dw': src}, **kw)
+    assert np.max(np.abs(p(tt)[..., :100] - ref)) < 1e-12
