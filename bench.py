@@ -40,7 +40,7 @@ Printed as one JSON line:
   gbm_c1      GBM 10k x 252 FP64 full path + pmean/pvar (latency-bound):
               kernel time, the end-to-end preset call with the host process's
               pmean/pvar, and the same through prepare(moments=True), whose
-              kernel reduces the rows as it stores them
+              launch reduces the rows right after the kernel stores them
   batched     1024 heterogeneous GBM / HW2F instances in one persistent
               launch; per-instance FP32 moments vs FP64 runs of the same paths;
               VALU issue rate vs the nominal ceiling (SQ_INSTS_VALU per launch
@@ -697,9 +697,9 @@ def main():
             x = c1_proc()(tt1)
             m, v = x.pmean()[-1], x.pvar()[-1]
         e2e = (time.perf_counter() - t0) / reps
-        # the same through a prepared run whose kernel reduces the rows as
-        # it stores them: the path array still comes back to the host, the
-        # moments without another upload or pass
+        # the same through a prepared run whose launch reduces the rows after
+        # the kernel stores them: the path array still comes back to the host,
+        # the moments without an upload
         run = c1_proc().prepare(tt1, moments=True)
         run.run()
         t0 = time.perf_counter()

@@ -446,13 +446,14 @@ typedef struct sdegpu_heston_greeks {
   double strike, maturity;
   uint32_t key[2]; /* Philox key of the dw source */
   uint32_t epoch;
-  int32_t method;  /* 0: reverse-mode adjoint (swept over segments of the path, each
-                      while its partial derivatives are in registers); 1: forward
-                      mode, the derivatives carried along step by step; the same
-                      estimator either way */
+  int32_t method;  /* 0: reverse-mode adjoint (FP64 variance: swept over segments of the
+                      path, each while its partial derivatives are in registers; FP32:
+                      over the whole path, from variance checkpoints every 8 steps and
+                      normals drawn again); 1: forward mode, the derivatives carried
+                      along step by step; the same estimator either way */
   int32_t variance_f64; /* SDEGPU_F32 only, 1: the variance and every derivative in
-                           FP64, the log price, the Philox normals and Box-Muller in FP32; where the
-                           Feller condition fails the pathwise variance Greeks go
+                           FP64, the log price, the Philox normals and Box-Muller in
+                           FP32; where the Feller condition fails the pathwise variance Greeks go
                            through 1/sqrt(v) near v = 0, and FP32 rounding of v moves
                            single paths' values by more than their standard error */
 } sdegpu_heston_greeks;

@@ -205,9 +205,9 @@ __device__ __forceinline__ double sqrt_mid(double v) {
   return fma(fma(-g, g, v), h, g);
 }
 
-// sqrt(v) for v >= 0 (0, infinity and NaN as sqrt gives them; below 1e-300 only
-// the order of magnitude): sqrt_mid's steps without the scaling of tiny
-// arguments that a full-range sqrt takes.
+// sqrt(v) for v >= 0 (0, infinity and NaN as sqrt gives them; below 1e-300
+// too small, of the size of v 1e150): sqrt_mid's steps without the scaling of
+// tiny arguments that a full-range sqrt takes.
 __device__ __forceinline__ double sqrt_nonneg(double v) {
   const double y = __builtin_amdgcn_rsq(fmax(v, 1e-300));
   double g = v * y, h = 0.5 * y;

@@ -13,9 +13,10 @@ its preset processes define:
 
 The kernels run the forward Euler pass on the same Philox draws as the
 process classes (a process built with the same ``rng`` seed gives the same
-paths) and sweep the adjoint backwards; for Heston over segments of the path,
-each while its partial derivatives are in registers, so no path history is
-stored or recomputed.  ``heston_price_fd`` is the FP64 forward plus central
+paths) and sweep the adjoint backwards; for Heston with an FP64 variance over
+segments of the path, each while its partial derivatives are in registers, in
+FP32 over the whole path, recomputed segment by segment from variance
+checkpoints every 8 steps (4 bytes each per path) and the Philox counters.  ``heston_price_fd`` is the FP64 forward plus central
 finite-difference baseline on common random numbers.
 
 ``HestonPrice.apply(params, config)`` exposes the price to torch autograd:
@@ -119,10 +120,11 @@ class GreeksResult:
 class HestonGreeks:
     """A prepared Heston Greeks run (step table, workspace and output on the
     device); ``launch()`` issues the kernels, ``result()`` reads the sums.
-    ``method='adjoint'`` sweeps the reverse-mode adjoint over segments of the
-    path and chains them; ``method='tangent'`` carries the five derivative
+    ``method='adjoint'`` is the reverse-mode adjoint: with an FP64 variance
+    swept over segments of the path that are chained, in FP32 over the whole
+    path from checkpoints; ``method='tangent'`` carries the five derivative
     directions along the forward pass step by step; both give the same
-    pathwise estimator.
+    pathwise estimator.  The workspace has room for either.
     ``variance_dtype=np.float64`` with an FP32 run carries the variance and
     every derivative in FP64, with the log price and the normals in FP32."""
 

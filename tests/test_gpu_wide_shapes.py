@@ -90,3 +90,19 @@ def test_order_of_blocks_and_rows_of_partial_lines(gpu, dtype, cls, kw):
         for key in ('negative_y_count', 'jump_count'):
             if key in info:
                 assert np.array_equal(info[key], ref_info[key][..., :paths])
+
+
+@pytest.mark.parametrize('m', [48, 49, 64])
+def test_jumps_of_many_coupled_components(gpu, m):
+    """FP64 jump models of 48 to 64 coupled components (up to 93 KB of LDS)."""
+    P, n, tt = 67, 3, np.linspace(0., 1., 3)
+    info, ref_info, jump = {}, {}, dict(lam=6., a=-.05, b=.1)
+    p = sa.merton_jumpdiff_process(paths=P, vshape=m, steps=n, corr=_corr(m), info=info, x0=1.,
+                                   mu=.03, sigma=.2, rng=np.random.default_rng(5), **jump)
+    src = {'dw': ora.PhiloxWiener(p.sources['dw'].key, 0, P, (m,), corr=_corr(m)),
+           'dj': ora.PhiloxCPoisson(p.sources['dj'].key, 0, P, (m,), **jump)}
+    got = p(tt)
+    ref = ora.integrate('jumpdiff', tt, paths=P, vshape=(m,), steps=n, sources=src,
+                        info=ref_info, x0=1., mu=.03, sigma=.2)
+    assert np.array_equal(info['jump_count'], ref_info['jump_count'])
+    assert np.max(np.abs(got / ref - 1)) < 1e-12
