@@ -22,7 +22,7 @@ path of ``sdepy_amd`` can be checked against it on identical inputs:
   differences for the Greeks kernels.
 
 Only ``tests/``, ``__graft_entry__.smoke()`` and the ``cpu_baseline`` leg of
-``bench.py`` may import this package, and only as the checker or the timed
+``bench.py`` may import this package, and only to check results or as the timed
 CPU baseline: the product path (``sdepy_amd``) never imports it and fails
 loudly when its HIP library is missing.
 

@@ -1,5 +1,5 @@
 """Test infrastructure: a NumPy restatement of sdepy's ``montecarlo``
-(infrastructure.py:2716-3083) used as the checker of the GPU summaries.
+(infrastructure.py:2716-3083) that the GPU summaries are compared with.
 
 It follows the reference step by step -- antithetic folding in the sample's
 type (:2885-2900), moments of the deviations from the first sample's mean

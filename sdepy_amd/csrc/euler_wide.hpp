@@ -15,9 +15,10 @@
 // v_mfma_f64_4x4x4 multiplies four rows of the square by four normals of the 16
 // paths.  Its operands are one 8-byte LDS read each, 512 bytes for 256
 // multiply-adds; as 16-byte broadcasts to lanes of 64 paths the coefficients
-// took 1024 bytes for 128, and the kernel was bound by those reads (the LDS at
-// work 56% of the time, the vector units 48%).  Now half of what is left is
-// normals, and the waits at the two barriers of a step.
+// took 1024 bytes for 128, and the kernel was bound by those reads.  Now the vector
+// units are at work 62% of the time, the LDS 54%, the matrix cores 13%, and the
+// waves wait 42% of theirs, for the LDS and at the two barriers of a step (20
+// correlated lognormals, 100,000 paths x 252).
 // FP32: a wave holds components (Heston: pairs) w, w + W, w + 2 W, ... of all 64
 // paths and reads its coefficients as 16-byte broadcasts, four at a time, at
 // fixed offsets (with scalar loads and a wait per piece of a row it took
