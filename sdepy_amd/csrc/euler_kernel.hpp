@@ -527,7 +527,19 @@ __global__ __launch_bounds__(kBlock, MOM ? 8 : 1) void k_euler(const EulerArgs a
   // With fused row moments every thread of the block takes part in the LDS
   // reductions, so the lanes beyond the last path step a copy of the last
   // path and store nothing; otherwise they leave at once.
-  const int64_t tid = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  // One FP32 jump component, in place: its stores go through the L2 and XCD x takes the
+  // x-th eighth of the blocks (the last few, past whole eighths, keep their places).  Where
+  // rows begin off the 64-byte lines two blocks share a line, which streamed stores
+  // write in two parts, and from some 250 MB of rows on those writes bound this kernel: Merton
+  // 1,000,003 paths x 252, every row, 597 us streamed, 497 so; 500,003 x 600 723 and
+  // 522; 1M of either 496 and 495.  Several components write apart in time, and
+  // lose up to 14% so (2 of 800,008 x 500, every row, 1454 and 1688).
+  constexpr bool STREAM =
+      !(kJump && sizeof(T) == 4 && M == 1 && BOUND && !GEN && !DEFER && !MOM && !PP);
+  const unsigned eighth = STREAM ? 0u : gridDim.x >> 3;
+  const unsigned blk = blockIdx.x < 8u * eighth ? (blockIdx.x & 7u) * eighth + (blockIdx.x >> 3)
+                                                : blockIdx.x;
+  const int64_t tid = (int64_t)blk * kBlock + threadIdx.x;
   const bool live = tid < a.paths;
   if (!MOM && !live) return;
   const int64_t gid = live ? tid : a.paths - 1;
@@ -583,7 +595,7 @@ __global__ __launch_bounds__(kBlock, MOM ? 8 : 1) void k_euler(const EulerArgs a
     mkmax = kMomSlots / a.nout;
   }
   auto store = [&](int row) {
-    store_state<MODEL, T, M, D, GEN, MOM>(
+    store_state<MODEL, T, M, D, GEN, MOM, STREAM>(
         out, a, row, x, gid, live,
         MOM ? mcols + mk * a.nout * kMomStride + (threadIdx.x & 63) : nullptr);
     if constexpr (MOM) {

@@ -30,13 +30,21 @@ def test_deferred_forms_match_oracle(gpu, how, nvar, nsteps, lam):
     _check(how, nvar, np.linspace(0., 1., nsteps + 1), np.array([0., 1.]), lam, 1)
 
 
-def _check(how, nvar, grid, tt, lam, deferred):
+@pytest.mark.parametrize('paths', [65_537, 67_328, 67_584, 67_599])
+def test_one_component_in_place_every_block(gpu, paths):
+    """Rows on and off the 64-byte lines, of a number of blocks that is a multiple of eight
+    and one more; paths of every block."""
+    grid = np.linspace(0., 1., 97)
+    _check('plain', 1, grid, grid, .5, 0, paths, 127)
+
+
+def _check(how, nvar, grid, tt, lam, deferred, paths=PATHS, every=2_999):
     vshape = () if nvar == 1 else (nvar,)
     jump = dict(lam=lam, a=-.01, b=.02)
     anti = how == 'antithetic'
     info, ref_info = {}, {}
     p = sa.merton_jumpdiff_process(
-        paths=PATHS, vshape=vshape, steps=grid, dtype=np.float32, info=info, mu=.03, sigma=.2,
+        paths=paths, vshape=vshape, steps=grid, dtype=np.float32, info=info, mu=.03, sigma=.2,
         dw=sa.odd_wiener_source if anti else None, rng=np.random.default_rng(9), **jump)
     dw, dj = p.sources['dw'], p.sources['dj']
     run = p.prepare(tt, moments=how == 'moments')
@@ -44,7 +52,7 @@ def _check(how, nvar, grid, tt, lam, deferred):
     assert (run._row_mom is not None) == (how == 'moments')
     x = run.run()
     # of antithetic paths the leading half, whose normals and jumps are a plain run's
-    at = np.arange(0, PATHS // 2 if anti else PATHS, 2_999)
+    at = np.arange(0, paths // 2 if anti else paths, every)
     key = dw.half.key if anti else dw.key
     ref = ora.integrate(
         'jumpdiff', tt, paths=at.size, vshape=vshape, steps=grid, info=ref_info, x0=1., mu=.03,
