@@ -88,10 +88,10 @@ VALU_ISSUE_PEAK_PER_S = 256 * 2.4e9
 # (FETCH reads half the copied bytes: x2.0; WRITE is exact: x1.0), and the
 # kernel's VALU wave-instructions per launch (SQ_INSTS_VALU); the summaries
 # they come from are in profiles/
-ADJ_TRAFFIC_BYTES = 1381737626        # k_heston_adjoint<8, true> (FP32), 4M x 365
+ADJ_TRAFFIC_BYTES = 1381867859        # k_heston_adjoint<8, true> (FP32), 4M x 365
 ADJ_VALU_WAVE_INSTS = 2003328125      # of which transcendental:
 ADJ_VALU_TRANS_WAVE_INSTS = 251187500  # (issued beside the other VALU work)
-OU_TRAFFIC_BYTES = 16028227946         # k_euler<OU, float, 4>, 1M x 1000
+OU_TRAFFIC_BYTES = 16024874346         # k_euler<OU, float, 4>, 1M x 1000
 BATCH_VALU_WAVE_INSTS = 28866568683    # k_batch_persistent, the 1024-instance set, 4 tiles per claim
 MERTON_VALU_WAVE_INSTS = 232900054     # k_loglin_greeks<float>, 2M x 252
 TANGENT_VALU_WAVE_INSTS = 1364203125   # k_heston_tangent<float, float>, 4M x 365
